@@ -248,6 +248,7 @@ int pfdd_gl_theta(pfdd_gl *h, double *theta);
 /* Autotuner (no counterpart in the reference): times each candidate LDS tile
  * shape (0, 1, 2: about 1K/2K/4K FP64 or 2K/4K/8K FP32 elements per tile) of
  * the four line passes -- forward z, forward y, inverse y, inverse z + update
+ * (with the next iteration's forward z transform, in choice[0]'s radix plan)
  * -- plus, for the first three, the FFT radix plan: choice 3, 4, 5 are shapes
  * 0, 1, 2 with radix-16 stages wherever they save a stage (lengths 16, 48,
  * 80, 128, 256: 128 = 16 x 8 instead of 8 x 8 x 2); 0-2 use radix 8 first.
@@ -255,8 +256,9 @@ int pfdd_gl_theta(pfdd_gl *h, double *theta);
  *   0  five kernels, x pass one tile per workgroup;
  *   1  five kernels, x pass on persistent workgroups that load the next tile
  *      while transforming the current one;
- *   2  three kernels (the "plane" iteration: 2-D FFT of each y-z plane in LDS,
- *      x pass, 2-D inverse FFT fused with the update), for square y-z planes
+ *   2  the "plane" iteration: x pass, then the 2-D inverse FFT of each y-z
+ *      plane in LDS fused with the update and the next iteration's 2-D forward
+ *      FFT (one more forward pass starts a run), for square y-z planes
  *      that fit in LDS (FP32 up to 128 x 128, FP64 up to 80 x 80), nx of
  *      16..128, on-the-fly B.
  * Timing runs on this handle's own buffers: after 20 warm-up iterations, two
@@ -275,16 +277,19 @@ int pfdd_gl_autotune(pfdd_gl *h, int nsteps, int choice[5]);
 /* Sets the choices explicitly (same meaning as pfdd_gl_autotune's output). */
 int pfdd_gl_set_tuning(pfdd_gl *h, const int choice[5]);
 
-/* Average device time (ms) of each kernel of one GL iteration over `nsteps`
- * iterations, measured with HIP events on the handle's stream that the kernel
- * dispatches record themselves (start and end of each kernel).  ms[0..4] =
- * forward z pass, forward y pass, x pass with contraction, inverse y pass,
- * inverse z pass with update; ms[5] = reduction; ms[6] = whole iteration.
- * nkernels receives the number of kernels of one iteration. */
+/* Average device time (ms) of each kernel of one GL iteration over one run of
+ * `nsteps` iterations, measured with HIP events on the handle's stream that
+ * the kernel dispatches record themselves (start and end of each kernel).
+ * ms[0] = the forward z pass (plane variant: forward plane pass) that starts a
+ * run; ms[1..4] = forward y pass, x pass with contraction, inverse y pass,
+ * inverse z pass with update and the next iteration's forward z pass; ms[5] =
+ * reduction; ms[6] = an iteration inside the run (without ms[0]).  nkernels
+ * receives the number of kernels timed. */
 int pfdd_gl_profile(pfdd_gl *h, int nsteps, double *ms, int *nkernels);
 
-/* Bytes the GL iteration moves, by the kernel split above (algorithmic
- * figure: each field element read/written once per kernel, B once). */
+/* Bytes each kernel of the split above moves per launch (algorithmic figure:
+ * each field element read/written once per kernel, B once), and the bytes of
+ * an iteration inside a run (slots 1-4). */
 int pfdd_gl_traffic(pfdd_gl *h, double *bytes_per_kernel, double *bytes_per_step);
 
 /* Several handles (e.g. batches of different grid sizes) stepped together by

@@ -12,13 +12,17 @@
 //              elastic-energy partial sums
 //   4  inv y   T2 -> T1[a][i][k][j]
 //   5  inv z   T1 -> g, fused core-energy derivative, applied stress, explicit
-//              Euler update, obstacle mask and reductions: xi_old -> xi_new
-//   +  one single-block kernel reduces the per-block partials in fixed order.
+//              Euler update, obstacle mask and reductions: xi_old -> xi_new;
+//              except in the last iteration of a run, also pass 1 of the next
+//              iteration (the block's lines of xi_new, back into T1)
+//   +  one small kernel reduces the per-block partials in fixed order.
+//
+// so pass 1 runs once per run and an iteration inside a run is four kernels.
 //
 // T2 is the ping-pong copy of xi that is not current, so the whole iteration
 // needs 3*S*N complex values plus B.  Every global access is a run of at least
 // 8 consecutive complex values (the pass transposes through LDS), and every
-// kernel reads and writes each field element exactly once.
+// kernel reads and writes each element of its fields exactly once.
 //
 // Reference functions replaced (fft_fftw_slab.cpp): core_energy_* :1130-1418,
 // forward_mode1 :1953-1964, internal_energy :1670-1695, backward_mode1
@@ -507,7 +511,7 @@ struct pfdd_gl {
     // graph launches; rocprofv3's kernel trace faults on them here)
     bool sg_on = true;
     bool plane_ok = false;             // the grid and precision allow the plane iteration
-    int nbA = 0, nbC = 0, nb3pl = 0;   // grids of the plane iteration's kernels
+    int nbA = 0, nbC = 0, nbCF = 0, nb3pl = 0; // grids of the plane iteration's kernels
     ThetaParams TP{};                  // core flag 5
     int ncu = 0;                       // compute units of the device
     double *stage2 = nullptr; // NSLOT * NB2
@@ -612,9 +616,14 @@ Maps make_maps_dims(long long nx, long long ny, long long nz, long long S)
 Maps make_maps(const pfdd_gl *h, long long S) { return make_maps_dims(h->nx, h->ny, h->nz, S); }
 
 // One GL iteration from xo into T2 (T2 doubles as the temporary of passes
-// 2-4), with the stress and core parameters P.
+// 2-4), with the stress and core parameters P, as part of a run of
+// iterations that each start from the previous one's result.  first: xo
+// enters the run here, so pass 1 (or the forward plane pass) runs; otherwise
+// the previous iteration left it in T1.  last: nothing follows, so the update
+// does not transform its result.  A run of one is first and last.
 template <typename R>
-int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, const StepParams &P)
+int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, const StepParams &P, bool first,
+              bool last)
 {
     const Maps m = make_maps(h, h->SM);
     hipStream_t st = h->stream;
@@ -648,9 +657,11 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
             return PFDD_OK;
         };
         int rc;
-        arm(0);
-        HIPCHK(launch_plane_fwd<R>(h->ny, h->nz, xo, h->T1, nplanes, h->nbA, h->tw[1], h->tw[2], h->done, st));
-        t_ev_start = t_ev_stop = nullptr;
+        if (first) {
+            arm(0);
+            HIPCHK(launch_plane_fwd<R>(h->ny, h->nz, xo, h->T1, nplanes, h->nbA, h->tw[1], h->tw[2], h->done, st));
+            t_ev_start = t_ev_stop = nullptr;
+        }
         if ((rc = empty(1))) return rc;
         arm(2);
         HIPCHK(launch_mid_pl<R>(h->nx, h->S, h->M, h->T1, h->G, (long long)h->ny * h->nz, h->N, h->tw[0],
@@ -658,12 +669,15 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
         t_ev_start = t_ev_stop = nullptr;
         if ((rc = empty(3))) return rc;
         arm(4);
-        HIPCHK(launch_plane_upd<R>(h->ny, h->nz, h->T1, xo, T2, h->mask, h->prev, h->cof ? h->cof : h->amp, nplanes,
-                                   h->nx, h->nbC, P, h->tw[1], h->tw[2], h->partial, h->pstride, h->done, st));
+        HIPCHK(launch_plane_upd<R>(h->ny, h->nz, !last, h->T1, xo, T2, h->mask, h->prev, h->cof ? h->cof : h->amp,
+                                   nplanes, h->nx, last ? h->nbC : h->nbCF, P, h->tw[1], h->tw[2], h->partial,
+                                   h->pstride, h->done, st));
     } else {
-    arm(0);
-    HIPCHK((launch_pass<R, false>(h->nz, xo, h->T1, m.p1i, m.p1o, m.n1, h->tw[2], h->done, st, nullptr,
-                                  h->tq[0])));
+    if (first) {
+        arm(0);
+        HIPCHK((launch_pass<R, false>(h->nz, xo, h->T1, m.p1i, m.p1o, m.n1, h->tw[2], h->done, st, nullptr,
+                                      h->tq[0])));
+    }
     arm(1);
     HIPCHK((launch_pass<R, false>(h->ny, h->T1, T2, m.p2i, m.p2o, m.n2, h->tw[1], h->done, st, nullptr,
                                   h->tq[1])));
@@ -678,9 +692,11 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
     HIPCHK((launch_pass<R, true>(h->ny, T2, h->T1, m.p2o, m.p2i, m.n2, h->tw[1], h->done, st, nullptr,
                                  h->tq[2])));
     arm(4);
-    HIPCHK(launch_update<R>(h->nz, h->tq[3], h->T1, xo, T2, h->mask, h->prev, h->cof ? h->cof : h->amp, m.p5i,
-                            m.p5o, m.n5, (long long)h->nx * h->ny, P, h->tw[2], h->partial, h->pstride, h->done,
-                            st));
+    // the transform that follows the update takes pass 1's radix plan, so that
+    // the field does not depend on how a run is cut into calls
+    HIPCHK(launch_update<R>(h->nz, h->tq[3], last ? 0 : 1 + h->tq[0] / 3, h->T1, xo, T2, h->mask, h->prev,
+                            h->cof ? h->cof : h->amp, m.p5i, m.p5o, m.n5, (long long)h->nx * h->ny, P, h->tw[2],
+                            h->partial, h->pstride, h->done, st));
     }
     arm(5);
     // E_core as the reference accumulates it (sum / nx); core_energy_extended
@@ -693,9 +709,9 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
 }
 
 template <typename R>
-int step_once(pfdd_gl *h, double tol, hipEvent_t *ev)
+int step_once(pfdd_gl *h, double tol, hipEvent_t *ev, bool first, bool last)
 {
-    const int rc = step_core<R>(h, tol, ev, h->xi[h->cur], h->xi[1 - h->cur], h->P);
+    const int rc = step_core<R>(h, tol, ev, h->xi[h->cur], h->xi[1 - h->cur], h->P, first, last);
     if (rc) return rc;
     h->cur = 1 - h->cur;
     h->stepped = true;
@@ -727,8 +743,16 @@ void set_tiles(pfdd_gl *h, const int tq[5])
     ++h->version; // captured graphs hold the old launch shapes
 }
 
-// Per-pass device time (ms) of the five tunable kernels over nsteps GL
-// iterations with the handle's current choices.
+// One iteration of h in its precision (see step_core).
+int step_any(pfdd_gl *h, double tol, bool first, bool last)
+{
+    return h->prec == PFDD_FP64 ? step_once<double>(h, tol, nullptr, first, last)
+                                : step_once<float>(h, tol, nullptr, first, last);
+}
+
+// Device time (ms) of the five tunable kernels, summed over nsteps GL
+// iterations from inside a run with the handle's current choices; acc[0] is
+// the one forward z pass that starts the run.
 template <typename R>
 int time_passes(pfdd_gl *h, int nsteps, double acc[5])
 {
@@ -738,13 +762,13 @@ int time_passes(pfdd_gl *h, int nsteps, double acc[5])
     const int pass_k[5] = {0, 1, 3, 4, 2}; // fwd z, fwd y, inv y, inv z + update, x pass
     int rc = PFDD_OK;
     for (int s = 0; s < nsteps && !rc; ++s) {
-        rc = step_once<R>(h, 0.0, ev);
+        rc = step_once<R>(h, 0.0, ev, s == 0, false);
         if (rc) break;
         if (hipEventSynchronize(ev[11]) != hipSuccess) {
             rc = fail(PFDD_ERR_HIP, "autotune timing failed");
             break;
         }
-        for (int p = 0; p < 5; ++p) {
+        for (int p = s == 0 ? 0 : 1; p < 5; ++p) {
             float t = 0;
             hipEventElapsedTime(&t, ev[2 * pass_k[p]], ev[2 * pass_k[p] + 1]);
             acc[p] += t;
@@ -818,7 +842,8 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
     // common warm-up, in two interleaved rounds, keeping each kernel's best
     // time per candidate.  The five-kernel iteration takes the best shape and
     // plan of each kernel; the plane iteration replaces it if its whole step
-    // (three kernels) is faster than that sum.
+    // is faster than that sum (both as inside a run: the forward z or plane
+    // pass that starts a run is not part of the sums).
     const bool plan_z = radix16_plan_differs_rt(h->nz), plan_y = radix16_plan_differs_rt(h->ny);
     const int nshape = (plan_z || plan_y) ? 6 : 3;
     const int c_pipe = h->stored_B ? -1 : nshape;
@@ -843,26 +868,38 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
             if ((rc = time_passes<R>(h, 1, warm)) || (rc = time_passes<R>(h, nsteps, t))) break;
             for (int p = 0; p < 5; ++p) tmin[c][p] = t[p] < tmin[c][p] ? t[p] : tmin[c][p];
         }
+    // the fastest shape of the forward z pass (run once per run) among those
+    // of one radix plan
+    auto best_z = [&](int plan) {
+        int b = 3 * plan;
+        for (int q = 3 * plan; q < 3 * plan + 3 && q < nshape; ++q) b = tmin[q][0] < tmin[b][0] ? q : b;
+        return b;
+    };
     if (!rc) {
         double best[5] = {1e300, 1e300, 1e300, 1e300, 1e300};
+        // the update carries the next forward z transform, so its shape and
+        // the radix plan of the z transforms are chosen together
+        int zplan = 0;
         for (int q = 0; q < nshape; ++q) {
             const int nl = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, q) : tile_lines_rt<float>(h->nz, q);
             const bool upd_ok = ((long long)h->nx * h->ny) % nl == 0;
-            // a plan-1 candidate counts for a line pass only where its length
-            // has a distinct radix-16 plan; the update takes shapes 0-2
-            const bool use[4] = {q < 3 || plan_z, q < 3 || plan_y, q < 3 || plan_y, q < 3 && upd_ok};
-            for (int p = 0; p < 4; ++p)
+            // a plan-1 candidate counts for a pass only where its length has a
+            // distinct radix-16 plan
+            const bool use[4] = {false, q < 3 || plan_y, q < 3 || plan_y, (q < 3 || plan_z) && upd_ok};
+            for (int p = 1; p < 4; ++p)
                 if (use[p] && tmin[q][p] < best[p]) {
                     best[p] = tmin[q][p];
-                    arg[p] = q;
+                    arg[p] = q % 3 + (p < 3 ? q / 3 * 3 : 0);
+                    if (p == 3) zplan = q / 3;
                 }
             best[4] = tmin[q][4] < best[4] ? tmin[q][4] : best[4];
         }
+        arg[0] = best_z(zplan);
         if (c_pipe >= 0 && tmin[c_pipe][4] < best[4]) {
             best[4] = tmin[c_pipe][4];
             arg[4] = 1;
         }
-        double five = best[0] + best[1] + best[2] + best[3] + best[4];
+        double five = best[1] + best[2] + best[3] + best[4];
         // The kernels of a step share the last-level cache (a whole FP32
         // field of 128^3 x 12 fits in it), so a kernel's time depends on the
         // tiles of its neighbours, and the mix of per-kernel winners was
@@ -876,7 +913,7 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
             int u1 = -1, u2 = -1;
             double s1 = 1e300, s2 = 1e300;
             for (int q = 0; q < nshape; ++q) {
-                const double s = tmin[q][0] + tmin[q][1] + tmin[q][2] + tmin[q][3] + tmin[q][4];
+                const double s = tmin[q][1] + tmin[q][2] + tmin[q][3] + tmin[q][4];
                 if (s < s1) { s2 = s1; u2 = u1; s1 = s; u1 = q; }
                 else if (s < s2) { s2 = s; u2 = q; }
             }
@@ -885,7 +922,7 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
                 const int nl = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, q % 3)
                                                     : tile_lines_rt<float>(h->nz, q % 3);
                 const bool upd_ok = ((long long)h->nx * h->ny) % nl == 0;
-                const int u[5] = {q < 3 || plan_z ? q : q % 3, q < 3 || plan_y ? q : q % 3,
+                const int u[5] = {best_z(plan_z ? q / 3 : 0), q < 3 || plan_y ? q : q % 3,
                                   q < 3 || plan_y ? q : q % 3, upd_ok ? q % 3 : arg[3], arg[4]};
                 bool dup = false;
                 for (int c = 0; c < nc; ++c) dup = dup || std::equal(u, u + 5, cand[c]);
@@ -902,7 +939,7 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
                         hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
                         double warm[5], t[5];
                         if ((rc = time_passes<R>(h, 1, warm)) || (rc = time_passes<R>(h, nsteps, t))) break;
-                        const double s = t[0] + t[1] + t[2] + t[3] + t[4];
+                        const double s = t[1] + t[2] + t[3] + t[4];
                         ts[c] = s < ts[c] ? s : ts[c];
                     }
                 int bc = 0;
@@ -914,8 +951,8 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
             }
         }
         if (!rc && c_plane >= 0) {
-            const double three = tmin[c_plane][0] + tmin[c_plane][3] + tmin[c_plane][4];
-            if (three < five) arg[4] = 2;
+            const double two = tmin[c_plane][3] + tmin[c_plane][4];
+            if (two < five) arg[4] = 2;
         }
     }
     int rc2 = restore();
@@ -1324,8 +1361,10 @@ int tape_backward_any(pfdd_gl *h, const void *dxi_T, bool dev_in, void *dxi_0, b
         const int s0 = sg * T.every, len = std::min(T.every, T.nsteps - s0);
         xs[0] = T.ckpt[sg];
         for (int j = 1; j < len; ++j) {
-            rc = h->prec == PFDD_FP64 ? step_core<double>(h, 0.0, nullptr, xs[j - 1], T.seg[j - 1], T.P)
-                                      : step_core<float>(h, 0.0, nullptr, xs[j - 1], T.seg[j - 1], T.P);
+            const bool first = j == 1, last = j == len - 1;
+            rc = h->prec == PFDD_FP64
+                     ? step_core<double>(h, 0.0, nullptr, xs[j - 1], T.seg[j - 1], T.P, first, last)
+                     : step_core<float>(h, 0.0, nullptr, xs[j - 1], T.seg[j - 1], T.P, first, last);
             if (rc) return rc;
             xs[j] = T.seg[j - 1];
         }
@@ -1387,7 +1426,7 @@ int self_graph_capture(pfdd_gl *h, double tol, int par)
     HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     int rc = PFDD_OK;
     for (int it = 0; it < SG_ITERS && !rc; ++it)
-        rc = h->prec == PFDD_FP64 ? step_once<double>(h, tol, nullptr) : step_once<float>(h, tol, nullptr);
+        rc = step_any(h, tol, it == 0, it == SG_ITERS - 1);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(h->stream, &graph);
     h->cur = cur0;
@@ -1598,6 +1637,8 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
                          : plane_blocks<float>(h->ny, h->nz, nplanes, h->ncu, 0);
             h->nbC = f64 ? plane_blocks<double>(h->ny, h->nz, nplanes, h->ncu, gen ? 2 : 1)
                          : plane_blocks<float>(h->ny, h->nz, nplanes, h->ncu, gen ? 2 : 1);
+            h->nbCF = f64 ? plane_blocks<double>(h->ny, h->nz, nplanes, h->ncu, gen ? 4 : 3)
+                          : plane_blocks<float>(h->ny, h->nz, nplanes, h->ncu, gen ? 4 : 3);
             const long long mx = h->nb3pl > nplanes ? h->nb3pl : nplanes;
             if (mx > h->pstride) h->pstride = mx;
         }
@@ -1849,8 +1890,7 @@ int pfdd_gl_step(pfdd_gl *h, int nsteps, double tol, pfdd_gl_reduce *out)
         eager = nsteps % SG_ITERS;
     }
     for (int s = 0; s < eager; ++s) {
-        rc = h->prec == PFDD_FP64 ? step_once<double>(h, tol, nullptr) : step_once<float>(h, tol, nullptr);
-        if (rc) return rc;
+        if ((rc = step_any(h, tol, s == 0, s == eager - 1))) return rc;
     }
     if (!out && tol <= 0) return PFDD_OK;
     return collect_steps(h, cur0, out);
@@ -1887,8 +1927,7 @@ int pfdd_gl_tape_record(pfdd_gl *h, int nsteps, int every, pfdd_gl_reduce *out)
     for (int s = 0; s < nsteps; ++s) {
         if (s % every == 0)
             HIPCHK(hipMemcpyAsync(T.ckpt[s / every], h->xi[h->cur], fb, hipMemcpyDeviceToDevice, h->stream));
-        rc = h->prec == PFDD_FP64 ? step_once<double>(h, 0.0, nullptr) : step_once<float>(h, 0.0, nullptr);
-        if (rc) return rc;
+        if ((rc = step_any(h, 0.0, s == 0, s == nsteps - 1))) return rc;
     }
     pfdd_gl_reduce r{};
     if ((rc = collect_steps(h, cur0, &r))) return rc;
@@ -2035,17 +2074,18 @@ int pfdd_gl_profile(pfdd_gl *h, int nsteps, double *ms, int *nkernels)
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
     for (int s = 0; s < nsteps && !rc; ++s)
-        rc = h->prec == PFDD_FP64 ? step_once<double>(h, 0.0, &ev[12 * s]) : step_once<float>(h, 0.0, &ev[12 * s]);
+        rc = h->prec == PFDD_FP64 ? step_once<double>(h, 0.0, &ev[12 * s], s == 0, false)
+                                  : step_once<float>(h, 0.0, &ev[12 * s], s == 0, false);
     if (!rc && hipEventSynchronize(ev.back()) != hipSuccess) rc = fail(PFDD_ERR_HIP, "profile wait failed");
     for (int s = 0; s < nsteps && !rc; ++s) {
         const hipEvent_t *e = &ev[12 * s];
-        for (int q = 0; q < 6; ++q) {
+        for (int q = s == 0 ? 0 : 1; q < 6; ++q) {
             float t = 0;
             hipEventElapsedTime(&t, e[2 * q], e[2 * q + 1]);
-            acc[q] += t;
+            acc[q] += q == 0 ? t * nsteps : t; // the forward pass runs once
         }
         float t = 0;
-        hipEventElapsedTime(&t, e[0], e[11]);
+        hipEventElapsedTime(&t, e[2], e[11]);
         acc[6] += t;
     }
     for (auto &e : ev) (void)hipEventDestroy(e);
@@ -2062,12 +2102,13 @@ int pfdd_gl_traffic(pfdd_gl *h, double *bytes_per_kernel, double *bytes_per_step
     const double f = (double)h->SM * h->N * h->esz;
     const double bsz =
         h->stored_B ? (double)h->S * (h->S + 1) / 2 * h->N * (h->prec == PFDD_FP64 ? 8 : 4) : 0.0;
-    // the plane iteration has no separate y passes (slots 1 and 3)
-    const double k[5] = {2 * f, h->plane ? 0.0 : 2 * f, 2 * f + bsz, h->plane ? 0.0 : 2 * f, 3 * f};
+    // the plane iteration has no separate y passes (slots 1 and 3); slot 0
+    // runs once per run and is no part of an iteration
+    const double k[5] = {2 * f, h->plane ? 0.0 : 2 * f, 2 * f + bsz, h->plane ? 0.0 : 2 * f, 4 * f};
     double tot = 0;
     for (int q = 0; q < 5; ++q) {
         if (bytes_per_kernel) bytes_per_kernel[q] = k[q];
-        tot += k[q];
+        if (q > 0) tot += k[q];
     }
     if (bytes_per_step) *bytes_per_step = tot;
     return PFDD_OK;
@@ -2128,7 +2169,7 @@ int graph_capture(pfdd_gl_graph *g, double tol)
             pfdd_gl *h = g->hs[i];
             e = hipStreamWaitEvent(h->stream, g->join[n], 0);
             for (int it = 0; it < g->iters && !rc && e == hipSuccess; ++it)
-                rc = h->prec == PFDD_FP64 ? step_once<double>(h, tol, nullptr) : step_once<float>(h, tol, nullptr);
+                rc = step_any(h, tol, it == 0, it == g->iters - 1);
             if (!rc && e == hipSuccess) e = hipEventRecord(g->join[i], h->stream);
             if (!rc && e == hipSuccess) e = hipStreamWaitEvent(g->stream, g->join[i], 0);
         }
@@ -2211,7 +2252,7 @@ int pfdd_gl_graph_run(pfdd_gl_graph *g, int nsteps, double tol, pfdd_gl_reduce *
         for (pfdd_gl *h : g->hs) {
             hipStream_t s0 = h->stream;
             h->stream = g->stream;
-            rc = h->prec == PFDD_FP64 ? step_once<double>(h, tol, nullptr) : step_once<float>(h, tol, nullptr);
+            rc = step_any(h, tol, it == 0, it == rem - 1);
             h->stream = s0;
             if (rc) return rc;
         }

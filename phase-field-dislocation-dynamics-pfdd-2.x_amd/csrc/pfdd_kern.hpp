@@ -353,8 +353,10 @@ hipError_t launch_pass(int n, const void *in, void *out, LineMap mi, LineMap mo,
                        int tq = 1);
 
 // Last inverse pass + GL update, and its reverse mode (pfdd_update.hip).
+// fw: 0 the update alone, 1 + plan also the next iteration's forward z pass of
+// the new field (T1 in place).
 template <typename R>
-hipError_t launch_update(int n, int tq, const void *T1, const void *xo, void *xn, const uint8_t *mask,
+hipError_t launch_update(int n, int tq, int fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
                          const long long *prev, const void *amp, LineMap mi, LineMap mo, long long nlines,
                          long long lps, const StepParams &P, const void *tw, double *partial,
                          long long pstride, const int *done, hipStream_t st);
@@ -381,17 +383,18 @@ hipError_t launch_mid_pl(int n, int S, int M, void *T, const GParams &G, long lo
 template <typename R> int mid_pl_blocks(int n, int S, int M, long long ncol);
 
 // Plane iteration (pfdd_plane.hip): the 2-D forward pass over y-z planes and
-// the 2-D inverse pass fused with the update, for square y-z planes that fit
-// in LDS; persistent grids of plane_blocks blocks.
+// the 2-D inverse pass fused with the update (and, with fw, with the next
+// iteration's forward pass, T in place), for square y-z planes that fit in
+// LDS; persistent grids of plane_blocks blocks.
 template <typename R> bool plane_supported(int ny, int nz);
 // which: 0 the forward kernel, 1 the update, 2 the update of the coupled /
-// Fourier core models.
+// Fourier core models; 3, 4 those updates with the next forward pass.
 template <typename R> int plane_blocks(int ny, int nz, long long nplanes, int ncu, int which);
 template <typename R>
 hipError_t launch_plane_fwd(int ny, int nz, const void *in, void *out, long long nplanes, int nblocks,
                             const void *twy, const void *twz, const int *done, hipStream_t st);
 template <typename R>
-hipError_t launch_plane_upd(int ny, int nz, const void *T, const void *xo, void *xn, const uint8_t *mask,
+hipError_t launch_plane_upd(int ny, int nz, bool fw, void *T, const void *xo, void *xn, const uint8_t *mask,
                             const long long *prev, const void *amp, long long nplanes, int nx, int nblocks,
                             const StepParams &P, const void *twy, const void *twz, double *partial,
                             long long pstride, const int *done, hipStream_t st);

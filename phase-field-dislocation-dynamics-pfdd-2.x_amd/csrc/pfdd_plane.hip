@@ -9,7 +9,10 @@
 //   C  k_plane_upd  T + xi_old -> xi_new: inverse 2-D FFT of each plane (along
 //                   j, then along k) fused with the GL update and its sums
 //
-// so an iteration moves 7 S N e bytes instead of 11 S N e.  Each line is
+// In a run of several iterations C also makes the next iteration's 2-D forward
+// transform of the plane it has just updated (FW) and writes it back to T, so
+// A runs once per run and an iteration is B and C: 6 S N e bytes against the
+// line passes' 10 S N e.  Each line is
 // transformed with the radix plan and twiddles of the line passes
 // (fft_stages_g), and the update is the same gl_update_cell, so the field is
 // bit-identical to the five-kernel iteration's.
@@ -118,9 +121,9 @@ __global__ void __launch_bounds__((plane_threads<R, NY, NZ>()))
 // plane's cells (gl_update_cell), and per-plane sums of xinorm^2, xiave, the
 // core energy and the stress work (partial[slot * pstride + plane]).  A plane holds one system, so tau and the core
 // coefficients are uniform over it.
-template <typename R, int NY, int NZ, bool GEN>
+template <typename R, int NY, int NZ, bool GEN, bool FW>
 __global__ void __launch_bounds__((plane_threads<R, NY, NZ>()))
-    k_plane_upd(const typename cvec<R>::type *__restrict__ T, const typename cvec<R>::type *__restrict__ xo,
+    k_plane_upd(typename cvec<R>::type *T, const typename cvec<R>::type *__restrict__ xo,
                 typename cvec<R>::type *__restrict__ xn, const uint8_t *__restrict__ mask,
                 const long long *__restrict__ prev, const R *__restrict__ amp, long long nplanes, int nx,
                 StepParams P, const typename cvec<R>::type *__restrict__ twy,
@@ -168,25 +171,40 @@ __global__ void __launch_bounds__((plane_threads<R, NY, NZ>()))
 #pragma unroll UNR
         for (int e = tid; e < TOT; e += NT) {
             const long long idx = base + e;
-            const V g = lds.ld((e % NZ) * LDY + e / NZ);
+            const int at = (e % NZ) * LDY + e / NZ;
+            const V g = lds.ld(at);
             const V x = ld_stream(&xo[idx]);
             R dens;
             double dn;
             const V y = gl_update_cell<R, GEN>(g, x, idx, tau, as % 3, [&](int m) { return lcf[m]; }, P, nm,
                                                cddt, invN, mask, prev, xo, amp, dn, dens);
             st_stream(&xn[idx], y);
+            if constexpr (FW) lds.st(at, y); // this thread's own cell, read above
             p_norm += dn;
             p_ave += (double)y.x;
             p_core += (double)dens;
             p_str += (double)tau * (double)x.x;
         }
         double v[4] = {p_norm, p_ave, p_core, p_str};
-        block_sum_comp<4, NT>(v, red, tid);
+        block_sum_comp<4, NT>(v, red, tid); // its barriers also order the tile writes above
         if (tid == 0) {
             partial[0 * pstride + pl] = v[0];
             partial[1 * pstride + pl] = v[1];
             partial[2 * pstride + pl] = v[2];
             partial[3 * pstride + pl] = v[3];
+        }
+        if constexpr (FW) {
+            // as k_plane_fwd, over this block's own plane of T, with addresses
+            // formed again (see k_update)
+            int t2 = tid;
+            __asm__ volatile("" : "+v"(t2));
+            fft_stages_g<NZ, 1, NY, 1, LDY, NT, false>(lds, tws + NY, t2);
+            fft_stages_g<NY, 1, NZ, LDY, 1, NT, false>(lds, tws, t2);
+#pragma unroll
+            for (int t = 0; t < PER; ++t) {
+                const int e = t2 + t * NT;
+                if (TOT % NT == 0 || e < TOT) st_stream(&T[base + e], lds.ld((e % NZ) * LDY + e / NZ));
+            }
         }
         __syncthreads();
     }
@@ -196,7 +214,8 @@ __global__ void __launch_bounds__((plane_threads<R, NY, NZ>()))
 #define PFDD_PLANE_SIZES(X) X(16) X(32) X(48) X(64) X(80) X(96) X(128)
 
 // Resident blocks per CU of kernel `which` (0 forward, 1 update, 2 update of
-// the coupled / Fourier core models) for N x N planes.
+// the coupled / Fourier core models, 3 and 4 the same with the next forward
+// pass) for N x N planes.
 template <typename R, int N> int plane_occupancy_n(int which)
 {
     auto occ = [](const void *f) {
@@ -204,9 +223,11 @@ template <typename R, int N> int plane_occupancy_n(int which)
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, f, plane_threads<R, N, N>(), 0) != hipSuccess) o = 1;
         return o > 0 ? o : 1;
     };
-    static const int o[3] = {occ((const void *)k_plane_fwd<R, N, N>), occ((const void *)k_plane_upd<R, N, N, false>),
-                             occ((const void *)k_plane_upd<R, N, N, true>)};
-    return o[which < 0 ? 0 : which > 2 ? 2 : which];
+    static const int o[5] = {
+        occ((const void *)k_plane_fwd<R, N, N>), occ((const void *)k_plane_upd<R, N, N, false, false>),
+        occ((const void *)k_plane_upd<R, N, N, true, false>), occ((const void *)k_plane_upd<R, N, N, false, true>),
+        occ((const void *)k_plane_upd<R, N, N, true, true>)};
+    return o[which < 0 ? 0 : which > 4 ? 4 : which];
 }
 
 template <typename R> bool plane_supported(int ny, int nz)
@@ -253,7 +274,7 @@ hipError_t launch_plane_fwd(int ny, int nz, const void *in, void *out, long long
 }
 
 template <typename R>
-hipError_t launch_plane_upd(int ny, int nz, const void *T, const void *xo, void *xn, const uint8_t *mask,
+hipError_t launch_plane_upd(int ny, int nz, bool fw, void *T, const void *xo, void *xn, const uint8_t *mask,
                             const long long *prev, const void *amp, long long nplanes, int nx, int nblocks,
                             const StepParams &P, const void *twy, const void *twz, double *partial,
                             long long pstride, const int *done, hipStream_t st)
@@ -261,24 +282,24 @@ hipError_t launch_plane_upd(int ny, int nz, const void *T, const void *xo, void 
     typedef typename cvec<R>::type V;
     if (ny != nz) return hipErrorInvalidValue;
     const bool gen = P.model == PFDD_CORE_EXTENDED || P.model == PFDD_CORE_PYRII || P.model == PFDD_CORE_FOURIER;
+#define PFDD_UPD(GEN_, FW_)                                                                                  \
+    PFDD_LAUNCH((k_plane_upd<R, N, N, GEN_, FW_>), dim3((unsigned)nblocks), dim3(plane_threads<R, N, N>()),  \
+                st, (V *)T, (const V *)xo, (V *)xn, mask, prev, (const R *)amp, nplanes, nx, P,              \
+                (const V *)twy, (const V *)twz, partial, pstride, done)
 #define PFDD_CASE(n_)                                                                                        \
     if (ny == n_) {                                                                                          \
-        if constexpr (plane_fits<R, n_, n_>()) {                                                             \
-            if (gen)                                                                                         \
-                PFDD_LAUNCH((k_plane_upd<R, n_, n_, true>), dim3((unsigned)nblocks),                         \
-                            dim3(plane_threads<R, n_, n_>()), st, (const V *)T, (const V *)xo, (V *)xn, mask,   \
-                            prev, (const R *)amp, nplanes, nx, P, (const V *)twy, (const V *)twz, partial,   \
-                            pstride, done);                                                                  \
-            else                                                                                             \
-                PFDD_LAUNCH((k_plane_upd<R, n_, n_, false>), dim3((unsigned)nblocks),                        \
-                            dim3(plane_threads<R, n_, n_>()), st, (const V *)T, (const V *)xo, (V *)xn, mask,   \
-                            prev, (const R *)amp, nplanes, nx, P, (const V *)twy, (const V *)twz, partial,   \
-                            pstride, done);                                                                  \
+        constexpr int N = n_;                                                                                \
+        if constexpr (plane_fits<R, N, N>()) {                                                               \
+            if (gen && fw) PFDD_UPD(true, true);                                                             \
+            else if (gen) PFDD_UPD(true, false);                                                             \
+            else if (fw) PFDD_UPD(false, true);                                                              \
+            else PFDD_UPD(false, false);                                                                     \
             return hipGetLastError();                                                                        \
         }                                                                                                    \
     }
     PFDD_PLANE_SIZES(PFDD_CASE)
 #undef PFDD_CASE
+#undef PFDD_UPD
     return hipErrorInvalidValue;
 }
 
@@ -287,7 +308,7 @@ hipError_t launch_plane_upd(int ny, int nz, const void *T, const void *xo, void 
     template int plane_blocks<R>(int, int, long long, int, int);                                              \
     template hipError_t launch_plane_fwd<R>(int, int, const void *, void *, long long, int, const void *,        \
                                             const void *, const int *, hipStream_t);                           \
-    template hipError_t launch_plane_upd<R>(int, int, const void *, const void *, void *, const uint8_t *,     \
+    template hipError_t launch_plane_upd<R>(int, int, bool, void *, const void *, void *, const uint8_t *,     \
                                             const long long *, const void *, long long, int, int,              \
                                             const StepParams &, const void *, const void *, double *, long long, \
                                             const int *, hipStream_t);

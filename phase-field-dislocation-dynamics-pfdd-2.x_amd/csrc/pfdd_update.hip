@@ -14,14 +14,21 @@ namespace pfdd {
 // lines at 128 points, 19-20 KB of LDS: 8 blocks per CU) asks for 8 waves per
 // SIMD: 64 instead of 68 VGPRs, 229 -> 224.5 us at 128^3 x 12.  The same
 // hint made the FP32 one 9 % slower.
-template <typename R, int N, int TQ, bool GEN> constexpr int update_waves()
+//
+// FW: 0 the update alone (last iteration of a run); 1, 2 the update followed
+// by the forward z transform of the new field, written back over the block's
+// own lines of T1: pass 1 of the next iteration, with radix plan FW - 1.  The
+// lines are complete in the tile after the update, so the next iteration
+// needs no pass that reads the field again: 4 S N e bytes instead of 5 in two
+// kernels.
+template <typename R, int N, int TQ, bool GEN, int FW> constexpr int update_waves()
 {
-    return (sizeof(R) == 8 && TQ == 0 && !GEN && N >= 32 && N <= 128) ? 8 : 1;
+    return (sizeof(R) == 8 && TQ == 0 && !GEN && FW < 2 && N >= 32 && N <= 128) ? 8 : 1;
 }
 
-template <typename R, int N, int TQ, bool GEN>
-__global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(update_waves<R, N, TQ, GEN>(), 8)))
-    k_update(const typename cvec<R>::type *__restrict__ T1, const typename cvec<R>::type *__restrict__ xo,
+template <typename R, int N, int TQ, bool GEN, int FW>
+__global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(update_waves<R, N, TQ, GEN, FW>(), 8)))
+    k_update(typename cvec<R>::type *T1, const typename cvec<R>::type *__restrict__ xo,
              typename cvec<R>::type *__restrict__ xn, const uint8_t *__restrict__ mask,
              const long long *__restrict__ prev, const R *__restrict__ amp, LineMap mi, LineMap mo,
              long long nlines, long long lines_per_sys, StepParams P,
@@ -100,18 +107,29 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(updat
         const V y = gl_update_cell<R, GEN>(g, x, idx, tau, lsub[l], [&](int m) { return lcoef[m * NL + l]; }, P, nm,
                                            cddt, invN, mask, prev, xo, amp, dn, dens);
         st_stream(&xn[idx], y);
+        if constexpr (FW != 0) lds.st(p * LDP + l, y); // this thread's own cell, read above
         s_norm += dn;
         s_ave += (double)y.x;
         s_core += (double)dens;
         s_str += (double)tau * (double)x.x;
     }
     double v[4] = {s_norm, s_ave, s_core, s_str};
-    block_sum_comp<4, NTHR>(v, red, tid);
+    block_sum_comp<4, NTHR>(v, red, tid); // its barriers also order the tile writes above
     if (tid == 0) {
         partial[0 * pstride + blockIdx.x] = v[0];
         partial[1 * pstride + blockIdx.x] = v[1];
         partial[2 * pstride + blockIdx.x] = v[2];
         partial[3 * pstride + blockIdx.x] = v[3];
+    }
+    if constexpr (FW != 0) {
+        // a thread index the compiler cannot trace: the addresses of the second
+        // transform are formed again instead of held in registers through the
+        // update
+        int t2 = tid;
+        __asm__ volatile("" : "+v"(t2));
+        if constexpr (FW == 2) fft_stages_x<N, 1, NL, NTHR, false>(lds, tw, t2);
+        else fft_stages<N, 1, NL, NTHR, false>(lds, tw, t2);
+        tile_store<N, NL, NTHR>(T1, lds, bin, mi.SP, t2);
     }
 }
 
@@ -250,7 +268,7 @@ __global__ void __launch_bounds__(NTHR)
 
 
 template <typename R>
-hipError_t launch_update(int n, int tq, const void *T1, const void *xo, void *xn, const uint8_t *mask,
+hipError_t launch_update(int n, int tq, int fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
                          const long long *prev, const void *amp, LineMap mi, LineMap mo, long long nlines,
                          long long lps, const StepParams &P, const void *tw, double *partial,
                          long long pstride, const int *done, hipStream_t st)
@@ -260,27 +278,30 @@ hipError_t launch_update(int n, int tq, const void *T1, const void *xo, void *xn
     // tile shape) so that the common sine-series kernel carries none of
     // their registers
     const bool gen = P.model == PFDD_CORE_EXTENDED || P.model == PFDD_CORE_PYRII || P.model == PFDD_CORE_FOURIER;
+    // plan 1 falls back to plan 0 where the two coincide
+#define PFDD_UPD(TQ_, GEN_, FW_)                                                                     \
+    PFDD_LAUNCH((k_update<R, N, TQ_, GEN_, FW_>),                                                    \
+                dim3((unsigned)((nlines + tile_lines_u<R, N, TQ_>() - 1) / tile_lines_u<R, N, TQ_>())), \
+                dim3(NTHR), st, (V *)T1, (const V *)xo, (V *)xn, mask, prev, (const R *)amp, mi, mo, \
+                nlines, lps, P, (const V *)tw, partial, pstride, done)
+#define PFDD_UPD_FW(TQ_, GEN_)                                                                       \
+    if (fw == 0) PFDD_UPD(TQ_, GEN_, 0);                                                             \
+    else if (fw == 2 && radix16_plan_differs<N>()) PFDD_UPD(TQ_, GEN_, (radix16_plan_differs<N>() ? 2 : 1)); \
+    else PFDD_UPD(TQ_, GEN_, 1)
 #define PFDD_CASE(n_)                                                                                \
     if (n == n_) {                                                                                   \
+        constexpr int N = n_;                                                                        \
         if (gen) {                                                                                   \
-            constexpr int NL = tile_lines_u<R, n_, 0>();                                             \
-            const unsigned nb = (unsigned)((nlines + NL - 1) / NL);                                  \
-            PFDD_LAUNCH((k_update<R, n_, 0, true>), dim3(nb), dim3(NTHR), st, (const V *)T1,         \
-                        (const V *)xo, (V *)xn, mask, prev, (const R *)amp, mi, mo, nlines, lps, P,  \
-                        (const V *)tw, partial, pstride, done);                                      \
+            PFDD_UPD_FW(0, true);                                                                    \
             return hipGetLastError();                                                                \
         }                                                                                            \
-        PFDD_TQ_DISPATCH(tq, {                                                                       \
-            constexpr int NL = tile_lines_u<R, n_, TQ>();                                            \
-            const unsigned nb = (unsigned)((nlines + NL - 1) / NL);                                  \
-            PFDD_LAUNCH((k_update<R, n_, TQ, false>), dim3(nb), dim3(NTHR), st, (const V *)T1,       \
-                               (const V *)xo, (V *)xn, mask, prev, (const R *)amp, mi, mo, nlines, lps, \
-                               P, (const V *)tw, partial, pstride, done);                            \
-        })                                                                                           \
+        PFDD_TQ_DISPATCH(tq, { PFDD_UPD_FW(TQ, false); })                                            \
         return hipGetLastError();                                                                    \
     }
     PFDD_SIZES(PFDD_CASE)
 #undef PFDD_CASE
+#undef PFDD_UPD_FW
+#undef PFDD_UPD
     return hipErrorInvalidValue;
 }
 
@@ -308,7 +329,7 @@ hipError_t launch_adj_update(int n, int tq, const void *T1, const void *lam, con
 }
 
 #define PFDD_INST(R)                                                                                          \
-    template hipError_t launch_update<R>(int, int, const void *, const void *, void *, const uint8_t *,          \
+    template hipError_t launch_update<R>(int, int, int, void *, const void *, void *, const uint8_t *,           \
                                          const long long *, const void *, LineMap, LineMap, long long, long long, \
                                          const StepParams &, const void *, double *, long long, const int *,      \
                                          hipStream_t);                                                            \
