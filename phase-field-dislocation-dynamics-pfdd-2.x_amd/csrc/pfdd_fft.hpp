@@ -28,11 +28,17 @@ template <typename V> __device__ __forceinline__ V mk(decltype(V{}.x) x, decltyp
 }
 template <typename V> __device__ __forceinline__ V cadd(V a, V b) { return mk<V>(a.x + b.x, a.y + b.y); }
 template <typename V> __device__ __forceinline__ V csub(V a, V b) { return mk<V>(a.x - b.x, a.y - b.y); }
+// a b + c d with one rounding of c d and one of the sum.  A sum of two products
+// leaves the compiler the choice which one enters the fused multiply-add; it
+// is made here, so that the same line transformed by different kernels rounds
+// alike.
+__device__ __forceinline__ double ab_cd(double a, double b, double c, double d) { return __builtin_fma(a, b, c * d); }
+__device__ __forceinline__ float ab_cd(float a, float b, float c, float d) { return __builtin_fmaf(a, b, c * d); }
 // a * w (forward) or a * conj(w) (inverse)
 template <bool INV, typename V> __device__ __forceinline__ V cmulw(V a, V w)
 {
     const auto wy = INV ? -w.y : w.y;
-    return mk<V>(a.x * w.x - a.y * wy, a.x * wy + a.y * w.x);
+    return mk<V>(ab_cd(a.x, w.x, -a.y, wy), ab_cd(a.x, wy, a.y, w.x));
 }
 // a * e^{-i pi/2} = -i a (forward), a * e^{+i pi/2} = +i a (inverse)
 template <bool INV, typename V> __device__ __forceinline__ V cmul_mi(V a)
@@ -180,8 +186,8 @@ template <bool INV, typename V> __device__ __forceinline__ void dft5(V *v)
     const V x0 = v[0];
     const V a1 = mk<V>(x0.x + c1 * t1.x + c2 * t2.x, x0.y + c1 * t1.y + c2 * t2.y);
     const V a2 = mk<V>(x0.x + c2 * t1.x + c1 * t2.x, x0.y + c2 * t1.y + c1 * t2.y);
-    const V b1 = mk<V>(s1 * d1.x + s2 * d2.x, s1 * d1.y + s2 * d2.y);
-    const V b2 = mk<V>(s2 * d1.x - s1 * d2.x, s2 * d1.y - s1 * d2.y);
+    const V b1 = mk<V>(ab_cd(s1, d1.x, s2, d2.x), ab_cd(s1, d1.y, s2, d2.y));
+    const V b2 = mk<V>(ab_cd(s2, d1.x, -s1, d2.x), ab_cd(s2, d1.y, -s1, d2.y));
     const V ib1 = mk<V>(-b1.y, b1.x), ib2 = mk<V>(-b2.y, b2.x); // i b
     v[0] = cadd(x0, cadd(t1, t2));
     if (INV) {
@@ -200,8 +206,8 @@ template <bool INV, typename V> __device__ __forceinline__ void dft5(V *v)
 // y * (c - i s) forward, y * (c + i s) inverse
 template <bool INV, typename V> __device__ __forceinline__ V crot(V y, decltype(V{}.x) c, decltype(V{}.x) s)
 {
-    if (INV) return mk<V>(y.x * c - y.y * s, y.y * c + y.x * s);
-    return mk<V>(y.x * c + y.y * s, y.y * c - y.x * s);
+    if (INV) return mk<V>(ab_cd(y.x, c, -y.y, s), ab_cd(y.y, c, y.x, s));
+    return mk<V>(ab_cd(y.x, c, y.y, s), ab_cd(y.y, c, -y.x, s));
 }
 
 // Length-16 DFT as 4 x 4 (n = 4 n1 + n2, k = k1 + 4 k2): length-4 DFTs over

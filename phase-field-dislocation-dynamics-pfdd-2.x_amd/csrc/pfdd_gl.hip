@@ -490,6 +490,7 @@ struct pfdd_gl {
     uint8_t *mask = nullptr;
     long long *prev = nullptr;
     void *amp = nullptr;
+    UpdNone *none = nullptr;
     double *partial = nullptr;
     long long pstride = 0;
     int nb3 = 0, nb5 = 0, nb5max = 0; // blocks of pass 3 / pass 5 (current tile, smallest tile)
@@ -694,9 +695,9 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
     arm(4);
     // the transform that follows the update takes pass 1's radix plan, so that
     // the field does not depend on how a run is cut into calls
-    HIPCHK(launch_update<R>(h->nz, h->tq[3], last ? 0 : 1 + h->tq[0] / 3, h->T1, xo, T2, h->mask, h->prev,
+    HIPCHK(launch_update<R>(h->nz, h->tq[3], h->tq[0] / 3, !last, h->T1, xo, T2, h->mask, h->prev,
                             h->cof ? h->cof : h->amp, m.p5i, m.p5o, m.n5, (long long)h->nx * h->ny, P, h->tw[2],
-                            h->partial, h->pstride, h->done, st));
+                            h->none, h->partial, h->pstride, h->done, st));
     }
     arm(5);
     // E_core as the reference accumulates it (sum / nx); core_energy_extended
@@ -736,8 +737,8 @@ void set_tiles(pfdd_gl *h, const int tq[5])
         h->nb3 = h->nb3pl;
     } else {
         const long long n5 = (long long)h->SM * h->nx * h->ny;
-        const int nl = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, h->tq[3])
-                                            : tile_lines_rt<float>(h->nz, h->tq[3]);
+        const int nl = h->prec == PFDD_FP64 ? update_lines<double>(h->nz, h->tq[3], m)
+                                            : update_lines<float>(h->nz, h->tq[3], m);
         h->nb5 = (int)((n5 + nl - 1) / nl);
     }
     ++h->version; // captured graphs hold the old launch shapes
@@ -1010,7 +1011,9 @@ int adjoint_core(pfdd_gl *h, const void *xs, const void *lam_in, void *lam_out, 
     HIPCHK(launch_adj_update<R>(h->nz, h->tq[3], h->T1, lam_in, xs, lam_out, h->mask, h->amp, m.p5i, m.p5o,
                                 m.n5, (long long)h->nx * h->ny, P, h->tw[2], h->tape.gpart, gstride, h->done,
                                 st));
-    hipLaunchKernelGGL(k_grad_reduce, dim3(h->S), dim3(NTHR), 0, st, h->tape.gpart, gstride, h->nb5 / h->S,
+    const int nla = tile_lines_rt<R>(h->nz, h->tq[3]);
+    hipLaunchKernelGGL(k_grad_reduce, dim3(h->S), dim3(NTHR), 0, st, h->tape.gpart, gstride,
+                       (int)((long long)h->nx * h->ny / nla),
                        h->tape.gacc, h->done);
     HIPCHK(hipGetLastError());
     return PFDD_OK;
@@ -1045,7 +1048,7 @@ void destroy_all(pfdd_gl *h)
     if (h->stream) hipStreamSynchronize(h->stream);
     self_graph_release(h);
     void *ptrs[] = {h->cof, h->taud, h->xi[0], h->xi[1], h->T1, h->B, h->tw[0], h->tw[1], h->tw[2], h->mask, h->prev,
-                    h->amp, h->partial, h->res, h->done, h->steps, h->stage2, h->ticket, h->dw[0], h->dw[1],
+                    h->amp, h->none, h->partial, h->res, h->done, h->steps, h->stage2, h->ticket, h->dw[0], h->dw[1],
                     h->deps, h->dsig, h->tape.lam[0], h->tape.lam[1], h->tape.gpart, h->tape.gacc};
     for (void *p : ptrs)
         if (p) hipFree(p);
@@ -1613,6 +1616,12 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
     const int nl5min = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, 0) : tile_lines_rt<float>(h->nz, 0);
     h->nb5 = (int)((n5 + nl5 - 1) / nl5);
     h->nb5max = (int)((n5 + nl5min - 1) / nl5min);
+    {
+        // the register update's tiles are smaller on short lines
+        const int nlr = h->prec == PFDD_FP64 ? update_lines<double>(h->nz, 0, d->core_model)
+                                             : update_lines<float>(h->nz, 0, d->core_model);
+        h->nb5max = std::max(h->nb5max, (int)((n5 + nlr - 1) / nlr));
+    }
     h->nb3 = h->M * (h->prec == PFDD_FP64 ? mid_blocks<double>(h->nx, h->S, (long long)h->ny * h->nz)
                                           : mid_blocks<float>(h->nx, h->S, (long long)h->ny * h->nz));
     if (h->M > 1) {
@@ -1646,6 +1655,12 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
     {
         const int dflt[5] = {1, 1, 1, 1, 0};
         set_tiles(h, dflt); // nb5 of the model's update tile
+    }
+    {
+        const UpdNone none = {1.0, 1.0f, 0};
+        if ((rc = alloc((void **)&h->none, sizeof(none)))) return bail(rc);
+        if (hipMemcpy(h->none, &none, sizeof(none), hipMemcpyHostToDevice) != hipSuccess)
+            return bail(fail(PFDD_ERR_HIP, "constant upload failed"));
     }
     if ((rc = alloc((void **)&h->partial, sizeof(double) * NSLOT * h->pstride))) return bail(rc);
     if ((rc = alloc((void **)&h->res, sizeof(double) * NRES))) return bail(rc);

@@ -58,27 +58,37 @@ struct StepParams {
 // points), against ~45 (FP32) and more (FP64) VALU instructions of the
 // library's sincospi, which the VALU-bound update kernels feel.  NaN and
 // infinite x give NaN.
+//
+// sconst: an FP64 literal held in scalar registers.  As an operand the compiler
+// can see, each literal is moved into a vector register pair for a fused
+// multiply-add that overwrites it: two more vector instructions per term, 530
+// of the 4300 of the register update's 16 cells.
+__device__ __forceinline__ double sconst(double c)
+{
+    __asm__("" : "+s"(c));
+    return c;
+}
 __device__ __forceinline__ void sincospi_poly(double x, double &s, double &c)
 {
     const double n = __builtin_rint(x);
     const double r = x - n, t = r * r;
-    double p = 0x1.9d2aaaaaaaaabp-21;
-    p = __builtin_fma(p, t, -0x1.6f79d8e38e38ep-16);
-    p = __builtin_fma(p, t, 0x1.e8f35feaaaaabp-12);
-    p = __builtin_fma(p, t, -0x1.e3074ddaa0000p-8);
-    p = __builtin_fma(p, t, 0x1.50783484ff78ep-4);
-    p = __builtin_fma(p, t, -0x1.32d2cce626dd4p-1);
-    p = __builtin_fma(p, t, 0x1.466bc6775aa52p+1);
-    p = __builtin_fma(p, t, -0x1.4abbce625be52p+2);
-    p = __builtin_fma(p, t, 0x1.921fb54442d18p+1);
-    double q = 0x1.167771c71c71cp-18;
-    q = __builtin_fma(q, t, -0x1.b69562aaaaaabp-14);
-    q = __builtin_fma(q, t, 0x1.f9d253ac38e39p-10);
-    q = __builtin_fma(q, t, -0x1.a6d1efc621c72p-6);
-    q = __builtin_fma(q, t, 0x1.e1f506812dcb9p-3);
-    q = __builtin_fma(q, t, -0x1.55d3c7e3bf9d1p+0);
-    q = __builtin_fma(q, t, 0x1.03c1f081b598cp+2);
-    q = __builtin_fma(q, t, -0x1.3bd3cc9be45dbp+2);
+    double p = sconst(0x1.9d2aaaaaaaaabp-21);
+    p = __builtin_fma(p, t, sconst(-0x1.6f79d8e38e38ep-16));
+    p = __builtin_fma(p, t, sconst(0x1.e8f35feaaaaabp-12));
+    p = __builtin_fma(p, t, sconst(-0x1.e3074ddaa0000p-8));
+    p = __builtin_fma(p, t, sconst(0x1.50783484ff78ep-4));
+    p = __builtin_fma(p, t, sconst(-0x1.32d2cce626dd4p-1));
+    p = __builtin_fma(p, t, sconst(0x1.466bc6775aa52p+1));
+    p = __builtin_fma(p, t, sconst(-0x1.4abbce625be52p+2));
+    p = __builtin_fma(p, t, sconst(0x1.921fb54442d18p+1));
+    double q = sconst(0x1.167771c71c71cp-18);
+    q = __builtin_fma(q, t, sconst(-0x1.b69562aaaaaabp-14));
+    q = __builtin_fma(q, t, sconst(0x1.f9d253ac38e39p-10));
+    q = __builtin_fma(q, t, sconst(-0x1.a6d1efc621c72p-6));
+    q = __builtin_fma(q, t, sconst(0x1.e1f506812dcb9p-3));
+    q = __builtin_fma(q, t, sconst(-0x1.55d3c7e3bf9d1p+0));
+    q = __builtin_fma(q, t, sconst(0x1.03c1f081b598cp+2));
+    q = __builtin_fma(q, t, sconst(-0x1.3bd3cc9be45dbp+2));
     q = __builtin_fma(q, t, 1.0);
     // (-1)^n from the parity of the integer-valued n (exact for |n| < 2^53)
     const double h = 0.5 * n;
@@ -237,7 +247,7 @@ __device__ __forceinline__ V gl_update_cell(const V g, const V x, long long idx,
                 const R c = coef(m - 1);
                 dens += c * sm * sm;
                 dE += c * ((R)m * (R)M_PI) * ((R)2 * sm * cm);
-                const R sn = sm * cp + cm * sp, cn = cm * cp - sm * sp;
+                const R sn = ab_cd(sm, cp, cm, sp), cn = ab_cd(cm, cp, -sm, sp);
                 sm = sn;
                 cm = cn;
             }
@@ -262,6 +272,49 @@ __device__ __forceinline__ V gl_update_cell(const V g, const V x, long long idx,
         dn = dr * dr + di * di;
     }
     return y;
+}
+
+// CH cells of one line of update_order_parameter with a sine-series core of
+// NM terms, as gl_update_cell but without branches (each basic block of a
+// per-cell branch cost the register update about 60 VGPRs): lc[m], ldp[m] are
+// the line's coefficient m and that times (m + 1) pi, zero past the model's
+// last term; MA: A holds the cells' amplitudes (1 where there are none) and
+// bit c of frozen is set where cell c keeps its value (its xinorm term is the
+// caller's).
+template <typename R, int NM, bool MA, int CH, typename V>
+__device__ __forceinline__ void gl_update_chunk(const V *g, const V *x, const R *A, unsigned frozen, R tau,
+                                                const R *lc, const R *ldp, R cddt, R invN, V *y, double *dn, R *dens)
+{
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        R sp, cp;
+        sincospi_poly(x[c].x, sp, cp);
+        R sm = sp, cm = cp, dE = (R)0;
+        dens[c] = (R)0;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            dens[c] += lc[m] * sm * sm;
+            dE += ldp[m] * ((R)2 * sm * cm);
+            if (m + 1 < NM) {
+                const R sn = ab_cd(sm, cp, cm, sp), cn = ab_cd(cm, cp, -sm, sp);
+                sm = sn;
+                cm = cn;
+            }
+        }
+        if constexpr (MA) {
+            dens[c] *= A[c];
+            dE *= A[c];
+        }
+        y[c].x = x[c].x - cddt * (g[c].x * invN - tau + dE);
+        y[c].y = x[c].y - cddt * (g[c].y * invN);
+        if constexpr (MA) {
+            const bool fz = (frozen >> c) & 1;
+            y[c].x = fz ? x[c].x : y[c].x;
+            y[c].y = fz ? x[c].y : y[c].y;
+        }
+        const double dr = (double)y[c].x - (double)x[c].x, di = (double)y[c].y - (double)x[c].y;
+        dn[c] = dr * dr + di * di;
+    }
 }
 
 struct BParams {
@@ -353,12 +406,19 @@ hipError_t launch_pass(int n, const void *in, void *out, LineMap mi, LineMap mo,
                        int tq = 1);
 
 // Last inverse pass + GL update, and its reverse mode (pfdd_update.hip).
-// fw: 0 the update alone, 1 + plan also the next iteration's forward z pass of
-// the new field (T1 in place).
+// plan: radix plan of the z transforms; fw: also the next iteration's forward
+// z pass of the new field (T1 in place).  Blocks (partials) of a launch:
+// nlines / update_lines.
+struct UpdNone {  // device constants read where a run has no mask or no amplitude
+    double one64;
+    float one32;
+    uint8_t zero;
+};
+template <typename R> int update_lines(int n, int tq, int model);
 template <typename R>
-hipError_t launch_update(int n, int tq, int fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
+hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
                          const long long *prev, const void *amp, LineMap mi, LineMap mo, long long nlines,
-                         long long lps, const StepParams &P, const void *tw, double *partial,
+                         long long lps, const StepParams &P, const void *tw, const UpdNone *none, double *partial,
                          long long pstride, const int *done, hipStream_t st);
 template <typename R>
 hipError_t launch_adj_update(int n, int tq, const void *T1, const void *lam, const void *xs, void *lam_out,

@@ -1,0 +1,174 @@
+// pfdd_reg.hpp -- line transforms held in registers.
+//
+// A block of W threads transforms a tile of NL lines of N points; every thread
+// holds VPT values of one line, W = NL * N / VPT.  In its natural ownership
+// thread (l, p0), p0 < D = N / VPT, holds the positions p0 + D m, m < VPT, of
+// line l.  These are the inputs of VPT / RAD butterflies of any radix RAD that
+// divides VPT, of a first stage as of a last one (a last stage's outputs
+// j + r N / RAD are its inputs' positions), so that
+//
+//   * the first stage reads its inputs straight from memory and the last one
+//     writes its outputs straight to memory: only the exchanges between stages
+//     go through LDS (128 = 16 x 8: one exchange, 2 LDS accesses per value,
+//     where stages that work in place in LDS take 6);
+//   * an inverse transform's results can be updated in place and transformed
+//     forward again without leaving the registers.
+//
+// The mapping of threads to (l, p0) is line-fastest or position-fastest and
+// may change at an exchange: a wave reads and writes runs of consecutive lines
+// on an axis where lines are neighbours in memory, and runs of consecutive
+// positions where the line is contiguous.
+//
+// Stages, radix order, twiddles and butterflies are those of fft_stages
+// (plan 0) and fft_stages_x (plan 1) of pfdd_fft.hpp, so a line transformed
+// here is bit for bit the line transformed there.
+#pragma once
+#include "pfdd_kern.hpp"
+
+namespace pfdd {
+
+template <int PL> constexpr int plan_radix(int m) { return PL == 1 ? pick_radix_x(m) : pick_radix(m); }
+
+// Exchange tile of NL lines: value (p, l) at an address whose low four bits
+// (the 8-byte slot within 128 bytes of LDS, which serves 16 lanes at a time)
+// are a linear function of the bits of p and l.  It has full rank on every
+// group of 16 lanes that the exchanges use: 16 lines of a row, 8 lines of two
+// rows that are 1, 8 or 16 apart, 16 consecutive positions of a line, 8
+// consecutive positions of two lines.  So there are no bank conflicts and no
+// padding.  The position comes as pv | ps with disjoint bits, ps known at
+// compile time: the ps part folds into constants.
+template <int NL> struct RegSwz {
+    static_assert(NL == 8 || NL % 16 == 0, "tiles of 8 lines or a multiple of 16");
+    __device__ __forceinline__ static constexpr int f(int p)
+    {
+        if constexpr (NL == 8) return (p & 6) | ((p >> 3) & 1) | (((p ^ (p >> 3) ^ (p >> 4)) & 1) << 3);
+        else return ((p & 7) << 1) | ((p >> 3) & 1);
+    }
+    __device__ __forceinline__ static int at(int pv, int ps, int l)
+    {
+        if constexpr (NL == 8) return (pv >> 1) * 16 + ((l ^ f(pv)) ^ f(ps)) + (ps >> 1) * 16;
+        else return pv * NL + ((l ^ f(pv)) ^ f(ps)) + ps * NL;
+    }
+};
+
+// Position written by butterfly j = p0 + D q, output r, of a stage (NS, RAD):
+// (j / NS) NS RAD + j % NS + r NS, split into its thread part and its static
+// part (NS, D powers of two).
+template <int D, int NS, int RAD> struct RegWr {
+    __device__ __forceinline__ static int pv(int p0)
+    {
+        if constexpr (NS <= D) return (p0 / NS) * (NS * RAD) + p0 % NS;
+        else return p0;
+    }
+    __device__ __forceinline__ static constexpr int ps(int q, int r)
+    {
+        if constexpr (NS <= D) return D * RAD * q + r * NS;
+        else return (q / (NS / D)) * (NS * RAD) + D * (q % (NS / D)) + r * NS;
+    }
+};
+
+// LDS of an exchange: FP32 values interleaved (8-byte accesses); FP64 values
+// one component at a time through a single plane of doubles, the real parts
+// first: as many LDS accesses as with two planes (each is 8 bytes wide), half
+// the LDS, two more barriers (none in one-wave blocks).
+template <typename V> struct RegLds;
+template <> struct RegLds<float2> {
+    static constexpr int bytes = 8;
+    float2 *p;
+};
+template <> struct RegLds<double2> {
+    static constexpr int bytes = 8;
+    double *p;
+};
+
+template <int NS, int RAD, int N, int NL, int VPT, bool PFA, bool PFB, bool FIRST, typename V>
+__device__ __forceinline__ void reg_exchange(V (&v)[VPT], RegLds<V> lds, int t)
+{
+    constexpr int D = N / VPT, NB = VPT / RAD;
+    typedef RegSwz<NL> S;
+    typedef RegWr<D, NS, RAD> Wr;
+    const int la = PFA ? t / D : t % NL, pa = PFA ? t % D : t / NL;
+    const int lb = PFB ? t / D : t % NL, pb = PFB ? t % D : t / NL;
+    const int pv = Wr::pv(pa);
+    if constexpr (!FIRST) __syncthreads(); // the last exchange's reads are done
+    if constexpr (sizeof(V) == 8) {
+#pragma unroll
+        for (int q = 0; q < NB; ++q)
+#pragma unroll
+            for (int r = 0; r < RAD; ++r) lds.p[S::at(pv, Wr::ps(q, r), la)] = v[q + NB * r];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) v[m] = lds.p[S::at(pb, D * m, lb)];
+    } else {
+#pragma unroll
+        for (int q = 0; q < NB; ++q)
+#pragma unroll
+            for (int r = 0; r < RAD; ++r) lds.p[S::at(pv, Wr::ps(q, r), la)] = v[q + NB * r].x;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) v[m].x = lds.p[S::at(pb, D * m, lb)];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NB; ++q)
+#pragma unroll
+            for (int r = 0; r < RAD; ++r) lds.p[S::at(pv, Wr::ps(q, r), la)] = v[q + NB * r].y;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) v[m].y = lds.p[S::at(pb, D * m, lb)];
+    }
+}
+
+// The transform of a tile from its natural ownership with mapping PFI
+// (position-fastest or not) to that with mapping PFO.  tws: twiddles of N in
+// LDS, complete before the first exchange's barrier.  FIRST: nothing of the
+// tile's LDS is still being read.
+template <int N, int NS, int PL, int NL, int VPT, bool INV, bool PFI, bool PFO, bool FIRST, typename V>
+__device__ __forceinline__ void reg_fft(V (&v)[VPT], RegLds<V> lds, const V *tws, int t)
+{
+    constexpr int RAD = plan_radix<PL>(N / NS), NB = VPT / RAD, D = N / VPT;
+    static_assert(VPT % RAD == 0, "a thread holds whole butterflies");
+    const int p0 = PFI ? t % D : t / NL;
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+        V x[RAD];
+#pragma unroll
+        for (int r = 0; r < RAD; ++r) x[r] = v[q + NB * r];
+        if constexpr (NS > 1) {
+            const int k = NS <= D ? p0 % NS : p0 + D * (q % (NS > D ? NS / D : 1));
+#pragma unroll
+            for (int r = 1; r < RAD; ++r) x[r] = cmulw<INV>(x[r], tws[r * k * (N / (NS * RAD))]);
+        }
+        dft<RAD, INV>(x);
+#pragma unroll
+        for (int r = 0; r < RAD; ++r) v[q + NB * r] = x[r];
+    }
+    if constexpr (NS * RAD < N) {
+        reg_exchange<NS, RAD, N, NL, VPT, PFI, PFO, FIRST>(v, lds, t);
+        reg_fft<N, NS * RAD, PL, NL, VPT, INV, PFO, PFO, false>(v, lds, tws, t);
+    }
+}
+
+// Twiddles of length N into LDS (complete at the block's next barrier).
+template <int N, int W, typename V>
+__device__ __forceinline__ void reg_twiddles(V *tws, const V *__restrict__ tw, int t)
+{
+#pragma unroll
+    for (int m = 0; m < (N + W - 1) / W; ++m)
+        if (N % W == 0 || t + m * W < N) tws[t + m * W] = tw[t + m * W];
+}
+
+// Line lengths with register transforms: powers of two with two or three
+// stages.  Other lengths (an odd factor, or a single stage) keep the stages in
+// LDS.
+template <int N> constexpr bool reg_length() { return N == 32 || N == 64 || N == 128 || N == 256 || N == 512; }
+
+// Values per thread and lines per tile: runs of 128 bytes or more on both
+// sides of a tile (NL lines, D = N / VPT positions), 64 bytes where that would
+// need more than 16 values per thread or short lines.
+template <typename R, int N> struct RegTile {
+    static constexpr int VPT = N <= 64 ? 8 : 16;
+    static constexpr int NL = sizeof(R) == 8 ? (N == 32 ? 16 : 8) : 16;
+    static constexpr int D = N / VPT, W = NL * D;
+};
+
+} // namespace pfdd

@@ -1,6 +1,7 @@
 // pfdd_update.hip -- the last inverse pass fused with the GL update, and its
 // reverse-mode counterpart, with their launchers.
 #include "pfdd_kern.hpp"
+#include "pfdd_reg.hpp"
 
 namespace pfdd {
 
@@ -130,6 +131,141 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(updat
         if constexpr (FW == 2) fft_stages_x<N, 1, NL, NTHR, false>(lds, tw, t2);
         else fft_stages<N, 1, NL, NTHR, false>(lds, tw, t2);
         tile_store<N, NL, NTHR>(T1, lds, bin, mi.SP, t2);
+    }
+}
+
+// Pass 5 with the transforms held in registers (pfdd_reg.hpp), for the lengths
+// that have them: a thread reads its values of T1 (line-fastest: runs of NL
+// lines), transforms them back, holds after the last stage VPT cells of one
+// row of xi (position-fastest: runs of D cells), updates them in place and,
+// with FW, transforms them forward from the same registers and writes T1.  Two
+// LDS accesses per value and transform are left (six in k_update at 128
+// points) and no barrier at all where a tile is one wave (FP64 up to 128
+// points).  The twiddles sit in LDS: loads from memory would wait, in order,
+// for the streams in flight.
+//
+// NM: terms of the core's sine series, padded to 2, 4 or 8; MA: with an
+// obstacle mask or a per-cell amplitude (whichever is absent is read from one
+// constant element: mstep, astep 0).
+template <typename R, int N, int PL, bool FW, int NM, bool MA>
+__global__ void __launch_bounds__((RegTile<R, N>::W)) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 4, 8)))
+    k_update_r(typename cvec<R>::type *T1, const typename cvec<R>::type *__restrict__ xo,
+               typename cvec<R>::type *__restrict__ xn, const uint8_t *__restrict__ mask,
+               const long long *__restrict__ prev, const R *__restrict__ amp, unsigned mstep, unsigned astep,
+               unsigned ny, unsigned lines_per_sys, StepParams P, const typename cvec<R>::type *__restrict__ tw, double *__restrict__ partial,
+               long long pstride, const int *__restrict__ done)
+{
+    typedef typename cvec<R>::type V;
+    typedef RegTile<R, N> G;
+    constexpr int NL = G::NL, VPT = G::VPT, D = G::D, W = G::W, NW = (W + 63) / 64;
+    if (*done) return;
+    __shared__ __align__(16) char mem[N * NL * RegLds<V>::bytes];
+    __shared__ V tws[N];
+    __shared__ double red[4 * NW];
+    RegLds<V> lds{(decltype(RegLds<V>::p))mem};
+    const int t = threadIdx.x;
+    // lines L = (a nx + i) ny + j; a tile may cross rows of j
+    const unsigned L0 = blockIdx.x * NL, r0 = L0 / ny;
+    V v[VPT];
+    unsigned o1; // byte offset of this thread's first value from the tile's T1 row
+    V *const T1b = T1 + (long long)r0 * ny * N;
+    {
+        const unsigned l = t % NL, p0 = t / NL;
+        const unsigned j = L0 - r0 * ny + l, row = j / ny;
+        o1 = (row * ny * N + (j - row * ny) + p0 * ny) * (unsigned)sizeof(V);
+#pragma unroll
+        for (int m = 0; m < VPT; ++m)
+            v[m] = ld_stream((const V *)((const char *)(T1b + (size_t)(D * m) * ny) + o1));
+    }
+    reg_twiddles<N, W>(tws, tw, t);
+    const unsigned l = t / D, p0 = t % D;
+    const unsigned a = (L0 + l) / lines_per_sys; // system in the batch
+    // this thread's line: its stress and core coefficients
+    const R tau = (R)(P.taud ? P.taud[a] : P.tau[a]);
+    const double *const cf = P.coef + (a % P.S) * MAXM;
+    R lc[NM], ldp[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+        lc[m] = (R)cf[m];
+        ldp[m] = lc[m] * ((R)(m + 1) * (R)M_PI);
+    }
+    const long long base = (long long)L0 * N;
+    const unsigned o2 = l * N + p0;
+    // the old field comes in chunks of CH cells, AHEAD chunks before the update
+    // (the first one during the transform): enough bytes in flight with 3-4
+    // waves per SIMD, where holding all of it costs the registers of one
+    constexpr int CH = 2, AHEAD = 1, NCK = VPT / CH;
+    V x[AHEAD + 1][CH];
+    auto fetch = [&](int ck) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) x[ck % (AHEAD + 1)][c] = ld_stream(xo + base + o2 + D * (ck * CH + c));
+    };
+#pragma unroll
+    for (int ck = 0; ck < AHEAD; ++ck) fetch(ck);
+    reg_fft<N, 1, PL, NL, VPT, true, false, true, true>(v, lds, tws, t);
+
+    const R cddt = (R)P.cddt, invN = (R)P.invN;
+    // a thread sums its VPT cells in FP64; block and grid levels as in k_update
+    double s_norm = 0.0, s_ave = 0.0, s_core = 0.0, s_str = 0.0;
+    unsigned frozen = 0; // this thread's masked cells
+#pragma unroll
+    for (int ck = 0; ck < NCK; ++ck) {
+        // one chunk's temporaries at a time
+        __builtin_amdgcn_sched_barrier(0);
+        if (ck + AHEAD < NCK) fetch(ck + AHEAD);
+        const V *xc = x[ck % (AHEAD + 1)];
+        unsigned fz = 0;
+        R A[CH];
+        if constexpr (MA) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                const long long at = base + D * (ck * CH + c); // uniform; o2 is the lane's offset
+                fz |= (unsigned)(mask + at * mstep)[o2 * mstep] << c; // 0 or 1
+                A[c] = (amp + at * astep)[o2 * astep];
+            }
+            frozen |= fz << (ck * CH);
+        }
+        V y[CH];
+        R dens[CH];
+        double dn[CH];
+        gl_update_chunk<R, NM, MA, CH>(&v[ck * CH], xc, A, fz, tau, lc, ldp, cddt, invN, y, dn, dens);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            st_stream(&xn[base + o2 + D * (ck * CH + c)], y[c]);
+            v[ck * CH + c] = y[c];
+            s_norm += dn[c];
+            s_ave += (double)y[c].x;
+            s_core += (double)dens[c];
+            s_str += (double)tau * (double)xc[c].x;
+        }
+        // the sums are formed here: sunk to their use behind the next branch
+        // they would keep every cell's values in registers until then
+        __asm__ volatile("" : "+v"(s_norm), "+v"(s_ave), "+v"(s_core), "+v"(s_str));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // quirk Q3: a masked cell's xinorm term takes the previous unmasked cell
+    while (MA && frozen) {
+        const unsigned m = __builtin_ctz(frozen);
+        frozen &= frozen - 1;
+        const long long idx = base + o2 + D * m, pi = prev[idx];
+        const V xm = xo[idx], pv = pi >= 0 ? xo[pi] : mk<V>((R)0, (R)0);
+        const double dr = (double)xm.x - (double)pv.x, di = (double)xm.y - (double)pv.y;
+        s_norm += dr * dr + di * di;
+    }
+    if constexpr (FW) {
+        // a thread index the compiler cannot trace: addresses are formed again
+        // instead of held in registers through the update
+        int t2 = t;
+        __asm__ volatile("" : "+v"(t2));
+        reg_fft<N, 1, PL, NL, VPT, false, true, false, false>(v, lds, tws, t2);
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) st_stream((V *)((char *)(T1b + (size_t)(D * m) * ny) + o1), v[m]);
+    }
+    double sum[4] = {s_norm, s_ave, s_core, s_str};
+    block_sum_comp<4, W>(sum, red, t);
+    if (t == 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) partial[q * pstride + blockIdx.x] = sum[q];
     }
 }
 
@@ -267,41 +403,86 @@ __global__ void __launch_bounds__(NTHR)
 }
 
 
+template <typename R> int update_lines(int n, int tq, int model)
+{
+    const bool gen = model == PFDD_CORE_EXTENDED || model == PFDD_CORE_PYRII || model == PFDD_CORE_FOURIER;
+#define PFDD_CASE(n_) if (n == n_ && reg_length<n_>() && !gen) return RegTile<R, n_>::NL;
+    PFDD_SIZES(PFDD_CASE)
+#undef PFDD_CASE
+    return tile_lines_rt<R>(n, tq);
+}
+
 template <typename R>
-hipError_t launch_update(int n, int tq, int fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
+hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
                          const long long *prev, const void *amp, LineMap mi, LineMap mo, long long nlines,
-                         long long lps, const StepParams &P, const void *tw, double *partial,
+                         long long lps, const StepParams &P, const void *tw, const UpdNone *none, double *partial,
                          long long pstride, const int *done, hipStream_t st)
 {
     typedef typename cvec<R>::type V;
+    const uint8_t *no_mask = &none->zero;
+    const R *no_amp = sizeof(R) == 8 ? (const R *)&none->one64 : (const R *)&none->one32;
+    (void)no_mask;
+    (void)no_amp;
     // the coupled and Fourier core models get their own instantiation (one
     // tile shape) so that the common sine-series kernel carries none of
     // their registers
     const bool gen = P.model == PFDD_CORE_EXTENDED || P.model == PFDD_CORE_PYRII || P.model == PFDD_CORE_FOURIER;
     // plan 1 falls back to plan 0 where the two coincide
+#define PFDD_UPR_(PL_, FW_, NM_, MA_)                                                                \
+    PFDD_LAUNCH((k_update_r<R, N, (PL_ && radix16_plan_differs<N>()), FW_, NM_, MA_>),               \
+                dim3((unsigned)(nlines / RegTile<R, N>::NL)), dim3(RegTile<R, N>::W), st, (V *)T1,   \
+                (const V *)xo, (V *)xn, mask ? mask : no_mask, prev,                                 \
+                amp ? (const R *)amp : no_amp, mask ? 1u : 0u, amp ? 1u : 0u, (unsigned)mi.D,        \
+                (unsigned)lps, P, (const V *)tw, partial, pstride, done)
+#define PFDD_UPR(PL_, FW_)                                                                           \
+    do {                                                                                             \
+        if (mask || amp) {                                                                           \
+            if (P.ncoef <= 2) PFDD_UPR_(PL_, FW_, 2, true);                                          \
+            else if (P.ncoef <= 4) PFDD_UPR_(PL_, FW_, 4, true);                                     \
+            else PFDD_UPR_(PL_, FW_, 8, true);                                                       \
+        } else {                                                                                     \
+            if (P.ncoef <= 2) PFDD_UPR_(PL_, FW_, 2, false);                                         \
+            else if (P.ncoef <= 4) PFDD_UPR_(PL_, FW_, 4, false);                                    \
+            else PFDD_UPR_(PL_, FW_, 8, false);                                                      \
+        }                                                                                            \
+    } while (0)
 #define PFDD_UPD(TQ_, GEN_, FW_)                                                                     \
     PFDD_LAUNCH((k_update<R, N, TQ_, GEN_, FW_>),                                                    \
                 dim3((unsigned)((nlines + tile_lines_u<R, N, TQ_>() - 1) / tile_lines_u<R, N, TQ_>())), \
                 dim3(NTHR), st, (V *)T1, (const V *)xo, (V *)xn, mask, prev, (const R *)amp, mi, mo, \
                 nlines, lps, P, (const V *)tw, partial, pstride, done)
 #define PFDD_UPD_FW(TQ_, GEN_)                                                                       \
-    if (fw == 0) PFDD_UPD(TQ_, GEN_, 0);                                                             \
-    else if (fw == 2 && radix16_plan_differs<N>()) PFDD_UPD(TQ_, GEN_, (radix16_plan_differs<N>() ? 2 : 1)); \
+    if (!fw) PFDD_UPD(TQ_, GEN_, 0);                                                                 \
+    else if (plan == 1 && radix16_plan_differs<N>()) PFDD_UPD(TQ_, GEN_, (radix16_plan_differs<N>() ? 2 : 1)); \
     else PFDD_UPD(TQ_, GEN_, 1)
 #define PFDD_CASE(n_)                                                                                \
     if (n == n_) {                                                                                   \
         constexpr int N = n_;                                                                        \
+        if constexpr (reg_length<N>()) {                                                             \
+            if (!gen) {                                                                              \
+                const bool p1 = plan == 1 && radix16_plan_differs<N>();                              \
+                if (p1 && fw) PFDD_UPR(1, true);                                                     \
+                else if (p1) PFDD_UPR(1, false);                                                     \
+                else if (fw) PFDD_UPR(0, true);                                                      \
+                else PFDD_UPR(0, false);                                                             \
+                return hipGetLastError();                                                            \
+            }                                                                                        \
+        }                                                                                            \
         if (gen) {                                                                                   \
             PFDD_UPD_FW(0, true);                                                                    \
             return hipGetLastError();                                                                \
         }                                                                                            \
-        PFDD_TQ_DISPATCH(tq, { PFDD_UPD_FW(TQ, false); })                                            \
+        if constexpr (!reg_length<N>()) {                                                            \
+            PFDD_TQ_DISPATCH(tq, { PFDD_UPD_FW(TQ, false); })                                        \
+        }                                                                                            \
         return hipGetLastError();                                                                    \
     }
     PFDD_SIZES(PFDD_CASE)
 #undef PFDD_CASE
 #undef PFDD_UPD_FW
 #undef PFDD_UPD
+#undef PFDD_UPR
+#undef PFDD_UPR_
     return hipErrorInvalidValue;
 }
 
@@ -329,10 +510,11 @@ hipError_t launch_adj_update(int n, int tq, const void *T1, const void *lam, con
 }
 
 #define PFDD_INST(R)                                                                                          \
-    template hipError_t launch_update<R>(int, int, int, void *, const void *, void *, const uint8_t *,           \
+    template int update_lines<R>(int, int, int);                                                                      \
+    template hipError_t launch_update<R>(int, int, int, bool, void *, const void *, void *, const uint8_t *,           \
                                          const long long *, const void *, LineMap, LineMap, long long, long long, \
-                                         const StepParams &, const void *, double *, long long, const int *,      \
-                                         hipStream_t);                                                            \
+                                         const StepParams &, const void *, const UpdNone *, double *, long long,   \
+                                         const int *, hipStream_t);                                               \
     template hipError_t launch_adj_update<R>(int, int, const void *, const void *, const void *, void *,         \
                                              const uint8_t *, const void *, LineMap, LineMap, long long,          \
                                              long long, const StepParams &, const void *, double *, long long,    \
