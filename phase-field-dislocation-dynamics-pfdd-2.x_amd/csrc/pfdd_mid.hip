@@ -1,6 +1,7 @@
 // pfdd_mid.hip -- the x pass: FFT along x, Green's-function contraction,
 // inverse FFT along x (stored-B and on-the-fly variants), and launchers.
 #include "pfdd_kern.hpp"
+#include "pfdd_reg.hpp"
 
 namespace pfdd {
 
@@ -127,7 +128,7 @@ __global__ void __launch_bounds__(NTHR)
     for (int e = tid; e < TOT; e += NTHR) {
         const int l = e / N, p = e % N;
         const int a = l / NP, q = l % NP;
-        if (c0 + q < ncol) st_stream(&T2[(long long)a * ntot + (c0 + q) * N + p], lds.ld(p * LDP + l));
+        if (c0 + q < ncol) T2[(long long)a * ntot + (c0 + q) * N + p] = lds.ld(p * LDP + l);
     }
     double v[1] = {el};
     block_sum_comp<1, NTHR>(v, red, tid);
@@ -158,6 +159,36 @@ template <typename T> struct GConst {
     T inv2C44, inv1mnu, invmu, C44x2, C12;
 };
 
+// Sig -> P = Sig - 2 C44 Q - C12 tr(Q) I at one k-point (real and imaginary
+// part; symmetric components xx, yy, zz, xy, xz, yz).  The order of every sum
+// of products is written out (ab_cd), so that all x-pass variants round alike.
+template <typename T>
+__device__ __forceinline__ void otf_green(T Pr[6], T Pi[6], const T f[3], T c2, T c4, const GConst<T> &G)
+{
+    auto dot3 = [](T a0, T a1, T a2, const T *b) { return ab_cd(a2, b[2], (T)1, ab_cd(a1, b[1], a0, b[0])); };
+    const T wr[3] = {dot3(Pr[0], Pr[3], Pr[4], f), dot3(Pr[3], Pr[1], Pr[5], f), dot3(Pr[4], Pr[5], Pr[2], f)};
+    const T wi[3] = {dot3(Pi[0], Pi[3], Pi[4], f), dot3(Pi[3], Pi[1], Pi[5], f), dot3(Pi[4], Pi[5], Pi[2], f)};
+    const T Vr = dot3(wr[0], wr[1], wr[2], f), Vi = dot3(wi[0], wi[1], wi[2], f);
+    // c2 multiplies (w_i f_j + w_j f_i), c4 multiplies V f_i f_j
+    const int ci[6] = {0, 1, 2, 0, 0, 1}, cj[6] = {0, 1, 2, 1, 2, 2};
+    const T vr = c4 * Vr, vi = c4 * Vi;
+    T Qr[6], Qi[6];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        const T ff = f[ci[c]] * f[cj[c]];
+        const T sr = ab_cd(wr[ci[c]], f[cj[c]], wr[cj[c]], f[ci[c]]);
+        const T si = ab_cd(wi[ci[c]], f[cj[c]], wi[cj[c]], f[ci[c]]);
+        Qr[c] = ab_cd(c2, sr, -vr, ff);
+        Qi[c] = ab_cd(c2, si, -vi, ff);
+    }
+    const T tr_r = G.C12 * (Qr[0] + Qr[1] + Qr[2]), tr_i = G.C12 * (Qi[0] + Qi[1] + Qi[2]);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        Pr[c] -= ab_cd(G.C44x2, Qr[c], (T)1, c < 3 ? tr_r : (T)0);
+        Pi[c] -= ab_cd(G.C44x2, Qi[c], (T)1, c < 3 ? tr_i : (T)0);
+    }
+}
+
 // Hands ghat_a for a = H*SA .. H*SA+SA-1 of one k-point to sink(aa, re, im,
 // xihat_a), computed in T (double in the FP64 path, float in the FP32 mode).
 // xihat_a is the value read for the contraction, kept in registers so that
@@ -183,30 +214,7 @@ __device__ __forceinline__ void otf_point(const Tile<V> lds, int p, int q, const
             Pi[c] += cst[b * 12 + c] * xi;
         }
     }
-    if (nzf) {
-        // symmetric components xx, yy, zz, xy, xz, yz
-        const T wr[3] = {Pr[0] * f[0] + Pr[3] * f[1] + Pr[4] * f[2], Pr[3] * f[0] + Pr[1] * f[1] + Pr[5] * f[2],
-                              Pr[4] * f[0] + Pr[5] * f[1] + Pr[2] * f[2]};
-        const T wi[3] = {Pi[0] * f[0] + Pi[3] * f[1] + Pi[4] * f[2], Pi[3] * f[0] + Pi[1] * f[1] + Pi[5] * f[2],
-                              Pi[4] * f[0] + Pi[5] * f[1] + Pi[2] * f[2]};
-        const T Vr = f[0] * wr[0] + f[1] * wr[1] + f[2] * wr[2];
-        const T Vi = f[0] * wi[0] + f[1] * wi[1] + f[2] * wi[2];
-        // c2 multiplies (w_i f_j + w_j f_i), c4 multiplies V f_i f_j
-        const int ci[6] = {0, 1, 2, 0, 0, 1}, cj[6] = {0, 1, 2, 1, 2, 2};
-        T Qr[6], Qi[6];
-#pragma unroll
-        for (int c = 0; c < 6; ++c) {
-            const T ff = f[ci[c]] * f[cj[c]];
-            Qr[c] = c2 * (wr[ci[c]] * f[cj[c]] + wr[cj[c]] * f[ci[c]]) - c4 * Vr * ff;
-            Qi[c] = c2 * (wi[ci[c]] * f[cj[c]] + wi[cj[c]] * f[ci[c]]) - c4 * Vi * ff;
-        }
-        const T tr_r = G.C12 * (Qr[0] + Qr[1] + Qr[2]), tr_i = G.C12 * (Qi[0] + Qi[1] + Qi[2]);
-#pragma unroll
-        for (int c = 0; c < 6; ++c) {
-            Pr[c] -= G.C44x2 * Qr[c] + (c < 3 ? tr_r : (T)0);
-            Pi[c] -= G.C44x2 * Qi[c] + (c < 3 ? tr_i : (T)0);
-        }
-    }
+    if (nzf) otf_green(Pr, Pi, f, c2, c4, G);
 #pragma unroll
     for (int aa = 0; aa < SA; ++aa) {
         __asm__ volatile("" ::: "memory");
@@ -251,10 +259,11 @@ __device__ __forceinline__ void otf_freq(const GParams &G, long long col, int p,
     const double kx = fr(p, G.nx, G.inv_n[0]), ky = fr(j, G.ny, G.inv_n[1]), kz = fr(k, G.nz, G.inv_n[2]);
     double fd[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) fd[c] = kx * G.four[c] + ky * G.four[3 + c] + kz * G.four[6 + c];
+    for (int c = 0; c < 3; ++c)
+        fd[c] = ab_cd(kz, G.four[6 + c], 1.0, ab_cd(ky, G.four[3 + c], kx, G.four[c]));
 #pragma unroll
     for (int c = 0; c < 3; ++c) f[c] = (T)fd[c];
-    const double f2 = fd[0] * fd[0] + fd[1] * fd[1] + fd[2] * fd[2];
+    const double f2 = ab_cd(fd[2], fd[2], 1.0, ab_cd(fd[1], fd[1], fd[0], fd[0]));
     nzf = f2 > 0;
     const double if2 = nzf ? 1.0 / f2 : 0.0;
     c2 = (T)(if2 * G.inv2C44);
@@ -537,10 +546,191 @@ __global__ void __launch_bounds__(NTHR)
 }
 
 
+// Tile of the register x pass: NP columns of S systems, W = S NP D threads of
+// VPT values, 192 threads for 3, 6 and 12 systems (384 for 12 systems of 512
+// points) and 128 for 1, 2 and 4.
+template <int N, int S> struct XTile {
+    static constexpr int VPT = N <= 64 ? 8 : 16, D = N / VPT;
+    static constexpr int pairs()
+    {
+        int np = 1;
+        while (2 * np * S * D <= 192) np *= 2;
+        return np;
+    }
+    static constexpr int NP = pairs(), NL = S * NP, W = NL * D;
+    static constexpr int PTS = (NP * N + W - 1) / W; // k-points per thread of the contraction
+};
+
+// x pass with the transforms in registers (pfdd_reg.hpp): natural ownership,
+// position-fastest, straight from memory into the first stage and from the last
+// stage back; through LDS go the exchanges between stages and the turn from
+// lines to k-points and back (every thread contracts whole k-points): 8 LDS
+// accesses per value at 128 and 256 points, 12 with the stages in LDS.  The
+// FP64 tile is one plane of doubles (real parts, then imaginary parts), half
+// the LDS of k_mid_otf for the same columns.
+template <typename R, int N, int S>
+__global__ void __launch_bounds__((XTile<N, S>::W)) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 4, 8)))
+    k_mid_r(typename cvec<R>::type *__restrict__ T2, GParams G, long long ncol, long long ntot, int bpm,
+            const typename cvec<R>::type *__restrict__ tw, double *__restrict__ part_el, const int *__restrict__ done)
+{
+    typedef typename cvec<R>::type V;
+    typedef XTile<N, S> X;
+    constexpr int NP = X::NP, NL = X::NL, VPT = X::VPT, D = X::D, W = X::W, PTS = X::PTS, NW = (W + 63) / 64;
+    typedef RegSwzX<N> L;
+    typedef RegNat<N, NL, VPT, true, L> Nat;
+    if (*done) return;
+    __shared__ __align__(16) char mem[N * NL * RegLds<V>::bytes];
+    __shared__ V tws[N];
+    __shared__ R cst[S * 12];
+    __shared__ double red[NW];
+    RegLds<V> lds{(decltype(RegLds<V>::p))mem};
+    const int t = threadIdx.x;
+    // member of a batch (bpm blocks per member), first column of the block
+    const int mem_b = blockIdx.x / bpm;
+    const long long c0 = (long long)(blockIdx.x - mem_b * bpm) * NP;
+    T2 += (long long)mem_b * S * ntot + c0 * N; // the NP columns of a system are contiguous
+    const int l = t / D;                        // line (a, q)
+    V *const own = T2 + (long long)(l / NP) * ntot + (l % NP) * N + t % D;
+    V v[VPT];
+#pragma unroll
+    for (int m = 0; m < VPT; ++m) v[m] = ld_stream(own + D * m);
+    reg_twiddles<N, W>(tws, tw, t);
+    GConst<R> gc;
+    for (int c = t; c < S * 12; c += W) cst[c] = (R)((c % 12) < 6 ? G.sig6[(c / 12) * 6 + c % 12]
+                                                                 : G.eps6[(c / 12) * 6 + c % 12 - 6]);
+    gc = GConst<R>{(R)G.inv2C44, (R)G.inv1mnu, (R)G.invmu, (R)G.C44x2, (R)G.C12};
+    reg_fft<N, 1, 1, NL, VPT, false, true, true, true, L>(v, lds, tws, t);
+    // lines -> k-points: slot i S + a of a thread is system a of point t + W i
+    V x[PTS * S];
+    int at[PTS];
+    bool ok[PTS];
+#pragma unroll
+    for (int i = 0; i < PTS; ++i) {
+        const int pt = t + W * i;
+        ok[i] = (NP * N) % W == 0 || pt < NP * N;
+        at[i] = ok[i] ? L::at(pt % N, 0, pt / N) : 0;
+    }
+    constexpr int AS = NP * N; // from one system to the next
+    const Nat nat(t);
+    __syncthreads();
+    if constexpr (sizeof(V) == 8) {
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) lds.p[nat(m)] = v[m];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PTS; ++i)
+#pragma unroll
+            for (int a = 0; a < S; ++a) x[i * S + a] = lds.p[at[i] + a * AS];
+    } else {
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) lds.p[nat(m)] = v[m].x;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PTS; ++i)
+#pragma unroll
+            for (int a = 0; a < S; ++a) x[i * S + a].x = lds.p[at[i] + a * AS];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) lds.p[nat(m)] = v[m].y;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PTS; ++i)
+#pragma unroll
+            for (int a = 0; a < S; ++a) x[i * S + a].y = lds.p[at[i] + a * AS];
+    }
+    // the contraction of each point in place; the elastic-energy term
+    // Re(conj(xihat_a) ghat_a) is taken as each ghat_a replaces xihat_a
+    double el = 0.0;
+#pragma unroll
+    for (int i = 0; i < PTS; ++i) {
+        if (ok[i]) {
+            // compiler-only barriers keep the (LDS-broadcast) constants from
+            // being held in registers across points and systems
+            __asm__ volatile("" ::: "memory");
+            const int pt = t + W * i;
+            R f[3], c2, c4;
+            bool nzf;
+            otf_freq<N, NP, S, R>(G, c0 + pt / N, pt % N, f, nzf, c2, c4);
+            R Pr[6] = {}, Pi[6] = {};
+#pragma unroll
+            for (int b = 0; b < S; ++b)
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    Pr[c] += cst[b * 12 + c] * x[i * S + b].x;
+                    Pi[c] += cst[b * 12 + c] * x[i * S + b].y;
+                }
+            if (nzf) otf_green(Pr, Pi, f, c2, c4, gc);
+#pragma unroll
+            for (int a = 0; a < S; ++a) {
+                __asm__ volatile("" ::: "memory");
+                R gr = 0, gi = 0;
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    gr += Pr[c] * cst[a * 12 + 6 + c];
+                    gi += Pi[c] * cst[a * 12 + 6 + c];
+                }
+                gr *= gc.invmu;
+                gi *= gc.invmu;
+                if (!nzf) gr = gi = (R)0;
+                el += (double)x[i * S + a].x * gr + (double)x[i * S + a].y * gi;
+                x[i * S + a] = mk<V>(gr, gi);
+            }
+        }
+        // formed here, not sunk past the next branch with every point alive
+        __asm__ volatile("" : "+v"(el));
+    }
+    __syncthreads();
+    if constexpr (sizeof(V) == 8) {
+#pragma unroll
+        for (int i = 0; i < PTS; ++i)
+#pragma unroll
+            for (int a = 0; a < S; ++a)
+                if (ok[i]) lds.p[at[i] + a * AS] = x[i * S + a];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) v[m] = lds.p[nat(m)];
+    } else {
+#pragma unroll
+        for (int i = 0; i < PTS; ++i)
+#pragma unroll
+            for (int a = 0; a < S; ++a)
+                if (ok[i]) lds.p[at[i] + a * AS] = x[i * S + a].x;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) v[m].x = lds.p[nat(m)];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PTS; ++i)
+#pragma unroll
+            for (int a = 0; a < S; ++a)
+                if (ok[i]) lds.p[at[i] + a * AS] = x[i * S + a].y;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < VPT; ++m) v[m].y = lds.p[nat(m)];
+    }
+    int t2 = t;
+    __asm__ volatile("" : "+v"(t2)); // addresses formed again, as in k_update_r
+    reg_fft<N, 1, 1, NL, VPT, true, true, true, false, L>(v, lds, tws, t2);
+#pragma unroll
+    for (int m = 0; m < VPT; ++m) st_stream(own + D * m, v[m]);
+    double sum[1] = {el};
+    block_sum_comp<1, W>(sum, red, t);
+    if (t == 0) part_el[blockIdx.x] = sum[0];
+}
+
 template <typename R, int S>
 int mid_blocks_rt(int n, long long ncol)
 {
-#define PFDD_CASE(n_) if (n == n_) return (int)((ncol + mid_pairs<R, n_, S>() - 1) / mid_pairs<R, n_, S>());
+    // the most blocks of any x-pass kernel of this length: sizes the partials
+#define PFDD_CASE(n_)                                                                           \
+    if (n == n_) {                                                                              \
+        const int nb = (int)((ncol + mid_pairs<R, n_, S>() - 1) / mid_pairs<R, n_, S>());       \
+        if constexpr (reg_length<n_>()) {                                                       \
+            const int nr = (int)(ncol / XTile<n_, S>::NP);                                      \
+            return nb > nr ? nb : nr;                                                           \
+        }                                                                                       \
+        return nb;                                                                              \
+    }
     PFDD_SIZES(PFDD_CASE)
 #undef PFDD_CASE
     return 0;
@@ -631,7 +821,15 @@ hipError_t launch_mid_otf_s(int n, int M, void *T2, const GParams &G, long long 
     typedef typename cvec<R>::type V;
 #define PFDD_CASE(n_)                                                                             \
     if (n == n_) {                                                                                \
-        if constexpr (mid_fits<R, n_, S>()) {                                                     \
+        if constexpr (mid_fits<R, n_, S>() && reg_length<n_>()) {                                 \
+            typedef XTile<n_, S> X;                                                               \
+            if (ncol % X::NP) return hipErrorInvalidValue;                                        \
+            const int bpm = (int)(ncol / X::NP);                                                  \
+            *nblocks = M * bpm;                                                                   \
+            PFDD_LAUNCH((k_mid_r<R, n_, S>), dim3((unsigned)*nblocks), dim3(X::W), st, (V *)T2, G, \
+                        ncol, ntot, bpm, (const V *)tw, part_el, done);                           \
+            return hipGetLastError();                                                             \
+        } else if constexpr (mid_fits<R, n_, S>()) {                                              \
             constexpr int NP = mid_pairs<R, n_, S>();                                             \
             const int bpm = (int)((ncol + NP - 1) / NP);                                          \
             if (!pipe) {                                                                          \

@@ -51,6 +51,30 @@ template <int NL> struct RegSwz {
     }
 };
 
+// Exchange tile of the x pass, whose lines are all contiguous: line by line,
+// the low four bits of the position XORed so that 16 lanes of any of its
+// accesses (consecutive positions of one line, or of neighbouring lines where
+// a line has fewer than 16 threads; stage outputs RAD apart) hit 16 slots.
+template <int N> struct RegSwzX {
+    __device__ __forceinline__ static constexpr int f(int p) // of position bits 4 and up
+    {
+        const int p4 = (p >> 4) & 1, p5 = (p >> 5) & 1, p6 = (p >> 6) & 1, p7 = (p >> 7) & 1;
+        if constexpr (N >= 256) return p4 | (p5 << 1) | (p6 * 12) ^ (p7 << 2);
+        else return p4 | (p5 << 1) | (p6 << 2);
+    }
+    __device__ __forceinline__ static constexpr int g(int l) // of the line
+    {
+        if constexpr (N >= 256) return 0;
+        else if constexpr (N == 128) return (l & 1) << 3;
+        else if constexpr (N == 64) return (l & 1) * 12;
+        else return ((l & 1) << 2) | ((l & 2) * 5); // N == 32: bit 0 -> 4, bit 1 -> 8 + 2
+    }
+    __device__ __forceinline__ static int at(int pv, int ps, int l)
+    {
+        return l * N + (((pv ^ f(pv)) ^ g(l)) ^ ((ps & 15) ^ f(ps))) + (ps & ~15);
+    }
+};
+
 // Position written by butterfly j = p0 + D q, output r, of a stage (NS, RAD):
 // (j / NS) NS RAD + j % NS + r NS, split into its thread part and its static
 // part (NS, D powers of two).
@@ -81,48 +105,82 @@ template <> struct RegLds<double2> {
     double *p;
 };
 
-template <int NS, int RAD, int N, int NL, int VPT, bool PFA, bool PFB, bool FIRST, typename V>
-__device__ __forceinline__ void reg_exchange(V (&v)[VPT], RegLds<V> lds, int t)
+// All values of the block through LDS: slot m goes to address wr(m) and comes
+// back from address rd(m).  FIRST: nothing of the tile's LDS is being read.
+template <int VPT, bool FIRST, typename V, typename WrA, typename RdA>
+__device__ __forceinline__ void reg_shuffle(V (&v)[VPT], RegLds<V> lds, WrA wr, RdA rd)
 {
-    constexpr int D = N / VPT, NB = VPT / RAD;
-    typedef RegSwz<NL> S;
-    typedef RegWr<D, NS, RAD> Wr;
-    const int la = PFA ? t / D : t % NL, pa = PFA ? t % D : t / NL;
-    const int lb = PFB ? t / D : t % NL, pb = PFB ? t % D : t / NL;
-    const int pv = Wr::pv(pa);
     if constexpr (!FIRST) __syncthreads(); // the last exchange's reads are done
     if constexpr (sizeof(V) == 8) {
 #pragma unroll
-        for (int q = 0; q < NB; ++q)
-#pragma unroll
-            for (int r = 0; r < RAD; ++r) lds.p[S::at(pv, Wr::ps(q, r), la)] = v[q + NB * r];
+        for (int m = 0; m < VPT; ++m) lds.p[wr(m)] = v[m];
         __syncthreads();
 #pragma unroll
-        for (int m = 0; m < VPT; ++m) v[m] = lds.p[S::at(pb, D * m, lb)];
+        for (int m = 0; m < VPT; ++m) v[m] = lds.p[rd(m)];
     } else {
 #pragma unroll
-        for (int q = 0; q < NB; ++q)
-#pragma unroll
-            for (int r = 0; r < RAD; ++r) lds.p[S::at(pv, Wr::ps(q, r), la)] = v[q + NB * r].x;
+        for (int m = 0; m < VPT; ++m) lds.p[wr(m)] = v[m].x;
         __syncthreads();
 #pragma unroll
-        for (int m = 0; m < VPT; ++m) v[m].x = lds.p[S::at(pb, D * m, lb)];
+        for (int m = 0; m < VPT; ++m) v[m].x = lds.p[rd(m)];
         __syncthreads();
 #pragma unroll
-        for (int q = 0; q < NB; ++q)
-#pragma unroll
-            for (int r = 0; r < RAD; ++r) lds.p[S::at(pv, Wr::ps(q, r), la)] = v[q + NB * r].y;
+        for (int m = 0; m < VPT; ++m) lds.p[wr(m)] = v[m].y;
         __syncthreads();
 #pragma unroll
-        for (int m = 0; m < VPT; ++m) v[m].y = lds.p[S::at(pb, D * m, lb)];
+        for (int m = 0; m < VPT; ++m) v[m].y = lds.p[rd(m)];
     }
 }
+
+// LDS address of slot m in natural ownership; S the tile's layout.
+template <int N, int NL, int VPT, bool PF, typename S = RegSwz<NL>> struct RegNat {
+    static constexpr int D = N / VPT;
+    int l, p0;
+    __device__ __forceinline__ RegNat(int t) : l(PF ? t / D : t % NL), p0(PF ? t % D : t / NL) {}
+    __device__ __forceinline__ int operator()(int m) const { return S::at(p0, D * m, l); }
+};
+// ... after stage (NS, RAD): slot q + NB r holds output r of butterfly q.
+template <int NS, int RAD, int N, int NL, int VPT, bool PF, typename S = RegSwz<NL>> struct RegOut {
+    static constexpr int D = N / VPT, NB = VPT / RAD;
+    int l, pv;
+    __device__ __forceinline__ RegOut(int t)
+        : l(PF ? t / D : t % NL), pv(RegWr<D, NS, RAD>::pv(PF ? t % D : t / NL))
+    {
+    }
+    __device__ __forceinline__ int operator()(int m) const
+    {
+        return S::at(pv, RegWr<D, NS, RAD>::ps(m % NB, m / NB), l);
+    }
+};
+// ... in linear ownership: slot m holds element t + W m of the tile's NL lines
+// in memory order (line by line), so that a wave reads or writes runs of 64
+// positions of contiguous lines.
+template <int N, int NL, int VPT> struct RegLin {
+    static constexpr int W = NL * N / VPT;
+    int t;
+    __device__ __forceinline__ RegLin(int t_) : t(t_) {}
+    __device__ __forceinline__ static int line(int t, int m)
+    {
+        if constexpr (W >= N) return t / N + (W / N) * m;
+        else return m / (N / W);
+    }
+    __device__ __forceinline__ static int pos_s(int m) // the static part of the position; the rest is t % min(N, W)
+    {
+        if constexpr (W >= N) return 0;
+        else return W * (m % (N / W));
+    }
+    __device__ __forceinline__ int operator()(int m) const
+    {
+        return RegSwz<NL>::at(t % (W < N ? W : N), pos_s(m), line(t, m));
+    }
+};
 
 // The transform of a tile from its natural ownership with mapping PFI
 // (position-fastest or not) to that with mapping PFO.  tws: twiddles of N in
 // LDS, complete before the first exchange's barrier.  FIRST: nothing of the
 // tile's LDS is still being read.
-template <int N, int NS, int PL, int NL, int VPT, bool INV, bool PFI, bool PFO, bool FIRST, typename V>
+template <int N, int NS, int PL, int NL, int VPT, bool INV, bool PFI, bool PFO, bool FIRST,
+          typename S = RegSwz<NL>, typename V>
 __device__ __forceinline__ void reg_fft(V (&v)[VPT], RegLds<V> lds, const V *tws, int t)
 {
     constexpr int RAD = plan_radix<PL>(N / NS), NB = VPT / RAD, D = N / VPT;
@@ -143,8 +201,8 @@ __device__ __forceinline__ void reg_fft(V (&v)[VPT], RegLds<V> lds, const V *tws
         for (int r = 0; r < RAD; ++r) v[q + NB * r] = x[r];
     }
     if constexpr (NS * RAD < N) {
-        reg_exchange<NS, RAD, N, NL, VPT, PFI, PFO, FIRST>(v, lds, t);
-        reg_fft<N, NS * RAD, PL, NL, VPT, INV, PFO, PFO, false>(v, lds, tws, t);
+        reg_shuffle<VPT, FIRST>(v, lds, RegOut<NS, RAD, N, NL, VPT, PFI, S>(t), RegNat<N, NL, VPT, PFO, S>(t));
+        reg_fft<N, NS * RAD, PL, NL, VPT, INV, PFO, PFO, false, S>(v, lds, tws, t);
     }
 }
 
@@ -162,12 +220,14 @@ __device__ __forceinline__ void reg_twiddles(V *tws, const V *__restrict__ tw, i
 // LDS.
 template <int N> constexpr bool reg_length() { return N == 32 || N == 64 || N == 128 || N == 256 || N == 512; }
 
-// Values per thread and lines per tile: runs of 128 bytes or more on both
-// sides of a tile (NL lines, D = N / VPT positions), 64 bytes where that would
-// need more than 16 values per thread or short lines.
+// Values per thread and lines per tile of the line passes and the update: 256
+// bytes of neighbouring lines (16 FP64, 32 FP32 lines) where the exchange tile
+// stays within 32 KB, and the 128 bytes of 16 FP32 lines beyond.  Half of that
+// cost the FP64 update at 512 x 512 x 256 x 3 2317 -> 2545 us; twice the LDS
+// cost the FP32 one 1245 -> 1459 us.
 template <typename R, int N> struct RegTile {
     static constexpr int VPT = N <= 64 ? 8 : 16;
-    static constexpr int NL = sizeof(R) == 8 ? (N == 32 ? 16 : 8) : 16;
+    static constexpr int NL = sizeof(R) == 8 ? 16 : (N >= 256 ? 16 : 32);
     static constexpr int D = N / VPT, W = NL * D;
 };
 
