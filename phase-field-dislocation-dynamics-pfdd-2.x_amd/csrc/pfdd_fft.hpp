@@ -32,8 +32,15 @@ template <typename V> __device__ __forceinline__ V csub(V a, V b) { return mk<V>
 // leaves the compiler the choice which one enters the fused multiply-add; it
 // is made here, so that the same line transformed by different kernels rounds
 // alike.
-__device__ __forceinline__ double ab_cd(double a, double b, double c, double d) { return __builtin_fma(a, b, c * d); }
-__device__ __forceinline__ float ab_cd(float a, float b, float c, float d) { return __builtin_fmaf(a, b, c * d); }
+// Likewise ab_c for a product and a sum that may land in different basic blocks.
+__device__ __forceinline__ double ab_c(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float ab_c(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+template <typename R> __device__ __forceinline__ R ab_cd(R a, R b, R c, R d) { return ab_c(a, b, c * d); }
+// a + s b, s real
+template <typename V> __device__ __forceinline__ V caxpy(decltype(V{}.x) s, V b, V a)
+{
+    return mk<V>(ab_c(s, b.x, a.x), ab_c(s, b.y, a.y));
+}
 // a * w (forward) or a * conj(w) (inverse)
 template <bool INV, typename V> __device__ __forceinline__ V cmulw(V a, V w)
 {
@@ -52,11 +59,16 @@ template <bool INV, typename V> __device__ __forceinline__ V cmul_mi(V a)
 // interleaved (8-byte accesses); double2 values are kept as two planes of
 // doubles (re, im) so that every LDS access is 8 bytes wide: 16-byte
 // accesses to the same tile patterns measured heavy bank conflicts.
-// Streaming accesses of the field passes.  Every element is read once and
-// written once per pass, so the loads carry the nontemporal hint (measured on
-// MI355X at 128^3 x 12: FP32 step -17 %, FP64 -6 %).  Stores carry it for
-// 16-byte elements only: for 8-byte elements it slowed the FP32 line passes
-// by a quarter, for 16-byte elements it gained another 3 %.
+// Accesses of the field passes.  Every element is read once per pass, so the
+// loads carry the nontemporal hint (at 128^3 x 12: FP32 step -17 %, FP64 -6 %;
+// plain loads of T1 and T2 cost the FP64 step 4 % and the FP32 one 7 % again).
+// The new field is not read before the end of the next iteration: its stores
+// are nontemporal, which leaves the 256 MB last-level cache to the work fields.
+// Stores to those (st_work) are plain where `keep` is set, because the next
+// kernel reads them and need not fetch from memory what that cache still holds
+// of a field of up to KEEP_BYTES (pfdd_kern.hpp); beyond that they only cost
+// the cache's write traffic, and 16-byte stores are nontemporal as well
+// (8-byte ones never are: the FP32 line passes ran a quarter slower so).
 template <typename V> __device__ __forceinline__ V ld_stream(const V *p)
 {
     typedef decltype(V{}.x) E;
@@ -66,16 +78,18 @@ template <typename V> __device__ __forceinline__ V ld_stream(const V *p)
 }
 template <typename V> __device__ __forceinline__ void st_stream(V *p, V v)
 {
-    if constexpr (sizeof(V) >= 16) {
-        typedef decltype(V{}.x) E;
-        typedef E E2 __attribute__((ext_vector_type(2)));
-        E2 t;
-        t.x = v.x;
-        t.y = v.y;
-        __builtin_nontemporal_store(t, reinterpret_cast<E2 *>(p));
-    } else {
-        *p = v;
-    }
+    typedef decltype(V{}.x) E;
+    typedef E E2 __attribute__((ext_vector_type(2)));
+    E2 t;
+    t.x = v.x;
+    t.y = v.y;
+    __builtin_nontemporal_store(t, reinterpret_cast<E2 *>(p));
+}
+
+template <typename V> __device__ __forceinline__ void st_work(V *p, V v, bool keep)
+{
+    if (sizeof(V) < 16 || keep) *p = v;
+    else st_stream(p, v);
 }
 
 template <typename V> struct Tile;
@@ -129,23 +143,24 @@ template <bool INV, typename V> __device__ __forceinline__ void dft8(V *v)
     dft4<INV>(e);
     dft4<INV>(o);
     const R s = (R)0.707106781186547524400844362104849039;
+    // sqrt(2) times the rotated o[1], o[3]
     V t1, t3;
     if (INV) {
-        t1 = mk<V>(s * (o[1].x - o[1].y), s * (o[1].x + o[1].y));
-        t3 = mk<V>(-s * (o[3].x + o[3].y), s * (o[3].x - o[3].y));
+        t1 = mk<V>(o[1].x - o[1].y, o[1].x + o[1].y);
+        t3 = mk<V>(-(o[3].x + o[3].y), o[3].x - o[3].y);
     } else {
-        t1 = mk<V>(s * (o[1].x + o[1].y), s * (o[1].y - o[1].x));
-        t3 = mk<V>(s * (o[3].y - o[3].x), -s * (o[3].x + o[3].y));
+        t1 = mk<V>(o[1].x + o[1].y, o[1].y - o[1].x);
+        t3 = mk<V>(o[3].y - o[3].x, -(o[3].x + o[3].y));
     }
     V t2 = cmul_mi<INV>(o[2]);
     v[0] = cadd(e[0], o[0]);
     v[4] = csub(e[0], o[0]);
-    v[1] = cadd(e[1], t1);
-    v[5] = csub(e[1], t1);
+    v[1] = caxpy(s, t1, e[1]);
+    v[5] = caxpy(-s, t1, e[1]);
     v[2] = cadd(e[2], t2);
     v[6] = csub(e[2], t2);
-    v[3] = cadd(e[3], t3);
-    v[7] = csub(e[3], t3);
+    v[3] = caxpy(s, t3, e[3]);
+    v[7] = caxpy(-s, t3, e[3]);
 }
 
 template <bool INV, typename V> __device__ __forceinline__ void dft3(V *v)
@@ -155,17 +170,12 @@ template <bool INV, typename V> __device__ __forceinline__ void dft3(V *v)
     V t = cadd(v[1], v[2]);
     V d = csub(v[1], v[2]);
     V y0 = cadd(v[0], t);
-    V m = mk<V>(v[0].x - (R)0.5 * t.x, v[0].y - (R)0.5 * t.y);
+    V m = caxpy((R)-0.5, t, v[0]);
     // forward: y1 = m - i h d, y2 = m + i h d ; inverse swaps
-    V ihd = mk<V>(-h * d.y, h * d.x); // +i h d
+    V id = mk<V>(-d.y, d.x);
     v[0] = y0;
-    if (INV) {
-        v[1] = cadd(m, ihd);
-        v[2] = csub(m, ihd);
-    } else {
-        v[1] = csub(m, ihd);
-        v[2] = cadd(m, ihd);
-    }
+    v[1] = caxpy(INV ? h : -h, id, m);
+    v[2] = caxpy(INV ? -h : h, id, m);
 }
 
 // Length-5 DFT from the symmetric pairs t = x1 + x4, x2 + x3 and the
@@ -184,8 +194,8 @@ template <bool INV, typename V> __device__ __forceinline__ void dft5(V *v)
     const V t1 = cadd(v[1], v[4]), t2 = cadd(v[2], v[3]);
     const V d1 = csub(v[1], v[4]), d2 = csub(v[2], v[3]);
     const V x0 = v[0];
-    const V a1 = mk<V>(x0.x + c1 * t1.x + c2 * t2.x, x0.y + c1 * t1.y + c2 * t2.y);
-    const V a2 = mk<V>(x0.x + c2 * t1.x + c1 * t2.x, x0.y + c2 * t1.y + c1 * t2.y);
+    const V a1 = caxpy(c2, t2, caxpy(c1, t1, x0));
+    const V a2 = caxpy(c1, t2, caxpy(c2, t1, x0));
     const V b1 = mk<V>(ab_cd(s1, d1.x, s2, d2.x), ab_cd(s1, d1.y, s2, d2.y));
     const V b2 = mk<V>(ab_cd(s2, d1.x, -s1, d2.x), ab_cd(s2, d1.y, -s1, d2.y));
     const V ib1 = mk<V>(-b1.y, b1.x), ib2 = mk<V>(-b2.y, b2.x); // i b
@@ -551,7 +561,7 @@ __device__ __forceinline__ void tile_load(const Tile<V> lds, const V *__restrict
 
 template <int N, int NL, int NTHR, typename V>
 __device__ __forceinline__ void tile_store(V *__restrict__ dst, const Tile<V> lds,
-                                           const long long *base, long long SP, int tid)
+                                           const long long *base, long long SP, int tid, bool keep)
 {
     constexpr int LDP = NL + 1, TOT = N * NL;
     if (SP == 1) {
@@ -559,14 +569,14 @@ __device__ __forceinline__ void tile_store(V *__restrict__ dst, const Tile<V> ld
         for (int e = tid; e < TOT; e += NTHR) {
             const int l = e / N, p = e % N;
             const long long b = base[l];
-            if (b >= 0) st_stream(&dst[b + p], lds.ld(p * LDP + l));
+            if (b >= 0) st_work(&dst[b + p], lds.ld(p * LDP + l), keep);
         }
     } else {
 #pragma unroll 4
         for (int e = tid; e < TOT; e += NTHR) {
             const int l = e % NL, p = e / NL;
             const long long b = base[l];
-            if (b >= 0) st_stream(&dst[b + p * SP], lds.ld(p * LDP + l));
+            if (b >= 0) st_work(&dst[b + p * SP], lds.ld(p * LDP + l), keep);
         }
     }
 }

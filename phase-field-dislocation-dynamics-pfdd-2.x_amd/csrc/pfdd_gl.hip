@@ -644,6 +644,7 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
                            (const typename cvec<R>::type *)xo, (R *)h->cof, h->TP, h->N, h->done);
         HIPCHK(hipGetLastError());
     }
+    const Order ord = order_of((size_t)h->SM * h->N * h->esz, (int)h->esz), zord = {ord.keep, false};
     if (h->plane) {
         // plane iteration: 2-D forward pass xo -> T1, x pass on T1 in its
         // plane layout, 2-D inverse pass + update T1 + xo -> T2.  The slots
@@ -677,11 +678,11 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
     if (first) {
         arm(0);
         HIPCHK((launch_pass<R, false>(h->nz, xo, h->T1, m.p1i, m.p1o, m.n1, h->tw[2], h->done, st, nullptr,
-                                      h->tq[0])));
+                                      h->tq[0], zord)));
     }
     arm(1);
     HIPCHK((launch_pass<R, false>(h->ny, h->T1, T2, m.p2i, m.p2o, m.n2, h->tw[1], h->done, st, nullptr,
-                                  h->tq[1])));
+                                  h->tq[1], ord)));
     arm(2);
     if (h->stored_B)
         HIPCHK((launch_mid<R>(h->nx, h->S, h->M, T2, h->B, (long long)h->ny * h->nz, h->N, h->tw[0],
@@ -691,13 +692,13 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
                                   h->partial + 4 * h->pstride, h->done, st, h->xpipe, h->ncu, &h->nb3)));
     arm(3);
     HIPCHK((launch_pass<R, true>(h->ny, T2, h->T1, m.p2o, m.p2i, m.n2, h->tw[1], h->done, st, nullptr,
-                                 h->tq[2])));
+                                 h->tq[2], ord)));
     arm(4);
     // the transform that follows the update takes pass 1's radix plan, so that
     // the field does not depend on how a run is cut into calls
     HIPCHK(launch_update<R>(h->nz, h->tq[3], h->tq[0] / 3, !last, h->T1, xo, T2, h->mask, h->prev,
                             h->cof ? h->cof : h->amp, m.p5i, m.p5o, m.n5, (long long)h->nx * h->ny, P, h->tw[2],
-                            h->none, h->partial, h->pstride, h->done, st));
+                            h->none, ord.keep, h->partial, h->pstride, h->done, st));
     }
     arm(5);
     // E_core as the reference accumulates it (sum / nx); core_energy_extended
@@ -995,10 +996,11 @@ int adjoint_core(pfdd_gl *h, const void *xs, const void *lam_in, void *lam_out, 
 {
     const Maps m = make_maps(h, h->SM);
     hipStream_t st = h->stream;
+    const Order ord = order_of((size_t)h->SM * h->N * h->esz, (int)h->esz), zord = {ord.keep, false};
     HIPCHK((launch_pass<R, false>(h->nz, lam_in, h->T1, m.p1i, m.p1o, m.n1, h->tw[2], h->done, st, h->mask,
-                                  h->tq[0])));
+                                  h->tq[0], zord)));
     HIPCHK((launch_pass<R, false>(h->ny, h->T1, lam_out, m.p2i, m.p2o, m.n2, h->tw[1], h->done, st, nullptr,
-                                  h->tq[1])));
+                                  h->tq[1], ord)));
     if (h->stored_B)
         HIPCHK((launch_mid<R>(h->nx, h->S, h->M, lam_out, h->B, (long long)h->ny * h->nz, h->N, h->tw[0],
                               h->partial + 4 * h->pstride, h->done, st)));
@@ -1006,7 +1008,7 @@ int adjoint_core(pfdd_gl *h, const void *xs, const void *lam_in, void *lam_out, 
         HIPCHK((launch_mid_otf<R>(h->nx, h->S, h->M, lam_out, h->G, (long long)h->ny * h->nz, h->N, h->tw[0],
                                   h->partial + 4 * h->pstride, h->done, st, h->xpipe, h->ncu, &h->nb3)));
     HIPCHK((launch_pass<R, true>(h->ny, lam_out, h->T1, m.p2o, m.p2i, m.n2, h->tw[1], h->done, st, nullptr,
-                                 h->tq[2])));
+                                 h->tq[2], ord)));
     const long long gstride = h->nb5max;
     HIPCHK(launch_adj_update<R>(h->nz, h->tq[3], h->T1, lam_in, xs, lam_out, h->mask, h->amp, m.p5i, m.p5o,
                                 m.n5, (long long)h->nx * h->ny, P, h->tw[2], h->tape.gpart, gstride, h->done,
@@ -1163,6 +1165,7 @@ int build_B(pfdd_gl *h)
     G.inv2C44 = bp.inv2C44;
     G.inv1mnu = bp.inv1mnu;
     G.invmu = bp.invmu;
+    G.keep = order_of((size_t)h->SM * h->N * h->esz, (int)h->esz).keep;
     G.nx = h->nx;
     G.ny = h->ny;
     G.nz = h->nz;

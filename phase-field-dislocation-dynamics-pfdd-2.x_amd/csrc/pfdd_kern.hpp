@@ -245,8 +245,8 @@ __device__ __forceinline__ V gl_update_cell(const V g, const V x, long long idx,
             R sm = sp, cm = cp;
             for (int m = 1; m <= nm; ++m) {
                 const R c = coef(m - 1);
-                dens += c * sm * sm;
-                dE += c * ((R)m * (R)M_PI) * ((R)2 * sm * cm);
+                dens = ab_c(c * sm, sm, dens);
+                dE = ab_c(c * ((R)m * (R)M_PI), (R)2 * sm * cm, dE);
                 const R sn = ab_cd(sm, cp, cm, sp), cn = ab_cd(cm, cp, -sm, sp);
                 sm = sn;
                 cm = cn;
@@ -266,8 +266,8 @@ __device__ __forceinline__ V gl_update_cell(const V g, const V x, long long idx,
         const double dr = (double)x.x - (double)pv.x, di = (double)x.y - (double)pv.y;
         dn = dr * dr + di * di;
     } else {
-        y.x = x.x - cddt * (g.x * invN - tau + dE);
-        y.y = x.y - cddt * (g.y * invN);
+        y.x = ab_c(-cddt, ab_c(g.x, invN, -tau) + dE, x.x);
+        y.y = ab_c(-cddt, g.y * invN, x.y);
         const double dr = (double)y.x - (double)x.x, di = (double)y.y - (double)x.y;
         dn = dr * dr + di * di;
     }
@@ -293,8 +293,8 @@ __device__ __forceinline__ void gl_update_chunk(const V *g, const V *x, const R 
         dens[c] = (R)0;
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
-            dens[c] += lc[m] * sm * sm;
-            dE += ldp[m] * ((R)2 * sm * cm);
+            dens[c] = ab_c(lc[m] * sm, sm, dens[c]);
+            dE = ab_c(ldp[m], (R)2 * sm * cm, dE);
             if (m + 1 < NM) {
                 const R sn = ab_cd(sm, cp, cm, sp), cn = ab_cd(cm, cp, -sm, sp);
                 sm = sn;
@@ -305,8 +305,8 @@ __device__ __forceinline__ void gl_update_chunk(const V *g, const V *x, const R 
             dens[c] *= A[c];
             dE *= A[c];
         }
-        y[c].x = x[c].x - cddt * (g[c].x * invN - tau + dE);
-        y[c].y = x[c].y - cddt * (g[c].y * invN);
+        y[c].x = ab_c(-cddt, ab_c(g[c].x, invN, -tau) + dE, x[c].x);
+        y[c].y = ab_c(-cddt, g[c].y * invN, x[c].y);
         if constexpr (MA) {
             const bool fz = (frozen >> c) & 1;
             y[c].x = fz ? x[c].x : y[c].x;
@@ -338,6 +338,7 @@ struct GParams {
     double C44x2, C12; // isotropic stiffness: C:Q = 2 C44 Q + C12 tr(Q) I
     double inv_n[3];   // 1/nx, 1/ny, 1/nz (frequencies by multiplication in the x pass)
     int nx, ny, nz;
+    bool keep;         // store the field for the next kernel to find in the last-level cache (Order)
 };
 
 __device__ __forceinline__ double frac_freq(int kk, int n)
@@ -399,11 +400,35 @@ int tile_lines_rt(int n, int tq)
 // Line pass (pfdd_pass.hip): FFT along one axis of nlines lines, input line
 // map mi, output line map mo; zmask (optional) zeroes input elements.  tq =
 // tile shape (0, 1, 2) + 3 * radix plan (0 radix 8 first, 1 radix 16 where it
-// saves a stage).
+// saves a stage).  keep, rev: how the pass
+// uses the last-level cache (Order).
+//
+// Order of a field's passes.  keep: the work fields are stored plainly, for
+// the next kernel to find in the 256 MB last-level cache.  rev: the y passes
+// take their lines from the last to the first: the kernel before them wrote
+// T1 (T2) upwards, so its end is what that cache holds when they start, and the
+// kernel after them finds its beginning there.  A field that fits in the cache
+// is found whole in either order (the FP32 step at 128^3 x 12, 201 MB, is 1.5 %
+// faster forwards); one many times larger is hardly found at all.  Measured,
+// us per iteration, FP64, nontemporal and forwards -> keep and rev (keep
+// alone): 128^3 x 6 (201 MB) 414 -> 364 (362), 128^3 x 12 (403 MB) 803 -> 753
+// (814), 256^3 x 3 (805 MB) 1588 -> 1532 (1614), 256 x 256 x 128 x 12 (1.6 GB)
+// 3146 -> 3184 (3202), 512 x 512 x 256 x 3 (3.2 GB) 6171 -> 6456.  FP32 fields
+// are always kept (st_work); forwards -> rev: 256^3 x 3 (403 MB) 834 -> 792,
+// 256 x 256 x 128 x 12 (805 MB) 1620 -> 1569, 256^3 x 12 (1.6 GB) 3283 -> 3217.
+constexpr size_t LLC_BYTES = (size_t)256 << 20, KEEP_BYTES = 4 * LLC_BYTES;
+struct Order {
+    bool keep, rev;
+};
+inline Order order_of(size_t field_bytes, int elem_bytes)
+{
+    const bool keep = elem_bytes < 16 || field_bytes <= KEEP_BYTES;
+    return Order{keep, keep && field_bytes > LLC_BYTES};
+}
 template <typename R, bool INV>
 hipError_t launch_pass(int n, const void *in, void *out, LineMap mi, LineMap mo, long long nlines,
                        const void *tw, const int *done, hipStream_t st, const uint8_t *zmask = nullptr,
-                       int tq = 1);
+                       int tq = 1, Order order = Order{true, false});
 
 // Last inverse pass + GL update, and its reverse mode (pfdd_update.hip).
 // plan: radix plan of the z transforms; fw: also the next iteration's forward
@@ -418,8 +443,8 @@ template <typename R> int update_lines(int n, int tq, int model);
 template <typename R>
 hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
                          const long long *prev, const void *amp, LineMap mi, LineMap mo, long long nlines,
-                         long long lps, const StepParams &P, const void *tw, const UpdNone *none, double *partial,
-                         long long pstride, const int *done, hipStream_t st);
+                         long long lps, const StepParams &P, const void *tw, const UpdNone *none, bool keep,
+                         double *partial, long long pstride, const int *done, hipStream_t st);
 template <typename R>
 hipError_t launch_adj_update(int n, int tq, const void *T1, const void *lam, const void *xs, void *lam_out,
                              const uint8_t *mask, const void *amp, LineMap mi, LineMap mo, long long nlines,

@@ -128,7 +128,7 @@ __global__ void __launch_bounds__(NTHR)
     for (int e = tid; e < TOT; e += NTHR) {
         const int l = e / N, p = e % N;
         const int a = l / NP, q = l % NP;
-        if (c0 + q < ncol) T2[(long long)a * ntot + (c0 + q) * N + p] = lds.ld(p * LDP + l);
+        if (c0 + q < ncol) st_work(&T2[(long long)a * ntot + (c0 + q) * N + p], lds.ld(p * LDP + l), false);
     }
     double v[1] = {el};
     block_sum_comp<1, NTHR>(v, red, tid);
@@ -396,7 +396,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(otf_w
     for (int e = tid; e < TOT; e += NTHR) {
         const int l = e / N, p = e % N;
         const int a = l / NP, q = l % NP;
-        if (c0 + q < ncol) st_stream(&T2[(long long)a * ntot + (c0 + q) * N + p], lds.ld(XA::at(p, l)));
+        if (c0 + q < ncol) st_work(&T2[(long long)a * ntot + (c0 + q) * N + p], lds.ld(XA::at(p, l)), G.keep);
     }
     block_sum_comp<1, NTHR>(v, red, tid);
     if (tid == 0) part_el[blockIdx.x] = v[0];
@@ -712,7 +712,7 @@ __global__ void __launch_bounds__((XTile<N, S>::W)) __attribute__((amdgpu_waves_
     __asm__ volatile("" : "+v"(t2)); // addresses formed again, as in k_update_r
     reg_fft<N, 1, 1, NL, VPT, true, true, true, false, L>(v, lds, tws, t2);
 #pragma unroll
-    for (int m = 0; m < VPT; ++m) st_stream(own + D * m, v[m]);
+    for (int m = 0; m < VPT; ++m) st_work(own + D * m, v[m], G.keep);
     double sum[1] = {el};
     block_sum_comp<1, W>(sum, red, t);
     if (t == 0) part_el[blockIdx.x] = sum[0];

@@ -12,7 +12,7 @@ template <typename R, int N, bool INV, int TQ, int PL>
 __global__ void __launch_bounds__(NTHR)
     k_fft_pass(const typename cvec<R>::type *__restrict__ in, typename cvec<R>::type *__restrict__ out,
                LineMap mi, LineMap mo, long long nlines, const typename cvec<R>::type *__restrict__ tw,
-               const int *__restrict__ done, const uint8_t *__restrict__ zmask)
+               const int *__restrict__ done, const uint8_t *__restrict__ zmask, Order order)
 {
     typedef typename cvec<R>::type V;
     if (*done) return;
@@ -20,7 +20,7 @@ __global__ void __launch_bounds__(NTHR)
     PFDD_TILE(V, lds, N * LDP);
     __shared__ long long bin[NL], bout[NL];
     const int tid = threadIdx.x;
-    const long long L0 = (long long)blockIdx.x * NL;
+    const long long L0 = (long long)(order.rev ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * NL;
     for (int l = tid; l < NL; l += NTHR) {
         const long long L = L0 + l;
         const bool ok = L < nlines;
@@ -41,7 +41,7 @@ __global__ void __launch_bounds__(NTHR)
     }
     if constexpr (PL == 1) fft_stages_x<N, 1, NL, NTHR, INV>(lds, tw, tid);
     else fft_stages<N, 1, NL, NTHR, INV>(lds, tw, tid);
-    tile_store<N, NL, NTHR>(out, lds, bout, mo.SP, tid);
+    tile_store<N, NL, NTHR>(out, lds, bout, mo.SP, tid, order.keep);
 }
 
 
@@ -80,7 +80,7 @@ template <typename R, int N, int PL, bool INV, bool CI, bool CO>
 __global__ void __launch_bounds__((RegTile<R, N>::W))
     k_pass_r(const typename cvec<R>::type *__restrict__ in, typename cvec<R>::type *__restrict__ out, LineMap mi,
              LineMap mo, const typename cvec<R>::type *__restrict__ tw, const int *__restrict__ done,
-             const uint8_t *__restrict__ zmask)
+             const uint8_t *__restrict__ zmask, Order order)
 {
     typedef typename cvec<R>::type V;
     typedef RegTile<R, N> G;
@@ -93,7 +93,7 @@ __global__ void __launch_bounds__((RegTile<R, N>::W))
     __shared__ unsigned li[CI ? NL : 1], lo[CO ? NL : 1];
     RegLds<V> lds{(decltype(RegLds<V>::p))mem};
     const int t = threadIdx.x;
-    const unsigned L0 = blockIdx.x * NL;
+    const unsigned L0 = (order.rev ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * NL;
     const RegBase bi(mi, L0), bo(mo, L0);
     constexpr int PW = W < N ? W : N; // positions that W threads cover in linear ownership
     if constexpr (CI || CO) {
@@ -125,20 +125,20 @@ __global__ void __launch_bounds__((RegTile<R, N>::W))
 #pragma unroll
         for (int m = 0; m < VPT; ++m) {
             const unsigned e = lo[Lin::line(t, m)] + Lin::pos_s(m) + t % PW;
-            st_stream((V *)((char *)(out + bo.ref) + e * (unsigned)sizeof(V)), v[m]);
+            st_work((V *)((char *)(out + bo.ref) + e * (unsigned)sizeof(V)), v[m], order.keep);
         }
     } else {
         const unsigned e = bo.line(t % NL) + (t / NL) * (unsigned)mo.SP;
 #pragma unroll
         for (int m = 0; m < VPT; ++m)
-            st_stream((V *)((char *)(out + bo.ref + D * m * mo.SP) + e * (unsigned)sizeof(V)), v[m]);
+            st_work((V *)((char *)(out + bo.ref + D * m * mo.SP) + e * (unsigned)sizeof(V)), v[m], order.keep);
     }
 }
 
 template <typename R, bool INV>
 hipError_t launch_pass(int n, const void *in, void *out, LineMap mi, LineMap mo, long long nlines,
                        const void *tw, const int *done, hipStream_t st, const uint8_t *zmask,
-                       int tq)
+                       int tq, Order order)
 {
     typedef typename cvec<R>::type V;
     // tq = shape + 3 * plan; plan 1 falls back to plan 0 where they coincide
@@ -146,7 +146,7 @@ hipError_t launch_pass(int n, const void *in, void *out, LineMap mi, LineMap mo,
 #define PFDD_PASS_R(PL_, PFI_, PFO_)                                                                \
     PFDD_LAUNCH((k_pass_r<R, N, (PL_ && radix16_plan_differs<N>()), INV, PFI_, PFO_>),              \
                 dim3((unsigned)(nlines / RegTile<R, N>::NL)), dim3(RegTile<R, N>::W), st,           \
-                (const V *)in, (V *)out, mi, mo, (const V *)tw, done, zmask)
+                (const V *)in, (V *)out, mi, mo, (const V *)tw, done, zmask, order)
 #define PFDD_CASE(n_)                                                                               \
     if (n == n_) {                                                                                  \
         constexpr int N = n_;                                                                       \
@@ -166,10 +166,10 @@ hipError_t launch_pass(int n, const void *in, void *out, LineMap mi, LineMap mo,
             if (plan == 1 && radix16_plan_differs<n_>())                                            \
                 PFDD_LAUNCH((k_fft_pass<R, n_, INV, TQ, radix16_plan_differs<n_>() ? 1 : 0>),      \
                             dim3(nb), dim3(NTHR), st, (const V *)in, (V *)out, mi, mo, nlines,      \
-                            (const V *)tw, done, zmask);                                       \
+                            (const V *)tw, done, zmask, order);                                       \
             else                                                                                    \
                 PFDD_LAUNCH((k_fft_pass<R, n_, INV, TQ, 0>), dim3(nb), dim3(NTHR), st,              \
-                            (const V *)in, (V *)out, mi, mo, nlines, (const V *)tw, done, zmask); \
+                            (const V *)in, (V *)out, mi, mo, nlines, (const V *)tw, done, zmask, order); \
         })                                                                                          \
         return hipGetLastError();                                                                   \
         }                                                                                           \
@@ -181,12 +181,12 @@ hipError_t launch_pass(int n, const void *in, void *out, LineMap mi, LineMap mo,
 }
 
 template hipError_t launch_pass<double, false>(int, const void *, void *, LineMap, LineMap, long long, const void *,
-                                               const int *, hipStream_t, const uint8_t *, int);
+                                               const int *, hipStream_t, const uint8_t *, int, Order);
 template hipError_t launch_pass<double, true>(int, const void *, void *, LineMap, LineMap, long long, const void *,
-                                              const int *, hipStream_t, const uint8_t *, int);
+                                              const int *, hipStream_t, const uint8_t *, int, Order);
 template hipError_t launch_pass<float, false>(int, const void *, void *, LineMap, LineMap, long long, const void *,
-                                              const int *, hipStream_t, const uint8_t *, int);
+                                              const int *, hipStream_t, const uint8_t *, int, Order);
 template hipError_t launch_pass<float, true>(int, const void *, void *, LineMap, LineMap, long long, const void *,
-                                             const int *, hipStream_t, const uint8_t *, int);
+                                             const int *, hipStream_t, const uint8_t *, int, Order);
 
 } // namespace pfdd

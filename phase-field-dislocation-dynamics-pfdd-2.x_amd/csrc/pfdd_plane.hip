@@ -111,7 +111,7 @@ __global__ void __launch_bounds__((plane_threads<R, NY, NZ>()))
 #pragma unroll
         for (int t = 0; t < PER; ++t) {
             const int e = tid + t * NT;
-            if (TOT % NT == 0 || e < TOT) st_stream(&o[e], lds.ld((e % NZ) * LDY + e / NZ));
+            if (TOT % NT == 0 || e < TOT) o[e] = lds.ld((e % NZ) * LDY + e / NZ);
         }
         __syncthreads();
     }
@@ -203,7 +203,7 @@ __global__ void __launch_bounds__((plane_threads<R, NY, NZ>()))
 #pragma unroll
             for (int t = 0; t < PER; ++t) {
                 const int e = t2 + t * NT;
-                if (TOT % NT == 0 || e < TOT) st_stream(&T[base + e], lds.ld((e % NZ) * LDY + e / NZ));
+                if (TOT % NT == 0 || e < TOT) T[base + e] = lds.ld((e % NZ) * LDY + e / NZ);
             }
         }
         __syncthreads();

@@ -33,7 +33,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(updat
              typename cvec<R>::type *__restrict__ xn, const uint8_t *__restrict__ mask,
              const long long *__restrict__ prev, const R *__restrict__ amp, LineMap mi, LineMap mo,
              long long nlines, long long lines_per_sys, StepParams P,
-             const typename cvec<R>::type *__restrict__ tw, double *__restrict__ partial,
+             const typename cvec<R>::type *__restrict__ tw, bool keep, double *__restrict__ partial,
              long long pstride, const int *__restrict__ done)
 {
     typedef typename cvec<R>::type V;
@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(updat
         __asm__ volatile("" : "+v"(t2));
         if constexpr (FW == 2) fft_stages_x<N, 1, NL, NTHR, false>(lds, tw, t2);
         else fft_stages<N, 1, NL, NTHR, false>(lds, tw, t2);
-        tile_store<N, NL, NTHR>(T1, lds, bin, mi.SP, t2);
+        tile_store<N, NL, NTHR>(T1, lds, bin, mi.SP, t2, keep);
     }
 }
 
@@ -152,8 +152,8 @@ __global__ void __launch_bounds__((RegTile<R, N>::W)) __attribute__((amdgpu_wave
     k_update_r(typename cvec<R>::type *T1, const typename cvec<R>::type *__restrict__ xo,
                typename cvec<R>::type *__restrict__ xn, const uint8_t *__restrict__ mask,
                const long long *__restrict__ prev, const R *__restrict__ amp, unsigned mstep, unsigned astep,
-               unsigned ny, unsigned lines_per_sys, StepParams P, const typename cvec<R>::type *__restrict__ tw, double *__restrict__ partial,
-               long long pstride, const int *__restrict__ done)
+               unsigned ny, unsigned lines_per_sys, StepParams P, const typename cvec<R>::type *__restrict__ tw,
+               bool keep, double *__restrict__ partial, long long pstride, const int *__restrict__ done)
 {
     typedef typename cvec<R>::type V;
     typedef RegTile<R, N> G;
@@ -259,7 +259,7 @@ __global__ void __launch_bounds__((RegTile<R, N>::W)) __attribute__((amdgpu_wave
         __asm__ volatile("" : "+v"(t2));
         reg_fft<N, 1, PL, NL, VPT, false, true, false, false>(v, lds, tws, t2);
 #pragma unroll
-        for (int m = 0; m < VPT; ++m) st_stream((V *)((char *)(T1b + (size_t)(D * m) * ny) + o1), v[m]);
+        for (int m = 0; m < VPT; ++m) st_work((V *)((char *)(T1b + (size_t)(D * m) * ny) + o1), v[m], keep);
     }
     double sum[4] = {s_norm, s_ave, s_core, s_str};
     block_sum_comp<4, W>(sum, red, t);
@@ -415,8 +415,8 @@ template <typename R> int update_lines(int n, int tq, int model)
 template <typename R>
 hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
                          const long long *prev, const void *amp, LineMap mi, LineMap mo, long long nlines,
-                         long long lps, const StepParams &P, const void *tw, const UpdNone *none, double *partial,
-                         long long pstride, const int *done, hipStream_t st)
+                         long long lps, const StepParams &P, const void *tw, const UpdNone *none, bool keep,
+                         double *partial, long long pstride, const int *done, hipStream_t st)
 {
     typedef typename cvec<R>::type V;
     const uint8_t *no_mask = &none->zero;
@@ -433,7 +433,7 @@ hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void 
                 dim3((unsigned)(nlines / RegTile<R, N>::NL)), dim3(RegTile<R, N>::W), st, (V *)T1,   \
                 (const V *)xo, (V *)xn, mask ? mask : no_mask, prev,                                 \
                 amp ? (const R *)amp : no_amp, mask ? 1u : 0u, amp ? 1u : 0u, (unsigned)mi.D,        \
-                (unsigned)lps, P, (const V *)tw, partial, pstride, done)
+                (unsigned)lps, P, (const V *)tw, keep, partial, pstride, done)
 #define PFDD_UPR(PL_, FW_)                                                                           \
     do {                                                                                             \
         if (mask || amp) {                                                                           \
@@ -450,7 +450,7 @@ hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void 
     PFDD_LAUNCH((k_update<R, N, TQ_, GEN_, FW_>),                                                    \
                 dim3((unsigned)((nlines + tile_lines_u<R, N, TQ_>() - 1) / tile_lines_u<R, N, TQ_>())), \
                 dim3(NTHR), st, (V *)T1, (const V *)xo, (V *)xn, mask, prev, (const R *)amp, mi, mo, \
-                nlines, lps, P, (const V *)tw, partial, pstride, done)
+                nlines, lps, P, (const V *)tw, keep, partial, pstride, done)
 #define PFDD_UPD_FW(TQ_, GEN_)                                                                       \
     if (!fw) PFDD_UPD(TQ_, GEN_, 0);                                                                 \
     else if (plan == 1 && radix16_plan_differs<N>()) PFDD_UPD(TQ_, GEN_, (radix16_plan_differs<N>() ? 2 : 1)); \
@@ -513,7 +513,7 @@ hipError_t launch_adj_update(int n, int tq, const void *T1, const void *lam, con
     template int update_lines<R>(int, int, int);                                                                      \
     template hipError_t launch_update<R>(int, int, int, bool, void *, const void *, void *, const uint8_t *,           \
                                          const long long *, const void *, LineMap, LineMap, long long, long long, \
-                                         const StepParams &, const void *, const UpdNone *, double *, long long,   \
+                                         const StepParams &, const void *, const UpdNone *, bool, double *, long long, \
                                          const int *, hipStream_t);                                               \
     template hipError_t launch_adj_update<R>(int, int, const void *, const void *, const void *, void *,         \
                                              const uint8_t *, const void *, LineMap, LineMap, long long,          \
