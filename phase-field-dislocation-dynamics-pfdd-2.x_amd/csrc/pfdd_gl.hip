@@ -200,70 +200,99 @@ __global__ void __launch_bounds__(NTHR)
     }
 }
 
+// Scalars of a run's last iteration, in pinned host memory.
+struct RunStat {
+    double res[NRES];
+    int done, steps;
+};
+// The sums of an iteration: partials [NSLOT][pstride], nb5 of the update
+// (slots 0-3) and nb3 of the x pass (slot 4).
+struct Sums {
+    const double *partial;
+    long long pstride;
+    int nb5, nb3;
+    double invN, inv_nx, tol;
+    double *stage2;   // [NSLOT][NB2]
+    unsigned *ticket; // zero between launches
+    RunStat *stat;
+    int *done, *steps;
+    bool last;        // the run ends here
+};
+
 // Deterministic reduction of the block partials in two levels: every block
 // sums a fixed chunk (Kahan within a thread, fixed-shape tree across the
 // block) into stage2; the last block to finish (atomic ticket) sums stage2
 // with all its threads (one value per thread and slot, the compensated block
-// tree), writes the iteration's scalars, counts the iteration and raises
-// `done` on convergence or a non-finite result.
+// tree), forms the iteration's scalars, counts the iteration and raises `done`
+// on convergence or a non-finite result.  Where a run ends, it writes them to
+// the host's memory itself: three copies of a few bytes and the launch that
+// cleared the counters cost 60 of the 150 us of a one-iteration run at 32^3.
+// stage2 goes through relaxed agent-scope atomics, which reach the point where
+// all XCDs agree: only the wait for the stores stands before the ticket, no
+// fence with its write-back of the L2.  Having the update's last blocks do all
+// this (no launch of its own, 7 us) was slower from 64^3 x 3 up (53.0 -> 54.9
+// us per iteration, 749 -> 758 at 128^3 x 12): the wait for its stores holds a
+// wave of every block.
 constexpr int NB2 = 32;
 static_assert(NB2 <= NTHR, "the last block reads stage2 one value per thread");
 
-__global__ void __launch_bounds__(NTHR)
-    k_reduce(const double *__restrict__ partial, long long pstride, int nb5, int nb3, double invN,
-             double inv_nx, double tol, double *__restrict__ stage2, unsigned *__restrict__ ticket,
-             double *__restrict__ res, int *__restrict__ done, int *__restrict__ steps)
+__global__ void __launch_bounds__(NTHR) k_sums(Sums F)
 {
-    if (*done) return;
+    if (*F.done) return;
     __shared__ double red[NSLOT * (NTHR / 64)];
     __shared__ int last;
     const int tid = threadIdx.x;
-    double v[NSLOT];
+    double w[NSLOT];
 #pragma unroll
-    for (int s = 0; s < NSLOT; ++s) {
-        const int nb = s == 4 ? nb3 : nb5;
-        const int chunk = (nb + NB2 - 1) / NB2;
-        const int lo = blockIdx.x * chunk, hi = min(nb, lo + chunk);
+    for (int q = 0; q < NSLOT; ++q) {
+        const int n = q == 4 ? F.nb3 : F.nb5, chunk = (n + NB2 - 1) / NB2;
+        const int lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
         double sum = 0.0, c = 0.0;
         for (int b = lo + tid; b < hi; b += NTHR) {
-            const double y = partial[s * pstride + b] - c;
+            const double y = F.partial[q * F.pstride + b] - c;
             const double t = sum + y;
             c = (t - sum) - y;
             sum = t;
         }
-        v[s] = sum;
+        w[q] = sum;
     }
-    block_sum<NSLOT, NTHR>(v, red, tid);
+    block_sum<NSLOT, NTHR>(w, red, tid);
     if (tid == 0) {
 #pragma unroll
-        for (int s = 0; s < NSLOT; ++s) stage2[s * NB2 + blockIdx.x] = v[s];
-        __threadfence();
-        last = atomicAdd(ticket, 1u) == NB2 - 1;
+        for (int q = 0; q < NSLOT; ++q)
+            __hip_atomic_store((long long *)&F.stage2[q * NB2 + blockIdx.x], __double_as_longlong(w[q]),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        last = __hip_atomic_fetch_add(F.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == NB2 - 1;
     }
     __syncthreads();
     if (!last) return;
-    __threadfence();
-    // one dependent round trip instead of NB2 * NSLOT serial loads in one
-    // thread (the first level's stage2 writes are visible: ticket + fences)
-    double w[NSLOT];
 #pragma unroll
-    for (int s = 0; s < NSLOT; ++s) w[s] = tid < NB2 ? __builtin_nontemporal_load(&stage2[s * NB2 + tid]) : 0.0;
+    for (int q = 0; q < NSLOT; ++q)
+        w[q] = tid < NB2 ? __longlong_as_double(__hip_atomic_load((const long long *)&F.stage2[q * NB2 + tid],
+                                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                         : 0.0;
     block_sum_comp<NSLOT, NTHR>(w, red, tid);
     if (tid != 0) return;
-    *ticket = 0u;
+    *F.ticket = 0u;
     const double xinorm = sqrt(w[0]);
-    const double e_el = 0.5 * w[4] * invN;
-    res[0] = xinorm;
-    res[1] = w[1];
-    res[2] = e_el;
-    res[3] = w[2];
-    res[4] = w[3];
-    res[5] = e_el + w[2] - w[3];
-    res[6] = w[2] * inv_nx;
+    const double e_el = 0.5 * w[4] * F.invN;
     const bool finite = isfinite(xinorm) && isfinite(w[1]) && isfinite(e_el) && isfinite(w[2]);
-    res[7] = finite ? 0.0 : 1.0;
-    *steps += 1;
-    if (!finite || (tol > 0 && xinorm < tol)) *done = finite ? 1 : 2;
+    const int done = !finite ? 2 : (F.tol > 0 && xinorm < F.tol) ? 1 : 0;
+    const int steps = (int)((unsigned)*F.steps + 1u);
+    *F.steps = steps;
+    if (done) *F.done = done;
+    if (!F.last && !done) return;
+    F.stat->res[0] = xinorm;
+    F.stat->res[1] = w[1];
+    F.stat->res[2] = e_el;
+    F.stat->res[3] = w[2];
+    F.stat->res[4] = w[3];
+    F.stat->res[5] = e_el + w[2] - w[3];
+    F.stat->res[6] = w[2] * F.inv_nx;
+    F.stat->res[7] = finite ? 0.0 : 1.0;
+    F.stat->done = done;
+    F.stat->steps = steps;
 }
 
 // Streaming rate probes for pfdd_gl_stream_rates: one 16-byte element per
@@ -517,9 +546,14 @@ struct pfdd_gl {
     int ncu = 0;                       // compute units of the device
     double *stage2 = nullptr; // NSLOT * NB2
     unsigned *ticket = nullptr;
+    RunStat *stat = nullptr;  // pinned host memory
+    // the host knows that *done == 0 and *steps == steps0: set by
+    // collect_steps, and a run that starts so needs no k_reset
+    bool fresh = false;
+    int steps0 = 0;
+    bool captured = false;    // a caller captured a run, and may replay it at any time
     bool stored_B = false;    // stream packed B(k) from HBM instead of evaluating it on the fly
     GParams G{};
-    double *res = nullptr; // NRES doubles
     int *done = nullptr;
     int *steps = nullptr;
     StepParams P{};
@@ -616,6 +650,15 @@ Maps make_maps_dims(long long nx, long long ny, long long nz, long long S)
 
 Maps make_maps(const pfdd_gl *h, long long S) { return make_maps_dims(h->nx, h->ny, h->nz, S); }
 
+// *done = *steps = 0; iterations of a run that the host does not collect may
+// follow, so what they become is not known.
+void reset_run(pfdd_gl *h, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, st, h->done, h->steps);
+    h->steps0 = 0;
+    h->fresh = false;
+}
+
 // One GL iteration from xo into T2 (T2 doubles as the temporary of passes
 // 2-4), with the stress and core parameters P, as part of a run of
 // iterations that each start from the previous one's result.  first: xo
@@ -645,6 +688,9 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
         HIPCHK(hipGetLastError());
     }
     const Order ord = order_of((size_t)h->SM * h->N * h->esz, (int)h->esz), zord = {ord.keep, false};
+    // E_core as the reference accumulates it (sum / nx); core_energy_extended
+    // and core_energy_pyrII do not accumulate it (fft_fftw_slab.cpp:1320,1483)
+    const bool no_eref = P.model == PFDD_CORE_EXTENDED || P.model == PFDD_CORE_PYRII;
     if (h->plane) {
         // plane iteration: 2-D forward pass xo -> T1, x pass on T1 in its
         // plane layout, 2-D inverse pass + update T1 + xo -> T2.  The slots
@@ -672,8 +718,7 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
         if ((rc = empty(3))) return rc;
         arm(4);
         HIPCHK(launch_plane_upd<R>(h->ny, h->nz, !last, h->T1, xo, T2, h->mask, h->prev, h->cof ? h->cof : h->amp,
-                                   nplanes, h->nx, last ? h->nbC : h->nbCF, P, h->tw[1], h->tw[2], h->partial,
-                                   h->pstride, h->done, st));
+                                   nplanes, h->nx, last ? h->nbC : h->nbCF, P, h->tw[1], h->tw[2], h->partial, h->pstride, h->done, st));
     } else {
     if (first) {
         arm(0);
@@ -686,7 +731,7 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
     arm(2);
     if (h->stored_B)
         HIPCHK((launch_mid<R>(h->nx, h->S, h->M, T2, h->B, (long long)h->ny * h->nz, h->N, h->tw[0],
-                              h->partial + 4 * h->pstride, h->done, st)));
+                              h->partial + 4 * h->pstride, h->done, st, &h->nb3)));
     else
         HIPCHK((launch_mid_otf<R>(h->nx, h->S, h->M, T2, h->G, (long long)h->ny * h->nz, h->N, h->tw[0],
                                   h->partial + 4 * h->pstride, h->done, st, h->xpipe, h->ncu, &h->nb3)));
@@ -701,11 +746,9 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
                             h->none, ord.keep, h->partial, h->pstride, h->done, st));
     }
     arm(5);
-    // E_core as the reference accumulates it (sum / nx); core_energy_extended
-    // and core_energy_pyrII do not accumulate it (fft_fftw_slab.cpp:1320,1483)
-    const bool no_eref = P.model == PFDD_CORE_EXTENDED || P.model == PFDD_CORE_PYRII;
-    PFDD_LAUNCH(k_reduce, dim3(NB2), dim3(NTHR), st, h->partial, h->pstride, h->nb5, h->nb3, 1.0 / (double)h->N,
-                no_eref ? 0.0 : 1.0 / (double)h->nx, tol, h->stage2, h->ticket, h->res, h->done, h->steps);
+    PFDD_LAUNCH(k_sums, dim3(NB2), dim3(NTHR), st,
+                Sums{h->partial, h->pstride, h->nb5, h->nb3, 1.0 / (double)h->N, no_eref ? 0.0 : 1.0 / (double)h->nx,
+                     tol, h->stage2, h->ticket, h->stat, h->done, h->steps, last});
     HIPCHK(hipGetLastError());
     return PFDD_OK;
 }
@@ -735,7 +778,6 @@ void set_tiles(pfdd_gl *h, const int tq[5])
     h->xpipe = (h->stored_B || tq[4] != 1) ? 0 : 1;
     if (h->plane) {
         h->nb5 = (int)((long long)h->SM * h->nx); // one partial per y-z plane
-        h->nb3 = h->nb3pl;
     } else {
         const long long n5 = (long long)h->SM * h->nx * h->ny;
         const int nl = h->prec == PFDD_FP64 ? update_lines<double>(h->nz, h->tq[3], m)
@@ -827,7 +869,7 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
     auto restore = [&]() -> int {
         HIPCHK(hipMemcpyAsync(h->xi[cur0], save, fb, hipMemcpyDeviceToDevice, h->stream));
         if (stepped0) HIPCHK(hipMemcpyAsync(h->xi[1 - cur0], save + fb, fb, hipMemcpyDeviceToDevice, h->stream));
-        hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
+        reset_run(h, h->stream);
         HIPCHK(hipGetLastError());
         h->cur = cur0;
         h->stepped = stepped0;
@@ -855,7 +897,7 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
     for (int c = 0; c < 8; ++c)
         for (int p = 0; p < 5; ++p) tmin[c][p] = 1e300;
     {
-        hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
+        reset_run(h, h->stream);
         double warm[5];
         rc = time_passes<R>(h, 20, warm);
     }
@@ -865,7 +907,7 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
             const int var = c < nshape ? 0 : c == c_pipe ? 1 : 2;
             const int all[5] = {ln, ln, ln, up, var};
             set_tiles(h, all);
-            hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
+            reset_run(h, h->stream);
             double warm[5], t[5];
             if ((rc = time_passes<R>(h, 1, warm)) || (rc = time_passes<R>(h, nsteps, t))) break;
             for (int p = 0; p < 5; ++p) tmin[c][p] = t[p] < tmin[c][p] ? t[p] : tmin[c][p];
@@ -938,7 +980,7 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
                 for (int round = 0; round < 2 && !rc; ++round)
                     for (int c = 0; c < nc && !rc; ++c) {
                         set_tiles(h, cand[c]);
-                        hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
+                        reset_run(h, h->stream);
                         double warm[5], t[5];
                         if ((rc = time_passes<R>(h, 1, warm)) || (rc = time_passes<R>(h, nsteps, t))) break;
                         const double s = t[1] + t[2] + t[3] + t[4];
@@ -1003,7 +1045,7 @@ int adjoint_core(pfdd_gl *h, const void *xs, const void *lam_in, void *lam_out, 
                                   h->tq[1], ord)));
     if (h->stored_B)
         HIPCHK((launch_mid<R>(h->nx, h->S, h->M, lam_out, h->B, (long long)h->ny * h->nz, h->N, h->tw[0],
-                              h->partial + 4 * h->pstride, h->done, st)));
+                              h->partial + 4 * h->pstride, h->done, st, &h->nb3)));
     else
         HIPCHK((launch_mid_otf<R>(h->nx, h->S, h->M, lam_out, h->G, (long long)h->ny * h->nz, h->N, h->tw[0],
                                   h->partial + 4 * h->pstride, h->done, st, h->xpipe, h->ncu, &h->nb3)));
@@ -1050,7 +1092,7 @@ void destroy_all(pfdd_gl *h)
     if (h->stream) hipStreamSynchronize(h->stream);
     self_graph_release(h);
     void *ptrs[] = {h->cof, h->taud, h->xi[0], h->xi[1], h->T1, h->B, h->tw[0], h->tw[1], h->tw[2], h->mask, h->prev,
-                    h->amp, h->none, h->partial, h->res, h->done, h->steps, h->stage2, h->ticket, h->dw[0], h->dw[1],
+                    h->amp, h->none, h->partial, h->done, h->steps, h->stage2, h->ticket, h->dw[0], h->dw[1],
                     h->deps, h->dsig, h->tape.lam[0], h->tape.lam[1], h->tape.gpart, h->tape.gacc};
     for (void *p : ptrs)
         if (p) hipFree(p);
@@ -1058,6 +1100,7 @@ void destroy_all(pfdd_gl *h)
         if (p) hipFree(p);
     for (void *p : h->tape.seg)
         if (p) hipFree(p);
+    if (h->stat) (void)hipHostFree(h->stat);
     if (h->own_stream && h->stream) hipStreamDestroy(h->stream);
     delete h;
 }
@@ -1266,7 +1309,7 @@ int diag_fields(pfdd_gl *h, const double *sigma_rot, const double *avepst, const
     // strain() reads the k-space field of the pre-update xi (quirk Q2)
     const void *pre = h->stepped ? h->xi[1 - h->cur] : h->xi[h->cur];
     hipStream_t st = h->stream;
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, st, h->done, h->steps);
+    reset_run(h, st);
     HIPCHK(hipGetLastError());
     const Maps ms = make_maps(h, S), m6 = make_maps(h, 6);
     const long long ncol = (long long)h->ny * h->nz;
@@ -1299,14 +1342,15 @@ int diag_fields(pfdd_gl *h, const double *sigma_rot, const double *avepst, const
     return PFDD_OK;
 }
 
-int collect_steps(pfdd_gl *h, int cur0, pfdd_gl_reduce *out)
+int collect_steps(pfdd_gl *h, int cur0, int nsteps, pfdd_gl_reduce *out)
 {
-    double res[NRES];
-    int done = 0, steps = 0;
-    HIPCHK(hipMemcpyAsync(res, h->res, sizeof(res), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipMemcpyAsync(&done, h->done, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipMemcpyAsync(&steps, h->steps, sizeof(int), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
+    const double *res = h->stat->res;
+    // the last iteration that ran left its scalars in stat
+    const int done = nsteps > 0 ? h->stat->done : 0;
+    const int steps = nsteps > 0 ? (int)((unsigned)h->stat->steps - (unsigned)h->steps0) : 0;
+    if (nsteps > 0) h->steps0 = h->stat->steps;
+    h->fresh = done == 0 && !h->captured;
     // the field moved steps times from buffer cur0
     h->cur = (steps % 2) ? 1 - cur0 : cur0;
     if (done == 2)
@@ -1358,7 +1402,7 @@ int tape_backward_any(pfdd_gl *h, const void *dxi_T, bool dev_in, void *dxi_0, b
         return rc;
     }
     HIPCHK(hipMemsetAsync(T.gacc, 0, sizeof(double) * NG * MAXS, h->stream));
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
+    reset_run(h, h->stream);
     HIPCHK(hipGetLastError());
     int cur = 0;
     const int nseg = (T.nsteps + T.every - 1) / T.every;
@@ -1615,9 +1659,7 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
 
     // per-block partials
     const long long n5 = (long long)h->SM * h->nx * h->ny;
-    const int nl5 = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, 1) : tile_lines_rt<float>(h->nz, 1);
     const int nl5min = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, 0) : tile_lines_rt<float>(h->nz, 0);
-    h->nb5 = (int)((n5 + nl5 - 1) / nl5);
     h->nb5max = (int)((n5 + nl5min - 1) / nl5min);
     {
         // the register update's tiles are smaller on short lines
@@ -1666,15 +1708,17 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
             return bail(fail(PFDD_ERR_HIP, "constant upload failed"));
     }
     if ((rc = alloc((void **)&h->partial, sizeof(double) * NSLOT * h->pstride))) return bail(rc);
-    if ((rc = alloc((void **)&h->res, sizeof(double) * NRES))) return bail(rc);
     if ((rc = alloc((void **)&h->stage2, sizeof(double) * NSLOT * NB2)) ||
         (rc = alloc((void **)&h->ticket, sizeof(unsigned))))
         return bail(rc);
+    e = hipHostMalloc((void **)&h->stat, sizeof(RunStat), hipHostMallocDefault);
+    if (e != hipSuccess) return bail(fail(PFDD_ERR_HIP, "hipHostMalloc: %s", hipGetErrorString(e)));
+    *h->stat = RunStat{};
     e = hipMemsetAsync(h->ticket, 0, sizeof(unsigned), h->stream);
     if (e != hipSuccess) return bail(fail(PFDD_ERR_HIP, "hipMemset: %s", hipGetErrorString(e)));
     if ((rc = alloc((void **)&h->done, sizeof(int))) || (rc = alloc((void **)&h->steps, sizeof(int))))
         return bail(rc);
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
+    reset_run(h, h->stream);
 
     // obstacle mask + quirk Q3 predecessor table (restarting with every member)
     if (d->xo) {
@@ -1754,7 +1798,7 @@ int pfdd_gl_theta(pfdd_gl *h, double *theta)
     const size_t n = (size_t)h->SM * h->N;
     void *buf = nullptr;
     HIPCHK(hipMalloc(&buf, n * sizeof(double)));
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
+    reset_run(h, h->stream);
     if (h->prec == PFDD_FP64)
         hipLaunchKernelGGL((k_theta_cof<double, true>), dim3((unsigned)((h->N + NTHR - 1) / NTHR), h->SM), dim3(NTHR),
                            0, h->stream, (const double2 *)pre, (double *)buf, h->TP, h->N, h->done);
@@ -1892,14 +1936,18 @@ int pfdd_gl_step(pfdd_gl *h, int nsteps, double tol, pfdd_gl_reduce *out)
     int rc;
     if ((rc = check_handle(h)) || (rc = set_device(h))) return rc;
     if (nsteps < 0) return fail(PFDD_ERR_ARG, "nsteps < 0");
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
-    HIPCHK(hipGetLastError());
     const int cur0 = h->cur;
     int eager = nsteps;
     // long runs replay a graph of SG_ITERS iterations (one launch instead of
     // 6 SG_ITERS), unless the caller is capturing this stream itself
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIPCHK(hipStreamIsCapturing(h->stream, &cs));
+    if (cs != hipStreamCaptureStatusNone) h->captured = true;
+    if (h->captured || !h->fresh) {
+        reset_run(h, h->stream);
+        HIPCHK(hipGetLastError());
+    }
+    h->fresh = false;
     if (h->sg_on && nsteps >= 2 * SG_ITERS && cs == hipStreamCaptureStatusNone) {
         if ((rc = self_graph_ready(h, tol))) return rc;
         // SG_ITERS is even: every replay leaves the parity where it was
@@ -1911,7 +1959,7 @@ int pfdd_gl_step(pfdd_gl *h, int nsteps, double tol, pfdd_gl_reduce *out)
         if ((rc = step_any(h, tol, s == 0, s == eager - 1))) return rc;
     }
     if (!out && tol <= 0) return PFDD_OK;
-    return collect_steps(h, cur0, out);
+    return collect_steps(h, cur0, nsteps, out);
 }
 
 int pfdd_gl_tape_record(pfdd_gl *h, int nsteps, int every, pfdd_gl_reduce *out)
@@ -1939,7 +1987,7 @@ int pfdd_gl_tape_record(pfdd_gl *h, int nsteps, int every, pfdd_gl_reduce *out)
         HIPCHK(hipMalloc(&p, fb));
         T.ckpt.push_back(p);
     }
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
+    reset_run(h, h->stream);
     HIPCHK(hipGetLastError());
     const int cur0 = h->cur;
     for (int s = 0; s < nsteps; ++s) {
@@ -1948,7 +1996,7 @@ int pfdd_gl_tape_record(pfdd_gl *h, int nsteps, int every, pfdd_gl_reduce *out)
         if ((rc = step_any(h, 0.0, s == 0, s == nsteps - 1))) return rc;
     }
     pfdd_gl_reduce r{};
-    if ((rc = collect_steps(h, cur0, &r))) return rc;
+    if ((rc = collect_steps(h, cur0, nsteps, &r))) return rc;
     if (out) *out = r;
     T.nsteps = nsteps;
     T.every = every;
@@ -2090,7 +2138,7 @@ int pfdd_gl_profile(pfdd_gl *h, int nsteps, double *ms, int *nkernels)
     std::vector<hipEvent_t> ev((size_t)12 * nsteps);
     for (auto &e : ev) HIPCHK(hipEventCreate(&e));
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, h->stream, h->done, h->steps);
+    reset_run(h, h->stream);
     for (int s = 0; s < nsteps && !rc; ++s)
         rc = h->prec == PFDD_FP64 ? step_once<double>(h, 0.0, &ev[12 * s], s == 0, false)
                                   : step_once<float>(h, 0.0, &ev[12 * s], s == 0, false);
@@ -2260,7 +2308,7 @@ int pfdd_gl_graph_run(pfdd_gl_graph *g, int nsteps, double tol, pfdd_gl_reduce *
     for (size_t i = 0; i < n; ++i) {
         pfdd_gl *h = g->hs[i];
         cur0[i] = h->cur;
-        hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, g->stream, h->done, h->steps);
+        reset_run(h, g->stream);
         HIPCHK(hipGetLastError());
     }
     for (int r = 0; r < nsteps / g->iters; ++r) HIPCHK(hipGraphLaunch(g->exec, g->stream));
@@ -2278,7 +2326,7 @@ int pfdd_gl_graph_run(pfdd_gl_graph *g, int nsteps, double tol, pfdd_gl_reduce *
     int first_err = PFDD_OK;
     for (size_t i = 0; i < n; ++i) {
         pfdd_gl_reduce r{};
-        rc = collect_steps(g->hs[i], cur0[i], &r);
+        rc = collect_steps(g->hs[i], cur0[i], nsteps, &r);
         if (rc && !first_err) first_err = rc;
         if (out) out[i] = r;
     }

@@ -457,7 +457,7 @@ template <typename R> int mid_blocks(int n, int S, long long ncol);
 template <typename R> bool mid_supported(int n, int S);
 template <typename R>
 hipError_t launch_mid(int n, int S, int M, void *T2, const void *B, long long ncol, long long ntot, const void *tw,
-                      double *part_el, const int *done, hipStream_t st);
+                      double *part_el, const int *done, hipStream_t st, int *nblocks);
 template <typename R>
 hipError_t launch_mid_otf(int n, int S, int M, void *T2, const GParams &G, long long ncol, long long ntot,
                           const void *tw, double *part_el, const int *done, hipStream_t st, int pipe, int ncu,

@@ -757,7 +757,7 @@ template <typename R, int N, int S> constexpr bool mid_fits()
 
 template <typename R, int S>
 hipError_t launch_mid_s(int n, int M, void *T2, const void *B, long long ncol, long long ntot, const void *tw,
-                        double *part_el, const int *done, hipStream_t st)
+                        double *part_el, const int *done, hipStream_t st, int *nblocks)
 {
     typedef typename cvec<R>::type V;
 #define PFDD_CASE(n_)                                                                             \
@@ -765,6 +765,7 @@ hipError_t launch_mid_s(int n, int M, void *T2, const void *B, long long ncol, l
         if constexpr (mid_fits<R, n_, S>()) {                                                     \
             constexpr int NP = mid_pairs<R, n_, S>();                                             \
             const int bpm = (int)((ncol + NP - 1) / NP);                                          \
+            *nblocks = M * bpm;                                                                   \
             PFDD_LAUNCH((k_mid<R, R, n_, S>), dim3((unsigned)(M * bpm)), dim3(NTHR), st,          \
                                (V *)T2, (const R *)B, ncol, ntot, bpm, (const V *)tw, part_el, done); \
             return hipGetLastError();                                                             \
@@ -800,15 +801,15 @@ bool mid_supported(int n, int S)
 
 template <typename R>
 hipError_t launch_mid(int n, int S, int M, void *T2, const void *B, long long ncol, long long ntot, const void *tw,
-                      double *part_el, const int *done, hipStream_t st)
+                      double *part_el, const int *done, hipStream_t st, int *nblocks)
 {
     switch (S) {
-    case 1: return launch_mid_s<R, 1>(n, M, T2, B, ncol, ntot, tw, part_el, done, st);
-    case 2: return launch_mid_s<R, 2>(n, M, T2, B, ncol, ntot, tw, part_el, done, st);
-    case 3: return launch_mid_s<R, 3>(n, M, T2, B, ncol, ntot, tw, part_el, done, st);
-    case 4: return launch_mid_s<R, 4>(n, M, T2, B, ncol, ntot, tw, part_el, done, st);
-    case 6: return launch_mid_s<R, 6>(n, M, T2, B, ncol, ntot, tw, part_el, done, st);
-    case 12: return launch_mid_s<R, 12>(n, M, T2, B, ncol, ntot, tw, part_el, done, st);
+    case 1: return launch_mid_s<R, 1>(n, M, T2, B, ncol, ntot, tw, part_el, done, st, nblocks);
+    case 2: return launch_mid_s<R, 2>(n, M, T2, B, ncol, ntot, tw, part_el, done, st, nblocks);
+    case 3: return launch_mid_s<R, 3>(n, M, T2, B, ncol, ntot, tw, part_el, done, st, nblocks);
+    case 4: return launch_mid_s<R, 4>(n, M, T2, B, ncol, ntot, tw, part_el, done, st, nblocks);
+    case 6: return launch_mid_s<R, 6>(n, M, T2, B, ncol, ntot, tw, part_el, done, st, nblocks);
+    case 12: return launch_mid_s<R, 12>(n, M, T2, B, ncol, ntot, tw, part_el, done, st, nblocks);
     }
     return hipErrorInvalidValue;
 }
@@ -935,7 +936,7 @@ int mid_pl_blocks(int n, int S, int M, long long ncol)
     template int mid_blocks<R>(int, int, long long);                                                              \
     template bool mid_supported<R>(int, int);                                                                     \
     template hipError_t launch_mid<R>(int, int, int, void *, const void *, long long, long long, const void *,     \
-                                      double *, const int *, hipStream_t);                                        \
+                                      double *, const int *, hipStream_t, int *);                                        \
     template hipError_t launch_mid_otf<R>(int, int, int, void *, const GParams &, long long, long long,            \
                                           const void *, double *, const int *, hipStream_t, int, int, int *);      \
     template hipError_t launch_mid_pl<R>(int, int, int, void *, const GParams &, long long, long long,             \

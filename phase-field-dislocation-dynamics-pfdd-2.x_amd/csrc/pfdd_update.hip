@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(updat
     const int nm = P.ncoef;
     // each thread sums at most 16 cells in FP64 (relative error below 16 u);
     // the block level is a pairwise tree with a compensated wave combine
-    // (block_sum_comp), the grid level a Kahan sum (k_reduce)
+    // (block_sum_comp), the grid level a Kahan sum (k_sums)
     double s_norm = 0.0, s_ave = 0.0, s_core = 0.0, s_str = 0.0;
 #pragma unroll
     for (int t = 0; t < PER; ++t) {

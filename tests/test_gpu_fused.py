@@ -56,3 +56,26 @@ def test_run_equals_single_iterations(precision, shape, systems, core, choice):
     finally:
         a.close()
         b.close()
+
+
+def test_run_counters_over_runs_of_every_kind():
+    """A run counts its own iterations and reports its own end, whatever ran
+    on the handle before it: runs that were not waited for, converged runs,
+    empty runs, graph replays (20 iterations and more)."""
+    case = P.make_case(shape=(32, 32, 32), systems="basal3", core="sine", noise=1e-2, sigma_mu=0.004)
+    g = P.gpu_solver(case)
+    try:
+        g.step(3, sync=False)
+        for n, tol, done in ((2, 0.0, 0), (50, 1e30, 1), (4, 0.0, 0), (0, 0.0, 0), (25, 0.0, 0), (25, 1e30, 1),
+                             (3, 1e-300, 0)):
+            r = g.step(n, tol=tol)
+            assert (r["steps_done"], r["converged"]) == (1 if done else n, done), (n, tol, r)
+            g.step(1, sync=False)
+        h = P.gpu_solver(case)
+        try:
+            h.step(3 + 2 + 1 + 4 + 25 + 1 + 3 + 7)
+            assert np.array_equal(g.get_xi(), h.get_xi())
+        finally:
+            h.close()
+    finally:
+        g.close()
