@@ -25,7 +25,8 @@ def run(cmd):
 
 # Translation units of the HIP library, compiled in parallel and linked
 # into one shared object (no device code crosses a unit boundary).
-HIP_UNITS = ("pfdd_gl.hip", "pfdd_pass.hip", "pfdd_update.hip", "pfdd_mid.hip", "pfdd_plane.hip")
+HIP_UNITS = ("pfdd_gl.hip", "pfdd_pass.hip", "pfdd_update.hip", "pfdd_mid.hip", "pfdd_plane.hip",
+             "pfdd_cond.hip")
 
 
 def build_lib():

@@ -2359,97 +2359,6 @@ int pfdd_gl_graph_destroy(pfdd_gl_graph *g)
 // from the host as two arrays over the y index j: sig[j] (condsigma of row
 // j, scattering included) and dsig[j] (the difference of the bulk
 // conductivity across row j that multiplies the applied-field term).
-namespace {
-
-struct CondParams {
-    double four[9];
-    double El;       // material->El[1]
-    double eps0;     // material->epsilonzero
-    double rate;     // 1e-22 * app->timestep
-    double invN;     // 1 / (nx ny nz)
-    int nx, ny, nz;
-};
-
-// divcurrent on the transformed field in the [k][j][i] layout: a = i c f_y /
-// f^2 and b = c f_y^2 / f^2 (zero at f = 0), written as [2][k][j][i].  The
-// block also sums sig[(ny - j) mod ny] Re a over its k-points: backwardcond
-// called a second time on its own output (the trailing call of
-// SolveGLCond::iterate) transforms a back once more, and two unnormalised
-// inverse transforms give N a(-r).
-__global__ void __launch_bounds__(NTHR)
-    k_cond_div(const double2 *__restrict__ ch, double2 *__restrict__ ab, const double *__restrict__ sig, CondParams P,
-               long long N, double *__restrict__ part)
-{
-    __shared__ double red[NTHR / 64];
-    const int tid = threadIdx.x;
-    const long long idx = (long long)blockIdx.x * NTHR + tid;
-    double v[1] = {0.0};
-    if (idx < N) {
-        const int i = (int)(idx % P.nx);
-        const int j = (int)((idx / P.nx) % P.ny);
-        const int k = (int)(idx / ((long long)P.nx * P.ny));
-        const double kx = frac_freq(i, P.nx), ky = frac_freq(j, P.ny), kz = frac_freq(k, P.nz);
-        double f[3];
-        for (int c = 0; c < 3; ++c) f[c] = kx * P.four[c] + ky * P.four[3 + c] + kz * P.four[6 + c];
-        const double f2 = f[0] * f[0] + f[1] * f[1] + f[2] * f[2];
-        const double2 c = ch[idx];
-        double2 a = make_double2(0.0, 0.0), b = make_double2(0.0, 0.0);
-        if (f2 > 0.0) {
-            a.x = -(c.y * f[1] / f2);
-            a.y = c.x * f[1] / f2;
-            b.x = c.x * f[1] * f[1] / f2;
-            b.y = c.y * f[1] * f[1] / f2;
-        }
-        ab[idx] = a;
-        ab[N + idx] = b;
-        v[0] = sig[(P.ny - j) % P.ny] * a.x;
-    }
-    block_sum<1, NTHR>(v, red, tid);
-    if (tid == 0) part[blockIdx.x] = v[0];
-}
-
-// backwardcond's per-cell assembly on the (unnormalised) inverse transforms
-// a, b in the [2][i][j][k] layout, then update_conduct_order_param:
-//   j     = sig (El - Re a / eps0) - i sig Im a / eps0
-//   rhs   = (sig / eps0) b + (a / eps0 - El) dsig      (El on the real part)
-//   c    -= rate * rhs / N
-// Block sums: Re j, Im j, |dc|^2, Re c_new.
-__global__ void __launch_bounds__(NTHR)
-    k_cond_update(const double2 *__restrict__ ab, double2 *__restrict__ c, const double *__restrict__ sig,
-                  const double *__restrict__ dsig, CondParams P, long long N, double *__restrict__ part,
-                  long long pstride)
-{
-    __shared__ double red[4 * (NTHR / 64)];
-    const int tid = threadIdx.x;
-    const long long idx = (long long)blockIdx.x * NTHR + tid;
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
-    if (idx < N) {
-        const int j = (int)((idx / P.nz) % P.ny);
-        const double2 a = ab[idx], b = ab[N + idx];
-        const double s = sig[j], ds = dsig[j];
-        const double jr = s * (P.El - a.x / P.eps0);
-        const double ji = -s * a.y / P.eps0;
-        double rr = (s / P.eps0) * b.x, ri = (s / P.eps0) * b.y;
-        rr += (a.x / P.eps0 - P.El) * ds;
-        ri += (a.y / P.eps0) * ds;
-        const double2 c0 = c[idx];
-        double2 c1;
-        c1.x = c0.x - (P.rate * (rr * P.invN));
-        c1.y = c0.y - (P.rate * (ri * P.invN));
-        c[idx] = c1;
-        const double dr = c1.x - c0.x, di = c1.y - c0.y;
-        v[0] = jr;
-        v[1] = ji;
-        v[2] = dr * dr + di * di;
-        v[3] = c1.x;
-    }
-    block_sum<4, NTHR>(v, red, tid);
-    if (tid == 0)
-        for (int q = 0; q < 4; ++q) part[q * pstride + blockIdx.x] = v[q];
-}
-
-} // namespace
-
 struct pfdd_gl_cond {
     int device = 0, nx = 0, ny = 0, nz = 0;
     long long N = 0;
@@ -2461,7 +2370,8 @@ struct pfdd_gl_cond {
     double *sig = nullptr, *dsig = nullptr, *part = nullptr;
     int *done = nullptr;
     std::vector<double> sig_h;
-    long long nb = 0;
+    long long nb = 0;         // most partials of a kernel
+    CondStat *stat = nullptr; // pinned host memory
 };
 
 namespace {
@@ -2471,53 +2381,52 @@ void cond_release(pfdd_gl_cond *h)
     for (void *p : {(void *)h->c, (void *)h->w0, (void *)h->w1, (void *)h->sig, (void *)h->dsig, (void *)h->part,
                     (void *)h->done, h->tw[0], h->tw[1], h->tw[2]})
         if (p) hipFree(p);
+    if (h->stat) (void)hipHostFree(h->stat);
     if (h->own_stream && h->stream) hipStreamDestroy(h->stream);
 }
 
 // Same line maps as the GL passes, for S fields of the cond grid.
 Maps cond_maps(const pfdd_gl_cond *h, long long S) { return make_maps_dims(h->nx, h->ny, h->nz, S); }
 
-int cond_step(pfdd_gl_cond *h, pfdd_gl_cond_reduce *out)
+// One iteration of a run.  first: c enters the run here; last: nothing follows.
+int cond_step(pfdd_gl_cond *h, bool first, bool last, int &nu, int &nd)
 {
     hipStream_t st = h->stream;
     const Maps m1 = cond_maps(h, 1), m2 = cond_maps(h, 2);
     const long long ncol = (long long)h->ny * h->nz;
     const LineMap xs = {h->nx, 0, 0, 1, 1, 1};
-    // forwardcond: FFT of c (z, y, x passes) -> w0 in [k][j][i]
-    HIPCHK((launch_pass<double, false>(h->nz, h->c, h->w0, m1.p1i, m1.p1o, m1.n1, h->tw[2], h->done, st)));
-    HIPCHK((launch_pass<double, false>(h->ny, h->w0, h->w1, m1.p2i, m1.p2o, m1.n2, h->tw[1], h->done, st)));
-    HIPCHK((launch_pass<double, false>(h->nx, h->w1, h->w0, xs, xs, ncol, h->tw[0], h->done, st)));
-    // divcurrent -> w1 = [a, b] in k space
-    const unsigned nb = (unsigned)h->nb;
-    hipLaunchKernelGGL(k_cond_div, dim3(nb), dim3(NTHR), 0, st, (const double2 *)h->w0, h->w1, h->sig, h->P, h->N,
-                       h->part + 4 * h->nb);
-    HIPCHK(hipGetLastError());
-    // backwardcond's two inverse transforms -> w0 = [a, b] in [2][i][j][k]
-    HIPCHK((launch_pass<double, true>(h->nx, h->w1, h->w0, xs, xs, 2 * ncol, h->tw[0], h->done, st)));
-    HIPCHK((launch_pass<double, true>(h->ny, h->w0, h->w1, m2.p2o, m2.p2i, m2.n2, h->tw[1], h->done, st)));
-    HIPCHK((launch_pass<double, true>(h->nz, h->w1, h->w0, m2.p5i, m2.p5o, m2.n5, h->tw[2], h->done, st)));
-    hipLaunchKernelGGL(k_cond_update, dim3(nb), dim3(NTHR), 0, st, (const double2 *)h->w0, h->c, h->sig, h->dsig,
-                       h->P, h->N, h->part, h->nb);
-    HIPCHK(hipGetLastError());
-    std::vector<double> part((size_t)5 * h->nb);
-    HIPCHK(hipMemcpyAsync(part.data(), h->part, sizeof(double) * part.size(), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    // block partials summed in block order: deterministic
-    double s[5] = {0, 0, 0, 0, 0};
-    for (int q = 0; q < 5; ++q)
-        for (long long b = 0; b < h->nb; ++b) s[q] += part[(size_t)q * h->nb + b];
-    if (!std::isfinite(s[0]) || !std::isfinite(s[2]) || !std::isfinite(s[3]))
-        return fail(PFDD_ERR_NONFINITE, "non-finite conductivity reduction");
-    if (out) {
-        double mean_sig = 0.0;
-        for (double v : h->sig_h) mean_sig += v;
-        mean_sig /= (double)h->ny;
-        out->javerage_re = s[0] * h->P.invN;
-        out->javerage_im = s[1] * h->P.invN;
-        out->conductivity = out->javerage_re / h->P.El;
-        out->condxinorm = std::sqrt(s[2]);
-        out->condxiave = s[3];
-        out->conductivity_repeat = (h->P.El * mean_sig - s[4] / h->P.eps0) / h->P.El;
+    const bool xr = cond_reg_length(h->nx), zr = cond_reg_length(h->nz);
+    // forwardcond: FFT of c; divcurrent; backwardcond's two inverse
+    // transforms; every pass from one work buffer to the other
+    double2 *in = h->w0, *out = h->w1;
+    auto swap = [&] { std::swap(in, out); };
+    if (first || !zr) // (with the radix plan of the update's own forward transform)
+        HIPCHK((launch_pass<double, false>(h->nz, h->c, in, m1.p1i, m1.p1o, m1.n1, h->tw[2], h->done, st, nullptr,
+                                           zr ? 4 : 1)));
+    HIPCHK((launch_pass<double, false>(h->ny, in, out, m1.p2i, m1.p2o, m1.n2, h->tw[1], h->done, st)));
+    swap();
+    if (xr) {
+        HIPCHK(launch_cond_x(in, out, h->sig, h->P, h->tw[0], h->part + 4 * h->nb, &nd, h->done, st));
+        swap();
+    } else {
+        HIPCHK((launch_pass<double, false>(h->nx, in, out, xs, xs, ncol, h->tw[0], h->done, st)));
+        swap();
+        HIPCHK(launch_cond_div(in, out, h->sig, h->P, h->part + 4 * h->nb, &nd, h->done, st));
+        swap();
+        HIPCHK((launch_pass<double, true>(h->nx, in, out, xs, xs, 2 * ncol, h->tw[0], h->done, st)));
+        swap();
+    }
+    HIPCHK((launch_pass<double, true>(h->ny, in, out, m2.p2o, m2.p2i, m2.n2, h->tw[1], h->done, st)));
+    swap();
+    if (zr) {
+        // in is w1 here: the transform of the new c goes to w0, where the next
+        // iteration starts
+        HIPCHK(launch_cond_update_r(!last, in, h->c, out, h->sig, h->dsig, h->P, h->tw[2], h->part, h->nb, &nu,
+                                    h->done, st));
+    } else {
+        HIPCHK((launch_pass<double, true>(h->nz, in, out, m2.p5i, m2.p5o, m2.n5, h->tw[2], h->done, st)));
+        swap();
+        HIPCHK(launch_cond_update(in, h->c, h->sig, h->dsig, h->P, h->part, h->nb, &nu, h->done, st));
     }
     return PFDD_OK;
 }
@@ -2572,7 +2481,8 @@ int pfdd_gl_cond_create(const pfdd_gl_cond_desc *d, pfdd_gl_cond **out)
         (e = hipMalloc((void **)&h->sig, sizeof(double) * d->ny)) != hipSuccess ||
         (e = hipMalloc((void **)&h->dsig, sizeof(double) * d->ny)) != hipSuccess ||
         (e = hipMalloc((void **)&h->part, sizeof(double) * 5 * h->nb)) != hipSuccess ||
-        (e = hipMalloc((void **)&h->done, sizeof(int))) != hipSuccess)
+        (e = hipMalloc((void **)&h->done, sizeof(int))) != hipSuccess ||
+        (e = hipHostMalloc((void **)&h->stat, sizeof(CondStat), hipHostMallocDefault)) != hipSuccess)
         return bail(fail(PFDD_ERR_HIP, "hipMalloc: %s", hipGetErrorString(e)));
     const int dims[3] = {h->nx, h->ny, h->nz};
     for (int q = 0; q < 3; ++q) {
@@ -2625,9 +2535,29 @@ int pfdd_gl_cond_step(pfdd_gl_cond *h, int nsteps, pfdd_gl_cond_reduce *out)
     if (!h) return fail(PFDD_ERR_ARG, "null handle");
     if (nsteps < 1) return fail(PFDD_ERR_ARG, "nsteps must be >= 1");
     HIPCHK(hipSetDevice(h->device));
+    // the host waits once, at the end of the run (a wait, a copy of the
+    // partials and a sum on the host after every iteration cost 70 us of 225
+    // at 128^3); an iteration with sums that are not finite stops the rest
+    int nu = 0, nd = 0;
     for (int s = 0; s < nsteps; ++s) {
-        const int rc = cond_step(h, out);
+        const int rc = cond_step(h, s == 0, s == nsteps - 1, nu, nd);
         if (rc) return rc;
+    }
+    HIPCHK(launch_cond_sums(h->part, h->nb, nu, nd, h->stat, h->done, h->stream));
+    HIPCHK(hipStreamSynchronize(h->stream));
+    const double *s = h->stat->s;
+    if (h->stat->done || !std::isfinite(s[0]) || !std::isfinite(s[2]) || !std::isfinite(s[3]))
+        return fail(PFDD_ERR_NONFINITE, "non-finite conductivity reduction");
+    if (out) {
+        double mean_sig = 0.0;
+        for (double v : h->sig_h) mean_sig += v;
+        mean_sig /= (double)h->ny;
+        out->javerage_re = s[0] * h->P.invN;
+        out->javerage_im = s[1] * h->P.invN;
+        out->conductivity = out->javerage_re / h->P.El;
+        out->condxinorm = std::sqrt(s[2]);
+        out->condxiave = s[3];
+        out->conductivity_repeat = (h->P.El * mean_sig - s[4] / h->P.eps0) / h->P.El;
     }
     return PFDD_OK;
 }

@@ -484,4 +484,37 @@ hipError_t launch_plane_upd(int ny, int nz, bool fw, void *T, const void *xo, vo
                             const StepParams &P, const void *twy, const void *twz, double *partial,
                             long long pstride, const int *done, hipStream_t st);
 
+// Conductivity sub-problem (pfdd_cond.hip).  c is [i][j][k]; divcurrent reads
+// [k][j][i] and writes a, b as [2][k][j][i]; launch_cond_x also makes the x
+// transforms around it; the updates read a, b as [2][i][j][k], and
+// launch_cond_update_r, which also makes the z transforms before it (and with
+// fw the next forward one, into T [i][k][j]), as [2][i][k][j].  nparts: blocks,
+// that is partial sums, of a launch.  *done is raised by an update whose sums
+// are not finite; everything but the updates then returns at once.
+struct CondParams {
+    double four[9];
+    double El;       // material->El[1]
+    double eps0;     // material->epsilonzero
+    double rate;     // 1e-22 * app->timestep
+    double invN;     // 1 / (nx ny nz)
+    int nx, ny, nz;
+};
+struct CondStat {
+    double s[5]; // Re j, Im j, |dc|^2, Re c, sig Re a (divcurrent)
+    int done;
+};
+bool cond_reg_length(int n); // the length has the fused kernels
+hipError_t launch_cond_div(const double2 *ch, double2 *ab, const double *sig, const CondParams &P, double *part,
+                           int *nparts, const int *done, hipStream_t st);
+hipError_t launch_cond_x(const double2 *ch, double2 *ab, const double *sig, const CondParams &P, const void *tw,
+                         double *part, int *nparts, const int *done, hipStream_t st);
+hipError_t launch_cond_update(const double2 *ab, double2 *c, const double *sig, const double *dsig,
+                              const CondParams &P, double *part, long long pstride, int *nparts, int *done,
+                              hipStream_t st);
+hipError_t launch_cond_update_r(bool fw, const double2 *ab, double2 *c, double2 *T, const double *sig,
+                                const double *dsig, const CondParams &P, const void *tw, double *part,
+                                long long pstride, int *nparts, int *done, hipStream_t st);
+hipError_t launch_cond_sums(const double *part, long long pstride, int nu, int nd, CondStat *stat, int *done,
+                            hipStream_t st);
+
 } // namespace pfdd
