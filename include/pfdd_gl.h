@@ -296,7 +296,7 @@ int pfdd_gl_traffic(pfdd_gl *h, double *bytes_per_kernel, double *bytes_per_step
  * one hipGraph of `iters` (even) GL iterations, replayed nsteps/iters times
  * (the remainder runs eagerly); no host synchronisation inside the run.  No
  * counterpart in the reference.  The graph is captured on first use and again
- * after set_core_coef, a single-run handle's set_tau, a change of tol or an
+ * after set_core_coef, a change of tol or an
  * odd number of steps taken outside the graph.  pfdd_gl_graph_run reports
  * each handle's last iteration in out[i] (may be NULL); tol as in
  * pfdd_gl_step, per handle. */

@@ -45,6 +45,7 @@
 #include <vector>
 
 #include "pfdd_kern.hpp"
+#include "pfdd_stage.hpp"
 
 using namespace pfdd;
 
@@ -314,6 +315,14 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+struct TauArg {
+    double v[MAXS];
+};
+__global__ void k_set_tau(double *taud, TauArg tau, int n)
+{
+    if ((int)threadIdx.x < n) taud[threadIdx.x] = tau.v[threadIdx.x];
+}
+
 __global__ void k_reset(int *done, int *steps)
 {
     if (threadIdx.x == 0) {
@@ -488,12 +497,9 @@ __global__ void __launch_bounds__(NTHR)
     const int ci[6] = {0, 1, 2, 0, 0, 1}, cj[6] = {0, 1, 2, 1, 2, 2};
     for (int c = 0; c < 6; ++c) {
         const int ii = ci[c], jj = cj[c];
-        const double2 e = make_double2(er[c] + P.avepst6[c], ei[c]);
-        const double sv = 2.0 * P.C44 * x[c] + (ii == jj ? P.C12 * tr : 0.0);
-        eps[(long long)(ii + 3 * jj) * ntot + r] = e;
-        eps[(long long)(jj + 3 * ii) * ntot + r] = e;
-        sig[(long long)(ii + 3 * jj) * ntot + r] = sv + P.sigmu[3 * ii + jj];
-        sig[(long long)(jj + 3 * ii) * ntot + r] = sv + P.sigmu[3 * jj + ii];
+        // the symmetric components once; the host spreads them
+        eps[(long long)c * ntot + r] = make_double2(er[c] + P.avepst6[c], ei[c]);
+        sig[(long long)c * ntot + r] = 2.0 * P.C44 * x[c] + (ii == jj ? P.C12 * tr : 0.0);
     }
 }
 
@@ -503,9 +509,9 @@ __global__ void __launch_bounds__(NTHR)
 struct pfdd_gl {
     int nx = 0, ny = 0, nz = 0, S = 0, prec = PFDD_FP64;
     int M = 1, SM = 0;      // members of a batch, systems over all members (S*M)
-    double *taud = nullptr; // device tau[SM] of a batch
+    double *taud = nullptr; // device tau[SM]: of a batch, and for the captured graphs of a single-run handle
     void *cof = nullptr;    // core flag 5: per-element angle factor (R), refreshed every iteration
-    unsigned version = 0;   // bumped when kernel arguments change (tau, core coefficients)
+    unsigned version = 0;   // bumped when kernel arguments change (core coefficients, tiles)
     long long N = 0;
     size_t esz = 16; // bytes per complex element
     int device = 0;
@@ -563,8 +569,11 @@ struct pfdd_gl {
     double four[9];
     bool stepped = false; // a step ran since the last set_xi (xi[1-cur] holds the pre-update field)
     void *dw[2] = {nullptr, nullptr}; // output-step field workspace, max(S,6)*N complex each
-    double2 *deps = nullptr;          // 9*N strain field (complex)
-    double *dsig = nullptr;           // 9*N stress field (real)
+    double2 *deps = nullptr;          // strain field (complex), 6 components of N
+    double *dsig = nullptr;           // stress field (real) without sigma_rot, 6 components of N
+    Stage stage;                      // fields to and from the caller's memory
+    double *xs_part = nullptr;        // XS_NB * SM block sums of xi_sums, pinned host memory
+    bool tau_stale = true;            // single-run handle: taud does not hold P.tau
     // reverse mode: checkpoints of a recorded run and the adjoint workspace
     struct Tape {
         int nsteps = 0, every = 0;
@@ -657,6 +666,28 @@ void reset_run(pfdd_gl *h, hipStream_t st)
     hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, st, h->done, h->steps);
     h->steps0 = 0;
     h->fresh = false;
+}
+
+// A single-run handle passes tau to its kernels by value, and to those of a
+// captured graph in device memory, so that a new stress needs no new capture
+// (0.4 ms, a tenth of 100 iterations at 64^3): GraphTau around a capture,
+// graph_tau before a replay on st.
+struct GraphTau {
+    pfdd_gl *h;
+    const double *saved;
+    explicit GraphTau(pfdd_gl *h_) : h(h_), saved(h_->P.taud) { h->P.taud = h->taud; }
+    ~GraphTau() { h->P.taud = saved; }
+};
+int graph_tau(pfdd_gl *h, hipStream_t st)
+{
+    if (h->M > 1 || !h->tau_stale) return PFDD_OK;
+    static_assert(MAXS <= 64, "one wave writes tau");
+    TauArg t{};
+    for (int a = 0; a < h->S; ++a) t.v[a] = h->P.tau[a];
+    hipLaunchKernelGGL(k_set_tau, dim3(1), dim3(64), 0, st, h->taud, t, h->S);
+    HIPCHK(hipGetLastError());
+    h->tau_stale = false;
+    return PFDD_OK;
 }
 
 // One GL iteration from xo into T2 (T2 doubles as the temporary of passes
@@ -1101,6 +1132,8 @@ void destroy_all(pfdd_gl *h)
     for (void *p : h->tape.seg)
         if (p) hipFree(p);
     if (h->stat) (void)hipHostFree(h->stat);
+    if (h->xs_part) (void)hipHostFree(h->xs_part);
+    h->stage.release();
     if (h->own_stream && h->stream) hipStreamDestroy(h->stream);
     delete h;
 }
@@ -1224,6 +1257,19 @@ int build_B(pfdd_gl *h)
     return PFDD_OK;
 }
 
+// bytes to pageable host memory as they are.
+int copy_out(Stage &stage, const void *dev, void *host, size_t bytes, hipStream_t st)
+{
+    if (bytes < Stage::MIN_BYTES) {
+        HIPCHK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        return PFDD_OK;
+    }
+    HIPCHK(stage.out((char *)dev, bytes, st,
+                      [&](char *slot, size_t o, size_t n) { std::memcpy((char *)host + o, slot, n); }));
+    return PFDD_OK;
+}
+
 int upload_field_f64(pfdd_gl *h, const double *host, void *dst)
 {
     const long long n = (long long)h->SM * h->N;
@@ -1248,26 +1294,17 @@ int upload_field_f64(pfdd_gl *h, const double *host, void *dst)
     return PFDD_OK;
 }
 
+// The field to FP64 host memory; FP32 fields are widened on the way through the
+// slots.
 int download_field_f64(pfdd_gl *h, const void *src, double *host)
 {
-    const long long n = (long long)h->SM * h->N;
-    if (h->prec == PFDD_FP64) {
-        HIPCHK(hipMemcpyAsync(host, src, (size_t)n * 16, hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(hipStreamSynchronize(h->stream));
-        return PFDD_OK;
-    }
-    const long long chunk = 1LL << 22;
-    void *tmp = nullptr;
-    HIPCHK(hipMalloc(&tmp, (size_t)chunk * 16));
-    for (long long o = 0; o < n; o += chunk) {
-        const long long c = (n - o) < chunk ? (n - o) : chunk;
-        hipLaunchKernelGGL((k_to_f64<float>), dim3((unsigned)((c + 255) / 256)), dim3(256), 0, h->stream,
-                           (const float2 *)src + o, (double2 *)tmp, c);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(host + 2 * o, tmp, (size_t)c * 16, hipMemcpyDeviceToHost, h->stream));
-    }
-    HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(hipFree(tmp));
+    const size_t n = (size_t)h->SM * h->N * 2;
+    if (h->prec == PFDD_FP64) return copy_out(h->stage, src, host, n * 8, h->stream);
+    HIPCHK(h->stage.out((char *)src, n * 4, h->stream, [&](char *slot, size_t o, size_t len) {
+        const float *from = (const float *)slot;
+        double *to = host + o / 4;
+        for (size_t q = 0; q < len / 4; ++q) to[q] = (double)from[q];
+    }));
     return PFDD_OK;
 }
 
@@ -1279,8 +1316,8 @@ int diag_fields(pfdd_gl *h, const double *sigma_rot, const double *avepst, const
     const size_t wbytes = (size_t)SC * N * h->esz;
     for (int q = 0; q < 2; ++q)
         if (!h->dw[q]) HIPCHK(hipMalloc(&h->dw[q], wbytes));
-    if (!h->deps) HIPCHK(hipMalloc(&h->deps, sizeof(double2) * 9 * N));
-    if (!h->dsig) HIPCHK(hipMalloc(&h->dsig, sizeof(double) * 9 * N));
+    if (!h->deps) HIPCHK(hipMalloc(&h->deps, sizeof(double2) * 6 * N));
+    if (!h->dsig) HIPCHK(hipMalloc(&h->dsig, sizeof(double) * 6 * N));
     DParams P{};
     const int ci[6] = {0, 1, 2, 0, 0, 1}, cj[6] = {0, 1, 2, 1, 2, 2};
     for (int a = 0; a < S; ++a)
@@ -1327,18 +1364,43 @@ int diag_fields(pfdd_gl *h, const double *sigma_rot, const double *avepst, const
     hipLaunchKernelGGL((k_diag_real<R>), dim3(nb), dim3(NTHR), 0, st, (const V *)h->dw[0],
                        (const V *)h->xi[h->cur], h->deps, h->dsig, P, N);
     HIPCHK(hipGetLastError());
-    if (data_eps) HIPCHK(hipMemcpyAsync(data_eps, h->deps, sizeof(double2) * 9 * N, hipMemcpyDeviceToHost, st));
-    std::vector<double> sg;
-    if (data_sigma) {
-        sg.resize((size_t)9 * N);
-        HIPCHK(hipMemcpyAsync(sg.data(), h->dsig, sizeof(double) * 9 * N, hipMemcpyDeviceToHost, st));
-    }
-    HIPCHK(hipStreamSynchronize(st));
-    if (data_sigma)
-        for (long long q = 0; q < 9 * N; ++q) {
-            data_sigma[2 * q] = sg[q];
-            data_sigma[2 * q + 1] = 0.0;
+    // component c = (i, j) goes to i + 3 j and j + 3 i of the caller's nine; the
+    // chunks run over component boundaries.  each(c, r0, n, from): n values of
+    // component c from cell r0 on
+    auto spread = [&](const char *slot, size_t o, size_t len, size_t esz, auto each) {
+        for (size_t q = o / esz, end = (o + len) / esz; q < end;) {
+            const size_t c = q / N, r0 = q % N, n = std::min((size_t)N - r0, end - q);
+            each((int)c, r0, n, slot + (q * esz - o));
+            q += n;
         }
+    };
+    if (data_eps)
+        HIPCHK(h->stage.out((char *)h->deps, sizeof(double2) * 6 * N, st, [&](char *slot, size_t o, size_t len) {
+            spread(slot, o, len, sizeof(double2), [&](int c, size_t r0, size_t n, const char *from) {
+                std::memcpy(data_eps + 2 * ((ci[c] + 3 * cj[c]) * N + r0), from, n * sizeof(double2));
+                if (ci[c] != cj[c])
+                    std::memcpy(data_eps + 2 * ((cj[c] + 3 * ci[c]) * N + r0), from, n * sizeof(double2));
+            });
+        }));
+    if (data_sigma)
+        HIPCHK(h->stage.out((char *)h->dsig, sizeof(double) * 6 * N, st, [&](char *slot, size_t o, size_t len) {
+            spread(slot, o, len, sizeof(double), [&](int c, size_t r0, size_t n, const char *from) {
+                const double *v = (const double *)from;
+                const int i = ci[c], j = cj[c];
+                double *to = data_sigma + 2 * ((i + 3 * j) * N + r0);
+                for (size_t q = 0; q < n; ++q) {
+                    to[2 * q] = v[q] + P.sigmu[3 * i + j];
+                    to[2 * q + 1] = 0.0;
+                }
+                if (i == j) return;
+                to = data_sigma + 2 * ((j + 3 * i) * N + r0);
+                for (size_t q = 0; q < n; ++q) {
+                    to[2 * q] = v[q] + P.sigmu[3 * j + i];
+                    to[2 * q + 1] = 0.0;
+                }
+            });
+        }));
+    HIPCHK(hipStreamSynchronize(st));
     return PFDD_OK;
 }
 
@@ -1475,8 +1537,11 @@ int self_graph_capture(pfdd_gl *h, double tol, int par)
     h->cur = par;
     HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     int rc = PFDD_OK;
-    for (int it = 0; it < SG_ITERS && !rc; ++it)
-        rc = step_any(h, tol, it == 0, it == SG_ITERS - 1);
+    {
+        const GraphTau in_device_memory(h);
+        for (int it = 0; it < SG_ITERS && !rc; ++it)
+            rc = step_any(h, tol, it == 0, it == SG_ITERS - 1);
+    }
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(h->stream, &graph);
     h->cur = cur0;
@@ -1669,8 +1734,8 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
     }
     h->nb3 = h->M * (h->prec == PFDD_FP64 ? mid_blocks<double>(h->nx, h->S, (long long)h->ny * h->nz)
                                           : mid_blocks<float>(h->nx, h->S, (long long)h->ny * h->nz));
+    if ((rc = alloc((void **)&h->taud, sizeof(double) * h->SM))) return bail(rc);
     if (h->M > 1) {
-        if ((rc = alloc((void **)&h->taud, sizeof(double) * h->SM))) return bail(rc);
         e = hipMemsetAsync(h->taud, 0, sizeof(double) * h->SM, h->stream);
         if (e != hipSuccess) return bail(fail(PFDD_ERR_HIP, "hipMemset: %s", hipGetErrorString(e)));
         h->P.taud = h->taud;
@@ -1918,7 +1983,7 @@ int pfdd_gl_set_tau(pfdd_gl *h, const double *tau)
         return PFDD_OK;
     }
     for (int a = 0; a < h->S; ++a) h->P.tau[a] = tau[a];
-    ++h->version;
+    h->tau_stale = true;
     return PFDD_OK;
 }
 
@@ -1949,7 +2014,7 @@ int pfdd_gl_step(pfdd_gl *h, int nsteps, double tol, pfdd_gl_reduce *out)
     }
     h->fresh = false;
     if (h->sg_on && nsteps >= 2 * SG_ITERS && cs == hipStreamCaptureStatusNone) {
-        if ((rc = self_graph_ready(h, tol))) return rc;
+        if ((rc = self_graph_ready(h, tol)) || (rc = graph_tau(h, h->stream))) return rc;
         // SG_ITERS is even: every replay leaves the parity where it was
         for (int r = 0; r < nsteps / SG_ITERS; ++r) HIPCHK(hipGraphLaunch(h->sg[h->cur].exec, h->stream));
         h->stepped = true;
@@ -2020,20 +2085,19 @@ int pfdd_gl_xi_sums(pfdd_gl *h, double *sum_re)
     int rc;
     if ((rc = check_handle(h)) || (rc = set_device(h))) return rc;
     if (!sum_re) return fail(PFDD_ERR_ARG, "null output");
+    // the block sums go to the host's memory, in stream order after the run
     const int nb = XS_NB;
-    double *part = nullptr;
-    HIPCHK(hipMalloc(&part, sizeof(double) * nb * h->SM));
+    if (!h->xs_part)
+        HIPCHK(hipHostMalloc((void **)&h->xs_part, sizeof(double) * nb * h->SM, hipHostMallocDefault));
+    const double *hp = h->xs_part;
     if (h->prec == PFDD_FP64)
         hipLaunchKernelGGL((k_sys_sums<double>), dim3(nb, h->SM), dim3(NTHR), 0, h->stream,
-                           (const double2 *)h->xi[h->cur], h->N, part);
+                           (const double2 *)h->xi[h->cur], h->N, h->xs_part);
     else
         hipLaunchKernelGGL((k_sys_sums<float>), dim3(nb, h->SM), dim3(NTHR), 0, h->stream,
-                           (const float2 *)h->xi[h->cur], h->N, part);
+                           (const float2 *)h->xi[h->cur], h->N, h->xs_part);
     HIPCHK(hipGetLastError());
-    std::vector<double> hp((size_t)nb * h->SM);
-    HIPCHK(hipMemcpyAsync(hp.data(), part, sizeof(double) * nb * h->SM, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(hipFree(part));
     for (int a = 0; a < h->SM; ++a) {
         double s = 0.0, c = 0.0;
         for (int b = 0; b < nb; ++b) {
@@ -2185,10 +2249,10 @@ int pfdd_gl_traffic(pfdd_gl *h, double *bytes_per_kernel, double *bytes_per_step
 // ================================================================== graphs
 // A hipGraph holding `iters` (even) GL iterations of several handles, replayed
 // as one launch.  Kernel arguments are frozen at capture: the graph is
-// captured again when a handle's kernel arguments changed (set_tau of a
-// single-run handle, set_core_coef), when its current ping-pong buffer is not
-// the one captured, or when tol changes.  A batch handle reads tau from
-// device memory, so set_tau needs no new capture.
+// captured again when a handle's kernel arguments changed (set_core_coef),
+// when its current ping-pong buffer is not the one captured, or when tol
+// changes.  The captured kernels read tau from device memory, so set_tau needs
+// no new capture.
 struct pfdd_gl_graph {
     std::vector<pfdd_gl *> hs;
     hipStream_t stream = nullptr;
@@ -2233,6 +2297,7 @@ int graph_capture(pfdd_gl_graph *g, double tol)
         e = hipEventRecord(g->join[n], g->stream); // fork
         for (size_t i = 0; i < n && !rc && e == hipSuccess; ++i) {
             pfdd_gl *h = g->hs[i];
+            const GraphTau in_device_memory(h);
             e = hipStreamWaitEvent(h->stream, g->join[n], 0);
             for (int it = 0; it < g->iters && !rc && e == hipSuccess; ++it)
                 rc = step_any(h, tol, it == 0, it == g->iters - 1);
@@ -2310,6 +2375,7 @@ int pfdd_gl_graph_run(pfdd_gl_graph *g, int nsteps, double tol, pfdd_gl_reduce *
         cur0[i] = h->cur;
         reset_run(h, g->stream);
         HIPCHK(hipGetLastError());
+        if ((rc = graph_tau(h, g->stream))) return rc;
     }
     for (int r = 0; r < nsteps / g->iters; ++r) HIPCHK(hipGraphLaunch(g->exec, g->stream));
     // the remainder eagerly, on the graph stream
@@ -2372,6 +2438,7 @@ struct pfdd_gl_cond {
     std::vector<double> sig_h;
     long long nb = 0;         // most partials of a kernel
     CondStat *stat = nullptr; // pinned host memory
+    Stage stage;
 };
 
 namespace {
@@ -2382,6 +2449,7 @@ void cond_release(pfdd_gl_cond *h)
                     (void *)h->done, h->tw[0], h->tw[1], h->tw[2]})
         if (p) hipFree(p);
     if (h->stat) (void)hipHostFree(h->stat);
+    h->stage.release();
     if (h->own_stream && h->stream) hipStreamDestroy(h->stream);
 }
 
@@ -2525,9 +2593,7 @@ int pfdd_gl_cond_get(pfdd_gl_cond *h, double *c_host)
 {
     if (!h || !c_host) return fail(PFDD_ERR_ARG, "null argument");
     HIPCHK(hipSetDevice(h->device));
-    HIPCHK(hipMemcpyAsync(c_host, h->c, sizeof(double2) * h->N, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    return PFDD_OK;
+    return copy_out(h->stage, h->c, c_host, sizeof(double2) * h->N, h->stream);
 }
 
 int pfdd_gl_cond_step(pfdd_gl_cond *h, int nsteps, pfdd_gl_cond_reduce *out)

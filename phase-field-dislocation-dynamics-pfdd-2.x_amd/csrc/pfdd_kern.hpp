@@ -36,7 +36,7 @@ extern thread_local hipEvent_t t_ev_start, t_ev_stop;
 
 struct StepParams {
     double tau[MAXS];          // resolved shear per system (single-run handles)
-    const double *taud;        // device tau per system of a batch (nullptr: use tau[])
+    const double *taud;        // device tau per system, of a batch or a captured graph (nullptr: use tau[])
     double coef[MAXS * MAXM];  // core coefficients per system of one member
     double a0;                 // constant term of the Fourier core models
     double cddt;
