@@ -199,6 +199,15 @@ __device__ __forceinline__ void core_extended_adj(const R x[3], const R mu[3], i
     hv = (R)h;
 }
 
+// Re xi of the other two systems of a plane, in cyclic order, at a cell of its
+// system j (x).
+template <typename R, typename V>
+__device__ __forceinline__ void other_systems(const V *__restrict__ x, int j, long long ncell, R *others)
+{
+    others[0] = x[j == 2 ? -2 * ncell : ncell].x;
+    others[1] = x[j == 0 ? 2 * ncell : -ncell].x;
+}
+
 // One cell of update_order_parameter (fft_fftw_slab.cpp:1746-1790): the
 // core-energy derivative of core_energy_* at Re xi of the old field x (the
 // reference evaluates it on data_fftw = xi before the update), the applied
@@ -210,7 +219,7 @@ __device__ __forceinline__ void core_extended_adj(const R x[3], const R mu[3], i
 // Returns the new value; dn is the cell's |xi_new - xi_old|^2 term of xinorm
 // and dens its core-energy density.
 template <typename R, bool GEN, typename V, typename Coef>
-__device__ __forceinline__ V gl_update_cell(const V g, const V x, long long idx, R tau, int sub, Coef coef,
+__device__ __forceinline__ V gl_update_cell(const V g, const V x, const R *others, long long idx, R tau, Coef coef,
                                             const StepParams &P, int nm, R cddt, R invN,
                                             const uint8_t *__restrict__ mask, const long long *__restrict__ prev,
                                             const V *__restrict__ xo, const R *__restrict__ amp, double &dn, R &dens)
@@ -218,17 +227,11 @@ __device__ __forceinline__ V gl_update_cell(const V g, const V x, long long idx,
     R dE = (R)0;
     dens = (R)0;
     if (GEN && P.model == PFDD_CORE_EXTENDED) {
-        // the other two systems of the plane at the same cell
-        const int j = sub;
-        const long long b0 = idx - (long long)j * P.ncell;
-        R y[3];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) y[q] = q == j ? x.x : xo[b0 + q * P.ncell].x;
         R cc[7];
 #pragma unroll
         for (int q = 0; q < 7; ++q) cc[q] = coef(q);
         R f;
-        core_extended<R>(y[j], y[(j + 1) % 3], y[(j + 2) % 3], cc, f, dE);
+        core_extended<R>(x.x, others[0], others[1], cc, f, dE);
         dens = f / (R)3; // each of the three systems carries a third of the plane's density
     } else {
         R sp, cp;

@@ -176,7 +176,9 @@ __global__ void __launch_bounds__((plane_threads<R, NY, NZ>()))
             const V x = ld_stream(&xo[idx]);
             R dens;
             double dn;
-            const V y = gl_update_cell<R, GEN>(g, x, idx, tau, as % 3, [&](int m) { return lcf[m]; }, P, nm,
+            R others[2] = {};
+            if (GEN && P.model == PFDD_CORE_EXTENDED) other_systems<R>(xo + idx, as % 3, P.ncell, others);
+            const V y = gl_update_cell<R, GEN>(g, x, others, idx, tau, [&](int m) { return lcf[m]; }, P, nm,
                                                cddt, invN, mask, prev, xo, amp, dn, dens);
             st_stream(&xn[idx], y);
             if constexpr (FW) lds.st(at, y); // this thread's own cell, read above

@@ -47,7 +47,19 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(updat
     __shared__ int lsub[NL]; // position of the line's system in its plane triple (coupled model)
     __shared__ double red[4 * (NTHR / 64)];
     const int tid = threadIdx.x;
-    const long long L0 = (long long)blockIdx.x * NL;
+    const bool ext = GEN && P.model == PFDD_CORE_EXTENDED;
+    unsigned tile = blockIdx.x;
+    if constexpr (GEN) {
+        // The coupled model reads Re xi of all three systems of a plane: the
+        // same lines of the three are 8 blocks apart, that is on the same XCD
+        // and close in time, so two of the three reads find them in its L2.
+        const unsigned per = (unsigned)(lines_per_sys / NL); // tiles of a system
+        if (ext && per % 8 == 0 && per * (unsigned)NL == lines_per_sys) {
+            const unsigned plane = tile / (3 * per), r = tile - plane * 3 * per, w = r % 24;
+            tile = (plane * 3 + w / 8) * per + r / 24 * 8 + w % 8;
+        }
+    }
+    const long long L0 = (long long)tile * NL;
     for (int l = tid; l < NL; l += NTHR) {
         const long long L = L0 + l;
         const bool ok = L < nlines;
@@ -67,24 +79,27 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(updat
     constexpr int PER = (TOT + NTHR - 1) / NTHR;
     constexpr bool PREF = sizeof(V) < 16;
     V xold[PER];
-    if constexpr (PREF) {
+    R others[GEN ? 2 * PER : 2] = {}; // coupled model: of the other two systems
+    auto load_old = [&] {
 #pragma unroll
         for (int t = 0; t < PER; ++t) {
             const int e = tid + t * NTHR;
             const long long b = (TOT % NTHR == 0 || e < TOT) ? bout[e / N] : -1;
-            xold[t] = b >= 0 ? ld_stream(&xo[b + e % N]) : mk<V>((R)0, (R)0);
+            const V *const at = xo + (b >= 0 ? b + e % N : 0);
+            xold[t] = GEN ? *at : ld_stream(at); // plain: the other systems' blocks read it, too
+            if constexpr (GEN) {
+                if (ext) {
+                    const int j = e < TOT ? lsub[e / N] : 0;
+                    others[2 * t] = at[j == 2 ? -2 * P.ncell : P.ncell].x;
+                    others[2 * t + 1] = at[j == 0 ? 2 * P.ncell : -P.ncell].x;
+                }
+            }
         }
-    }
+    };
+    if constexpr (PREF) load_old();
     __syncthreads();
     fft_stages<N, 1, NL, NTHR, true>(lds, tw, tid);
-    if constexpr (!PREF) {
-#pragma unroll
-        for (int t = 0; t < PER; ++t) {
-            const int e = tid + t * NTHR;
-            const long long b = (TOT % NTHR == 0 || e < TOT) ? bout[e / N] : -1;
-            xold[t] = b >= 0 ? ld_stream(&xo[b + e % N]) : mk<V>((R)0, (R)0);
-        }
-    }
+    if constexpr (!PREF) load_old();
 
     const R cddt = (R)P.cddt, invN = (R)P.invN;
     const int nm = P.ncoef;
@@ -105,7 +120,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(updat
         const R tau = ltau[l];
         R dens;
         double dn;
-        const V y = gl_update_cell<R, GEN>(g, x, idx, tau, lsub[l], [&](int m) { return lcoef[m * NL + l]; }, P, nm,
+        const V y = gl_update_cell<R, GEN>(g, x, others + (GEN ? 2 * t : 0), idx, tau, [&](int m) { return lcoef[m * NL + l]; }, P, nm,
                                            cddt, invN, mask, prev, xo, amp, dn, dens);
         st_stream(&xn[idx], y);
         if constexpr (FW != 0) lds.st(p * LDP + l, y); // this thread's own cell, read above
