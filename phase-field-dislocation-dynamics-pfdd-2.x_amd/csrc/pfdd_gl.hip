@@ -521,6 +521,7 @@ struct pfdd_gl {
     int cur = 0;
     void *T1 = nullptr;
     void *B = nullptr;
+    void *cst = nullptr;    // constants of the x pass (GParams)
     void *tw[3] = {nullptr, nullptr, nullptr}; // x, y, z twiddle tables
     uint8_t *mask = nullptr;
     long long *prev = nullptr;
@@ -1122,7 +1123,7 @@ void destroy_all(pfdd_gl *h)
     hipSetDevice(h->device);
     if (h->stream) hipStreamSynchronize(h->stream);
     self_graph_release(h);
-    void *ptrs[] = {h->cof, h->taud, h->xi[0], h->xi[1], h->T1, h->B, h->tw[0], h->tw[1], h->tw[2], h->mask, h->prev,
+    void *ptrs[] = {h->cof, h->taud, h->xi[0], h->xi[1], h->T1, h->B, h->cst, h->tw[0], h->tw[1], h->tw[2], h->mask, h->prev,
                     h->amp, h->none, h->partial, h->done, h->steps, h->stage2, h->ticket, h->dw[0], h->dw[1],
                     h->deps, h->dsig, h->tape.lam[0], h->tape.lam[1], h->tape.gpart, h->tape.gacc};
     for (void *p : ptrs)
@@ -1233,14 +1234,13 @@ int build_B(pfdd_gl *h)
         for (int c = 0; c < 6; ++c) {
             const int q = si[c], r = q / 3, cc = q % 3;
             G.sig6[a * 6 + c] = bp.sig[a * 9 + q];
-            G.eps6[a * 6 + c] = c < 3 ? bp.eps[a * 9 + q] : bp.eps[a * 9 + 3 * r + cc] + bp.eps[a * 9 + 3 * cc + r];
+            G.eps6[a * 6 + c] =
+                c < 3 ? bp.eps[a * 9 + q] : bp.eps[a * 9 + 3 * r + cc] + bp.eps[a * 9 + 3 * cc + r];
         }
     for (int q = 0; q < 9; ++q) G.four[q] = h->four[q];
-    G.C44x2 = 2.0 * h->C44;
-    G.C12 = h->C12;
-    G.inv2C44 = bp.inv2C44;
-    G.inv1mnu = bp.inv1mnu;
     G.invmu = bp.invmu;
+    G.c4f = 0.5 * bp.inv1mnu;
+    G.c5 = h->C12 * bp.inv2C44;
     G.keep = order_of((size_t)h->SM * h->N * h->esz, (int)h->esz).keep;
     G.nx = h->nx;
     G.ny = h->ny;
@@ -1248,6 +1248,16 @@ int build_B(pfdd_gl *h)
     G.inv_n[0] = 1.0 / h->nx;
     G.inv_n[1] = 1.0 / h->ny;
     G.inv_n[2] = 1.0 / h->nz;
+    {
+        R cst[MAXS * 12];
+        for (int q = 0; q < S * 6; ++q) {
+            cst[q] = (R)G.sig6[q];
+            cst[S * 6 + q] = (R)(G.eps6[q] * (sizeof(R) == 8 ? G.invmu : 1.0));
+        }
+        HIPCHK(hipMalloc(&h->cst, sizeof(R) * S * 12));
+        HIPCHK(hipMemcpy(h->cst, cst, sizeof(R) * S * 12, hipMemcpyHostToDevice));
+        G.cst = h->cst;
+    }
     if (!h->stored_B) return PFDD_OK;
     const long long np = (long long)S * (S + 1) / 2;
     HIPCHK(hipMalloc(&h->B, (size_t)np * h->N * sizeof(R)));

@@ -348,11 +348,12 @@ struct GParams {
     double sig6[MAXS * 6];
     double eps6[MAXS * 6];
     double four[9];
-    double inv2C44, inv1mnu, invmu;
-    double C44x2, C12; // isotropic stiffness: C:Q = 2 C44 Q + C12 tr(Q) I
+    double c4f, c5;    // c4 f^4 and c5 of the contraction
+    double invmu;
     double inv_n[3];   // 1/nx, 1/ny, 1/nz (frequencies by multiplication in the x pass)
     int nx, ny, nz;
     bool keep;         // store the field for the next kernel to find in the last-level cache (Order)
+    const void *cst;   // [S][6] sig6, [S][6] eps6 (FP64: over mu) in the precision of the x pass, device memory
 };
 
 __device__ __forceinline__ double frac_freq(int kk, int n)

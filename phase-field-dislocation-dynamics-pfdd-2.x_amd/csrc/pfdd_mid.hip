@@ -144,8 +144,12 @@ __global__ void __launch_bounds__(NTHR)
 //   w = Sig f,  V = f.w
 //   Q = [2 sym(w f)/f^2 - V f f/((1-nu) f^4)] / (2 C44)
 //   P = Sig - C:Q = Sig - 2 C44 Q - C12 tr(Q) I
+//     = Sig - D - c5 tr(D) I,  D = u f + f u,  u = c2 w - c4 V f,
+//       c2 = 1/f^2, c4 = 1/(2 (1-nu) f^4), c5 = C12 / (2 C44)
 //   ghat_a = eps_a : P / mu
-// (sigma_a:Q = eps_a:(C:Q) for the isotropic C), and ghat = 0 at f = 0
+// (80 instead of 110 instructions a point for P from Sig; FP32 error of P over
+// the k-points of planar fields on 48 to 160 points, rms: 2.1e-7 to 3.9e-7 ->
+// 1.8e-7 to 2.7e-7.  sigma_a:Q = eps_a:(C:Q) for the isotropic C), and ghat = 0 at f = 0
 // (B(0) = 0).  TPP threads share one k-point (wave-uniform split of the
 // systems), each producing S/TPP of the outputs.
 template <typename R, int N, int S> constexpr int otf_tpp()
@@ -154,39 +158,46 @@ template <typename R, int N, int S> constexpr int otf_tpp()
     return (2 * pts == NTHR && S % 2 == 0) ? 2 : 1;
 }
 
-// Scalars of the contraction in the arithmetic type T of the x pass.
-template <typename T> struct GConst {
-    T inv2C44, inv1mnu, invmu, C44x2, C12;
+// A k-point: f and the scalars of P and ghat (above) in the arithmetic type T of
+// the x pass; nz: f != 0.  In FP64 the constants eps_a hold 1/mu.  In FP32 it is
+// a factor of ghat: the components of eps_a are mostly exact, those of eps_a /
+// mu are not, and the energy's error at 128^3 x 12 grew from 2e-11 to 1.5e-7.
+template <typename T> struct KPoint {
+    T f[3], c2, c4, c5, invmu;
+    bool nz;
 };
 
-// Sig -> P = Sig - 2 C44 Q - C12 tr(Q) I at one k-point (real and imaginary
-// part; symmetric components xx, yy, zz, xy, xz, yz).  The order of every sum
-// of products is written out (ab_cd), so that all x-pass variants round alike.
-template <typename T>
-__device__ __forceinline__ void otf_green(T Pr[6], T Pi[6], const T f[3], T c2, T c4, const GConst<T> &G)
+// Sig -> P at one k-point (real and imaginary part; symmetric components xx,
+// yy, zz, xy, xz, yz).  The order of every sum of products is written out, so
+// that all x-pass variants round alike.
+template <typename T> __device__ __forceinline__ void otf_green(T Pr[6], T Pi[6], const KPoint<T> &K)
 {
-    auto dot3 = [](T a0, T a1, T a2, const T *b) { return ab_cd(a2, b[2], (T)1, ab_cd(a1, b[1], a0, b[0])); };
-    const T wr[3] = {dot3(Pr[0], Pr[3], Pr[4], f), dot3(Pr[3], Pr[1], Pr[5], f), dot3(Pr[4], Pr[5], Pr[2], f)};
-    const T wi[3] = {dot3(Pi[0], Pi[3], Pi[4], f), dot3(Pi[3], Pi[1], Pi[5], f), dot3(Pi[4], Pi[5], Pi[2], f)};
-    const T Vr = dot3(wr[0], wr[1], wr[2], f), Vi = dot3(wi[0], wi[1], wi[2], f);
-    // c2 multiplies (w_i f_j + w_j f_i), c4 multiplies V f_i f_j
-    const int ci[6] = {0, 1, 2, 0, 0, 1}, cj[6] = {0, 1, 2, 1, 2, 2};
-    const T vr = c4 * Vr, vi = c4 * Vi;
-    T Qr[6], Qi[6];
+    const T *const f = K.f;
+    auto half = [&](T *p) { // one of the two parts
+        auto dot3 = [](T a0, T a1, T a2, const T *b) { return ab_c(a2, b[2], ab_cd(a1, b[1], a0, b[0])); };
+        const T w[3] = {dot3(p[0], p[3], p[4], f), dot3(p[3], p[1], p[5], f), dot3(p[4], p[5], p[2], f)};
+        const T V = dot3(w[0], w[1], w[2], f), v = K.c4 * V;
+        T u[3], d[3];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        const T ff = f[ci[c]] * f[cj[c]];
-        const T sr = ab_cd(wr[ci[c]], f[cj[c]], wr[cj[c]], f[ci[c]]);
-        const T si = ab_cd(wi[ci[c]], f[cj[c]], wi[cj[c]], f[ci[c]]);
-        Qr[c] = ab_cd(c2, sr, -vr, ff);
-        Qi[c] = ab_cd(c2, si, -vi, ff);
-    }
-    const T tr_r = G.C12 * (Qr[0] + Qr[1] + Qr[2]), tr_i = G.C12 * (Qi[0] + Qi[1] + Qi[2]);
+        for (int i = 0; i < 3; ++i) u[i] = ab_cd(K.c2, w[i], -v, f[i]);
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        Pr[c] -= ab_cd(G.C44x2, Qr[c], (T)1, c < 3 ? tr_r : (T)0);
-        Pi[c] -= ab_cd(G.C44x2, Qi[c], (T)1, c < 3 ? tr_i : (T)0);
-    }
+        for (int i = 0; i < 3; ++i) d[i] = u[i] * ((T)2 * f[i]);
+        const T tr = K.c5 * (d[0] + d[1] + d[2]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) p[i] -= d[i] + tr;
+        const int ci[3] = {0, 0, 1}, cj[3] = {1, 2, 2};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) p[3 + c] = ab_c(-u[ci[c]], f[cj[c]], ab_c(-u[cj[c]], f[ci[c]], p[3 + c]));
+    };
+    half(Pr);
+    half(Pi);
+}
+
+// P at f = 0, where B vanishes.
+template <typename T> __device__ __forceinline__ void otf_zero(T Pr[6], T Pi[6])
+{
+#pragma unroll
+    for (int c = 0; c < 6; ++c) Pr[c] = Pi[c] = (T)0;
 }
 
 // Hands ghat_a for a = H*SA .. H*SA+SA-1 of one k-point to sink(aa, re, im,
@@ -195,13 +206,13 @@ __device__ __forceinline__ void otf_green(T Pr[6], T Pi[6], const T f[3], T c2, 
 // the sink does not read the tile again (FP64 x pass at 128^3 x 12: 189 ->
 // 186 us).
 template <typename T, int S, int SA, int H, int NP, typename XA, typename V, typename Sink>
-__device__ __forceinline__ void otf_point(const Tile<V> lds, int p, int q, const T f[3], bool nzf, T c2, T c4,
-                                          const T *__restrict__ cst, const GConst<T> &G, Sink sink)
+__device__ __forceinline__ void otf_point(const Tile<V> lds, int p, int q, const KPoint<T> &K,
+                                          const T *__restrict__ cst, Sink sink)
 {
     // compiler-only barriers keep the (LDS-broadcast) constants from being
     // hoisted and held in registers across points and systems
     __asm__ volatile("" ::: "memory");
-    T Pr[6] = {}, Pi[6] = {}; // Sig, then P
+    T Pr[6], Pi[6]; // Sig, then P
     V xk[SA];
 #pragma unroll
     for (int b = 0; b < S; ++b) {
@@ -210,38 +221,44 @@ __device__ __forceinline__ void otf_point(const Tile<V> lds, int p, int q, const
         const T xr = (T)v.x, xi = (T)v.y;
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
-            Pr[c] += cst[b * 12 + c] * xr;
-            Pi[c] += cst[b * 12 + c] * xi;
+            Pr[c] = b ? ab_c(cst[b * 12 + c], xr, Pr[c]) : cst[c] * xr;
+            Pi[c] = b ? ab_c(cst[b * 12 + c], xi, Pi[c]) : cst[c] * xi;
         }
     }
-    if (nzf) otf_green(Pr, Pi, f, c2, c4, G);
+    if (K.nz) otf_green(Pr, Pi, K);
+    else otf_zero(Pr, Pi);
 #pragma unroll
     for (int aa = 0; aa < SA; ++aa) {
         __asm__ volatile("" ::: "memory");
         const int a = H * SA + aa;
         const T *ep = cst + a * 12 + 6;
-        T gr = 0, gi = 0;
+        T gr = Pr[0] * ep[0], gi = Pi[0] * ep[0];
 #pragma unroll
-        for (int c = 0; c < 6; ++c) {
-            gr += Pr[c] * ep[c];
-            gi += Pi[c] * ep[c];
+        for (int c = 1; c < 6; ++c) {
+            gr = ab_c(Pr[c], ep[c], gr);
+            gi = ab_c(Pi[c], ep[c], gi);
         }
-        gr *= G.invmu;
-        gi *= G.invmu;
-        if (!nzf) gr = gi = (T)0;
+        if constexpr (sizeof(T) == 4) {
+            gr *= K.invmu;
+            gi *= K.invmu;
+        }
         sink(aa, gr, gi, xk[aa]);
     }
 }
 
-// f = four^T k~ of k-point (p, col) (frec, fft_fftw_slab.cpp:280-367) and the
-// scalars of the Green's function G = (2 I/f^2 - f f/((1-nu) f^4))/(2 C44)
-// (Bmatrix, :577-634), c2 = 1/(2 C44 f^2) and c4 = 1/((1-nu) 2 C44 f^4), all
-// formed in FP64 and rounded once to T: in the FP32 mode B(k) is built in
-// FP64 and only the contraction with xihat runs in FP32.  nzf: f != 0 (B(0)
-// = 0).  Column col is (k, j) = (col / ny, col % ny) in the line layout of the
-// five-kernel iteration and (j, k) = (col / nz, col % nz) in the plane layout.
-template <int N, int NP, int S, typename T, bool PL = false>
-__device__ __forceinline__ void otf_freq(const GParams &G, long long col, int p, T f[3], bool &nzf, T &c2, T &c4)
+// f = four^T k~ (frec, fft_fftw_slab.cpp:280-367) in two parts: that of a
+// column, (k, j) = (col / ny, col % ny) in the line layout of the five-kernel
+// iteration and (j, k) = (col / nz, col % nz) in the plane layout, and that of
+// position p.  All is formed in FP64 and rounded once to T: in the FP32 mode
+// B(k) is built in FP64 and only the contraction with xihat runs in FP32.
+// frec's k/n with the reciprocal of n (one rounding more than the division for
+// sizes that are not powers of two): the x pass evaluates it for every k-point
+// of every step.
+__device__ __forceinline__ double otf_frac(int kk, int n, double inv)
+{
+    return (double)(kk >= n / 2 ? kk - n : kk) * inv;
+}
+template <bool PL = false> __device__ __forceinline__ void otf_col(const GParams &G, long long col, double *fc)
 {
     const int c = (int)col; // column of one member: ny * nz < 2^31
     int j, k;
@@ -252,39 +269,34 @@ __device__ __forceinline__ void otf_freq(const GParams &G, long long col, int p,
         k = c / G.ny;
         j = c - k * G.ny;
     }
-    // frec's k/n with the reciprocal of n (one rounding more than the
-    // division for sizes that are not powers of two): the x pass evaluates it
-    // for every k-point of every step
-    auto fr = [](int kk, int n, double inv) { return (double)(kk >= n / 2 ? kk - n : kk) * inv; };
-    const double kx = fr(p, G.nx, G.inv_n[0]), ky = fr(j, G.ny, G.inv_n[1]), kz = fr(k, G.nz, G.inv_n[2]);
-    double fd[3];
+    const double ky = otf_frac(j, G.ny, G.inv_n[1]), kz = otf_frac(k, G.nz, G.inv_n[2]);
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
-        fd[c] = ab_cd(kz, G.four[6 + c], 1.0, ab_cd(ky, G.four[3 + c], kx, G.four[c]));
+    for (int c = 0; c < 3; ++c) fc[c] = ab_cd(kz, G.four[6 + c], ky, G.four[3 + c]);
+}
+template <typename T> __device__ __forceinline__ KPoint<T> otf_freq(const GParams &G, const double *fc, int p)
+{
+    // f rounded first, f^2 from what it was rounded to: c2 f f is then a
+    // projector to one rounding, and P of f parallel to the slip plane's normal,
+    // where it vanishes, keeps less of Sig
+    const double kx = otf_frac(p, G.nx, G.inv_n[0]);
+    double f[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) f[c] = (T)fd[c];
-    const double f2 = ab_cd(fd[2], fd[2], 1.0, ab_cd(fd[1], fd[1], fd[0], fd[0]));
-    nzf = f2 > 0;
-    const double if2 = nzf ? 1.0 / f2 : 0.0;
-    c2 = (T)(if2 * G.inv2C44);
-    c4 = (T)(G.inv1mnu * if2 * if2 * G.inv2C44);
+    for (int c = 0; c < 3; ++c) f[c] = (double)(T)ab_c(kx, G.four[c], fc[c]);
+    const double f2 = ab_c(f[2], f[2], ab_cd(f[1], f[1], f[0], f[0]));
+    const double if2 = 1.0 / f2;
+    return KPoint<T>{{(T)f[0], (T)f[1], (T)f[2]}, (T)if2, (T)(G.c4f * if2 * if2), (T)G.c5, (T)G.invmu, f2 > 0};
 }
 
 // Minimum waves per SIMD asked of the x pass (one wave per SIMD per resident
-// block of 256 threads).  The 12-system FP64 cases ask for 5, set when their
-// tiles were one column wide; with two-column tiles their LDS allows 3 blocks
-// per CU, which the compiler then reaches (measured, and kept: the register
-// allocation the hint produces is the one timed).  The 3-system passes ask
-// for 3 in FP64 (168 instead of 172-190 VGPRs, a few spilled; their tiles
-// allow 3-8 blocks): 3-system batches at 48^3 and 64^3 ran their x pass
-// 80 -> 67 and 193 -> 179 us, and 512-point lines (unpadded tile, 49 KB)
-// 2.25 -> 1.81 ms.  In FP32 only the 512-point lines ask for 5 (1.17 -> 1.11
-// ms); at 48-96 points 5 or 6 waves (96 or 80 VGPRs, with spills) were
-// slower than the compiler's 4.  Other system counts are not constrained.
+// block of 256 threads).  The 12- and 3-system FP64 passes ask for 3, 168
+// VGPRs instead of 172-190 (96 points x 12 at 96 x 80 x 48: 55.5 -> 48.5 us;
+// 3-system batches at 48^3: 80 -> 67 us).  Other system counts and FP32 are not
+// constrained: at 48-96 points 5 or 6 waves (96 or 80 VGPRs, with spills) were
+// slower than the compiler's 4.
 template <typename R, int N, int S> constexpr int otf_waves()
 {
-    if (S == 12 && sizeof(R) == 8 && N >= 32 && N <= 128) return 5;
-    if (S == 3) return sizeof(R) == 8 ? 3 : (N >= 512 ? 5 : 1);
+    if (S == 12 && sizeof(R) == 8) return 3;
+    if (S == 3 && sizeof(R) == 8) return 3;
     return 1;
 }
 
@@ -294,7 +306,7 @@ template <typename R, int N, int S> constexpr int otf_waves()
 template <typename R, int N, int S, bool PL = false>
 __device__ __forceinline__ double otf_tile(const Tile<typename cvec<R>::type> lds,
                                            const typename cvec<R>::type *__restrict__ tw, const GParams &G,
-                                           const GConst<R> &gc, const R *cst, long long c0, long long ncol, int tid)
+                                           const R *cst, long long c0, long long ncol, int tid)
 {
     typedef typename cvec<R>::type V;
     typedef R T;
@@ -314,10 +326,10 @@ __device__ __forceinline__ double otf_tile(const Tile<typename cvec<R>::type> ld
         for (int pt = tid; pt < NPT; pt += NTHR) {
             const int q = pt / N, p = pt % N;
             if (c0 + q >= ncol) continue;
-            T f[3], c2, c4;
-            bool nzf;
-            otf_freq<N, NP, S, T, PL>(G, c0 + q, p, f, nzf, c2, c4);
-            otf_point<T, S, SA, 0, NP, XA>(lds, p, q, f, nzf, c2, c4, cst, gc, [&](int a, T gr, T gi, V x) {
+            double fc[3];
+            otf_col<PL>(G, c0 + q, fc);
+            const KPoint<T> K = otf_freq<T>(G, fc, p);
+            otf_point<T, S, SA, 0, NP, XA>(lds, p, q, K, cst, [&](int a, T gr, T gi, V x) {
                 const int idx = XA::at(p, a * NP + q);
                 el += (double)x.x * gr + (double)x.y * gi;
                 lds.st(idx, mk<V>((R)gr, (R)gi));
@@ -329,9 +341,9 @@ __device__ __forceinline__ double otf_tile(const Tile<typename cvec<R>::type> ld
         const int h = tid / NPT, pt = tid % NPT;
         const int q = pt / N, p = pt % N;
         const bool ok = c0 + q < ncol;
-        T f[3], c2, c4;
-        bool nzf;
-        otf_freq<N, NP, S, T, PL>(G, c0 + q, p, f, nzf, c2, c4);
+        double fc[3];
+        otf_col<PL>(G, c0 + q, fc);
+        const KPoint<T> K = otf_freq<T>(G, fc, p);
         T g[SA][2];
         auto keep = [&](int aa, T gr, T gi, V) {
             g[aa][0] = gr;
@@ -339,9 +351,9 @@ __device__ __forceinline__ double otf_tile(const Tile<typename cvec<R>::type> ld
         };
         if (ok) {
             if (__builtin_amdgcn_readfirstlane(h) == 0)
-                otf_point<T, S, SA, 0, NP, XA>(lds, p, q, f, nzf, c2, c4, cst, gc, keep);
+                otf_point<T, S, SA, 0, NP, XA>(lds, p, q, K, cst, keep);
             else
-                otf_point<T, S, SA, 1, NP, XA>(lds, p, q, f, nzf, c2, c4, cst, gc, keep);
+                otf_point<T, S, SA, 1, NP, XA>(lds, p, q, K, cst, keep);
         }
         __syncthreads();
         if (ok) {
@@ -360,11 +372,11 @@ __device__ __forceinline__ double otf_tile(const Tile<typename cvec<R>::type> ld
 }
 
 template <typename R, int S>
-__device__ __forceinline__ void otf_consts(R *cst, GConst<R> &gc, const GParams &G, int tid)
+__device__ __forceinline__ void otf_consts(R *cst, const GParams &G, int tid)
 {
     for (int c = tid; c < S * 12; c += NTHR) cst[c] = (R)((c % 12) < 6 ? G.sig6[(c / 12) * 6 + c % 12]
-                                                                       : G.eps6[(c / 12) * 6 + c % 12 - 6]);
-    gc = GConst<R>{(R)G.inv2C44, (R)G.inv1mnu, (R)G.invmu, (R)G.C44x2, (R)G.C12};
+                                                                       : G.eps6[(c / 12) * 6 + c % 12 - 6] *
+                                                                             (sizeof(R) == 8 ? G.invmu : 1.0));
 }
 
 // x pass, one tile per block.
@@ -387,11 +399,10 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(otf_w
     const int mem = blockIdx.x / bpm;
     const long long c0 = (long long)(blockIdx.x - mem * bpm) * NP;
     T2 += (long long)mem * S * ntot;
-    GConst<R> gc;
-    otf_consts<R, S>(cst, gc, G, tid);
+    otf_consts<R, S>(cst, G, tid);
     tile_load_cols<N, NL, NP, NTHR, XA>(lds, T2, c0, ncol, ntot, tid);
     __syncthreads();
-    double v[1] = {otf_tile<R, N, S>(lds, tw, G, gc, cst, c0, ncol, tid)};
+    double v[1] = {otf_tile<R, N, S>(lds, tw, G, cst, c0, ncol, tid)};
 #pragma unroll 4
     for (int e = tid; e < TOT; e += NTHR) {
         const int l = e / N, p = e % N;
@@ -436,8 +447,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(otf_w
     const int mem = (int)(t / bpm);
     const long long c0 = (t - (long long)mem * bpm) * NP;
     T += (long long)mem * S * ntot;
-    GConst<R> gc;
-    otf_consts<R, S>(cst, gc, G, tid);
+    otf_consts<R, S>(cst, G, tid);
     // element e of the tile: column q fastest, then position p (= i), then
     // system a; every load of a thread is in flight before its LDS writes.
     // Plain (temporal) accesses: the lines are shared with the other tiles.
@@ -455,7 +465,7 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(otf_w
         if (TOT % NTHR == 0 || e < TOT) lds.st(XA::at(p, a * NP + q), r[k]);
     }
     __syncthreads();
-    double v[1] = {otf_tile<R, N, S, true>(lds, tw, G, gc, cst, c0, ncol, tid)};
+    double v[1] = {otf_tile<R, N, S, true>(lds, tw, G, cst, c0, ncol, tid)};
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
         const int e = tid + k * NTHR;
@@ -501,8 +511,7 @@ __global__ void __launch_bounds__(NTHR)
     PFDD_TILE(V, lds, XA::size(N));
     __shared__ R cst[S * 12];
     __shared__ double red[NTHR / 64];
-    GConst<R> gc;
-    otf_consts<R, S>(cst, gc, G, threadIdx.x);
+    otf_consts<R, S>(cst, G, threadIdx.x);
     int t = blockIdx.x;
     V r[PER];
     {
@@ -531,7 +540,7 @@ __global__ void __launch_bounds__(NTHR)
             cols_fetch<N, NL, NP, NTHR>(r, T2 + (long long)mn * S * ntot, (long long)(tn - mn * bpm) * NP, ncol,
                                         ntot, tid);
         }
-        el += otf_tile<R, N, S>(lds, tw, G, gc, cst, c0, ncol, tid);
+        el += otf_tile<R, N, S>(lds, tw, G, cst, c0, ncol, tid);
 #pragma unroll 4
         for (int e = tid; e < TOT; e += NTHR) {
             const int l = e / N, p = e % N;
@@ -568,6 +577,12 @@ template <int N, int S> struct XTile {
 // accesses per value at 128 and 256 points, 12 with the stages in LDS.  The
 // FP64 tile is one plane of doubles (real parts, then imaginary parts), half
 // the LDS of k_mid_otf for the same columns.
+// Bound by instructions as much as by memory (162 VALU instructions per value at
+// 3 systems before the following, 134 after): the constants of the contraction
+// come by scalar loads instead of LDS broadcasts, which were a third of all LDS
+// accesses; a column's part of f is formed once; P as above.  Measured, us:
+// 512 x 512 x 256 x 3 FP64 1613 -> 1410, FP32 893 -> 787; 128^3 x 12 192 -> 182,
+// 87 -> 81.
 template <typename R, int N, int S>
 __global__ void __launch_bounds__((XTile<N, S>::W)) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 4, 8)))
     k_mid_r(typename cvec<R>::type *__restrict__ T2, GParams G, long long ncol, long long ntot, int bpm,
@@ -581,8 +596,7 @@ __global__ void __launch_bounds__((XTile<N, S>::W)) __attribute__((amdgpu_waves_
     if (*done) return;
     __shared__ __align__(16) char mem[N * NL * RegLds<V>::bytes];
     __shared__ V tws[N];
-    __shared__ R cst[S * 12];
-    __shared__ double red[NW];
+    __shared__ double red[NW], fcol[3 * NP];
     RegLds<V> lds{(decltype(RegLds<V>::p))mem};
     const int t = threadIdx.x;
     // member of a batch (bpm blocks per member), first column of the block
@@ -595,10 +609,7 @@ __global__ void __launch_bounds__((XTile<N, S>::W)) __attribute__((amdgpu_waves_
 #pragma unroll
     for (int m = 0; m < VPT; ++m) v[m] = ld_stream(own + D * m);
     reg_twiddles<N, W>(tws, tw, t);
-    GConst<R> gc;
-    for (int c = t; c < S * 12; c += W) cst[c] = (R)((c % 12) < 6 ? G.sig6[(c / 12) * 6 + c % 12]
-                                                                 : G.eps6[(c / 12) * 6 + c % 12 - 6]);
-    gc = GConst<R>{(R)G.inv2C44, (R)G.inv1mnu, (R)G.invmu, (R)G.C44x2, (R)G.C12};
+    if (t < NP) otf_col(G, c0 + t, fcol + 3 * t);
     reg_fft<N, 1, 1, NL, VPT, false, true, true, true, L>(v, lds, tws, t);
     // lines -> k-points: slot i S + a of a thread is system a of point t + W i
     V x[PTS * S];
@@ -644,34 +655,38 @@ __global__ void __launch_bounds__((XTile<N, S>::W)) __attribute__((amdgpu_waves_
 #pragma unroll
     for (int i = 0; i < PTS; ++i) {
         if (ok[i]) {
-            // compiler-only barriers keep the (LDS-broadcast) constants from
-            // being held in registers across points and systems
-            __asm__ volatile("" ::: "memory");
             const int pt = t + W * i;
-            R f[3], c2, c4;
-            bool nzf;
-            otf_freq<N, NP, S, R>(G, c0 + pt / N, pt % N, f, nzf, c2, c4);
-            R Pr[6] = {}, Pi[6] = {};
+            const KPoint<R> K = otf_freq<R>(G, fcol + 3 * (pt / N), pt % N);
+            // the constants come by scalar loads, a few systems' at a time: each
+            // group through a pointer of its own
+            typedef const R __attribute__((address_space(4))) CR;
+            CR *cst = (CR *)G.cst;
+            R Pr[6], Pi[6];
 #pragma unroll
-            for (int b = 0; b < S; ++b)
+            for (int b = 0; b < S; ++b) {
+                if (b % (sizeof(R) == 8 ? 2 : 3) == 0) __asm__ volatile("" : "+s"(cst));
 #pragma unroll
                 for (int c = 0; c < 6; ++c) {
-                    Pr[c] += cst[b * 12 + c] * x[i * S + b].x;
-                    Pi[c] += cst[b * 12 + c] * x[i * S + b].y;
+                    Pr[c] = b ? ab_c(cst[b * 6 + c], x[i * S + b].x, Pr[c]) : cst[c] * x[i * S].x;
+                    Pi[c] = b ? ab_c(cst[b * 6 + c], x[i * S + b].y, Pi[c]) : cst[c] * x[i * S].y;
                 }
-            if (nzf) otf_green(Pr, Pi, f, c2, c4, gc);
+            }
+            if (K.nz) otf_green(Pr, Pi, K);
+            else otf_zero(Pr, Pi);
 #pragma unroll
             for (int a = 0; a < S; ++a) {
-                __asm__ volatile("" ::: "memory");
-                R gr = 0, gi = 0;
+                if (a % (sizeof(R) == 8 ? 2 : 3) == 0) __asm__ volatile("" : "+s"(cst));
+                CR *const ep = cst + S * 6 + a * 6;
+                R gr = Pr[0] * ep[0], gi = Pi[0] * ep[0];
 #pragma unroll
-                for (int c = 0; c < 6; ++c) {
-                    gr += Pr[c] * cst[a * 12 + 6 + c];
-                    gi += Pi[c] * cst[a * 12 + 6 + c];
+                for (int c = 1; c < 6; ++c) {
+                    gr = ab_c(Pr[c], ep[c], gr);
+                    gi = ab_c(Pi[c], ep[c], gi);
                 }
-                gr *= gc.invmu;
-                gi *= gc.invmu;
-                if (!nzf) gr = gi = (R)0;
+                if constexpr (sizeof(R) == 4) {
+                    gr *= K.invmu;
+                    gi *= K.invmu;
+                }
                 el += (double)x[i * S + a].x * gr + (double)x[i * S + a].y * gi;
                 x[i * S + a] = mk<V>(gr, gi);
             }
