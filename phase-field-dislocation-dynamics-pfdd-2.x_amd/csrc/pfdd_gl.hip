@@ -315,6 +315,25 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// A new handle's small arrays, and the x pass's constants: by kernels, which
+// wait for nothing.
+__global__ void k_init(double *taud, int ntau, UpdNone *none, unsigned *ticket, int *done, int *steps)
+{
+    for (int a = threadIdx.x; a < ntau; a += blockDim.x) taud[a] = 0.0;
+    if (threadIdx.x != 0) return;
+    *none = UpdNone{1.0, 1.0f, 0};
+    *ticket = 0u;
+    *done = 0;
+    *steps = 0;
+}
+template <typename R> struct ConstArg {
+    R v[MAXS * 12];
+};
+template <typename R> __global__ void k_set_consts(R *cst, ConstArg<R> c, int n)
+{
+    for (int q = threadIdx.x; q < n; q += blockDim.x) cst[q] = c.v[q];
+}
+
 struct TauArg {
     double v[MAXS];
 };
@@ -521,6 +540,7 @@ struct pfdd_gl {
     int cur = 0;
     void *T1 = nullptr;
     void *B = nullptr;
+    char *small = nullptr;  // taud, none, cst, stage2, ticket, done, steps
     void *cst = nullptr;    // constants of the x pass (GParams)
     void *tw[3] = {nullptr, nullptr, nullptr}; // x, y, z twiddle tables
     uint8_t *mask = nullptr;
@@ -1123,8 +1143,8 @@ void destroy_all(pfdd_gl *h)
     hipSetDevice(h->device);
     if (h->stream) hipStreamSynchronize(h->stream);
     self_graph_release(h);
-    void *ptrs[] = {h->cof, h->taud, h->xi[0], h->xi[1], h->T1, h->B, h->cst, h->tw[0], h->tw[1], h->tw[2], h->mask, h->prev,
-                    h->amp, h->none, h->partial, h->done, h->steps, h->stage2, h->ticket, h->dw[0], h->dw[1],
+    void *ptrs[] = {h->cof, h->small, h->xi[0], h->xi[1], h->T1, h->B, h->tw[0], h->tw[1], h->tw[2], h->mask, h->prev,
+                    h->amp, h->partial, h->dw[0], h->dw[1],
                     h->deps, h->dsig, h->tape.lam[0], h->tape.lam[1], h->tape.gpart, h->tape.gacc};
     for (void *p : ptrs)
         if (p) hipFree(p);
@@ -1249,13 +1269,13 @@ int build_B(pfdd_gl *h)
     G.inv_n[1] = 1.0 / h->ny;
     G.inv_n[2] = 1.0 / h->nz;
     {
-        R cst[MAXS * 12];
+        ConstArg<R> cst{};
         for (int q = 0; q < S * 6; ++q) {
-            cst[q] = (R)G.sig6[q];
-            cst[S * 6 + q] = (R)(G.eps6[q] * (sizeof(R) == 8 ? G.invmu : 1.0));
+            cst.v[q] = (R)G.sig6[q];
+            cst.v[S * 6 + q] = (R)(G.eps6[q] * (sizeof(R) == 8 ? G.invmu : 1.0));
         }
-        HIPCHK(hipMalloc(&h->cst, sizeof(R) * S * 12));
-        HIPCHK(hipMemcpy(h->cst, cst, sizeof(R) * S * 12, hipMemcpyHostToDevice));
+        hipLaunchKernelGGL((k_set_consts<R>), dim3(1), dim3(64), 0, h->stream, (R *)h->cst, cst, S * 12);
+        HIPCHK(hipGetLastError());
         G.cst = h->cst;
     }
     if (!h->stored_B) return PFDD_OK;
@@ -1744,11 +1764,30 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
     }
     h->nb3 = h->M * (h->prec == PFDD_FP64 ? mid_blocks<double>(h->nx, h->S, (long long)h->ny * h->nz)
                                           : mid_blocks<float>(h->nx, h->S, (long long)h->ny * h->nz));
-    if ((rc = alloc((void **)&h->taud, sizeof(double) * h->SM))) return bail(rc);
-    if (h->M > 1) {
-        e = hipMemsetAsync(h->taud, 0, sizeof(double) * h->SM, h->stream);
-        if (e != hipSuccess) return bail(fail(PFDD_ERR_HIP, "hipMemset: %s", hipGetErrorString(e)));
-        h->P.taud = h->taud;
+    {
+        // the handle's small arrays, one allocation
+        size_t bytes = 0;
+        auto place = [&](size_t b) {
+            const size_t o = bytes;
+            bytes += (b + 63) / 64 * 64;
+            return o;
+        };
+        const size_t o_tau = place(sizeof(double) * h->SM), o_none = place(sizeof(UpdNone)),
+                     o_cst = place(sizeof(double) * MAXS * 12), o_st2 = place(sizeof(double) * NSLOT * NB2),
+                     o_tick = place(sizeof(unsigned)), o_done = place(sizeof(int)), o_steps = place(sizeof(int));
+        if ((rc = alloc((void **)&h->small, bytes))) return bail(rc);
+        h->taud = (double *)(h->small + o_tau);
+        h->none = (UpdNone *)(h->small + o_none);
+        h->cst = h->small + o_cst;
+        h->stage2 = (double *)(h->small + o_st2);
+        h->ticket = (unsigned *)(h->small + o_tick);
+        h->done = (int *)(h->small + o_done);
+        h->steps = (int *)(h->small + o_steps);
+        hipLaunchKernelGGL(k_init, dim3(1), dim3(64), 0, h->stream, h->taud, h->SM, h->none, h->ticket, h->done,
+                           h->steps);
+        if ((e = hipGetLastError()) != hipSuccess)
+            return bail(fail(PFDD_ERR_HIP, "handle constants: %s", hipGetErrorString(e)));
+        if (h->M > 1) h->P.taud = h->taud;
     }
     h->pstride = h->nb5max > h->nb3 ? h->nb5max : h->nb3;
     // the plane iteration: FP32 or FP64 grids with square y-z planes that fit
@@ -1776,25 +1815,10 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
         const int dflt[5] = {1, 1, 1, 1, 0};
         set_tiles(h, dflt); // nb5 of the model's update tile
     }
-    {
-        const UpdNone none = {1.0, 1.0f, 0};
-        if ((rc = alloc((void **)&h->none, sizeof(none)))) return bail(rc);
-        if (hipMemcpy(h->none, &none, sizeof(none), hipMemcpyHostToDevice) != hipSuccess)
-            return bail(fail(PFDD_ERR_HIP, "constant upload failed"));
-    }
     if ((rc = alloc((void **)&h->partial, sizeof(double) * NSLOT * h->pstride))) return bail(rc);
-    if ((rc = alloc((void **)&h->stage2, sizeof(double) * NSLOT * NB2)) ||
-        (rc = alloc((void **)&h->ticket, sizeof(unsigned))))
-        return bail(rc);
     e = hipHostMalloc((void **)&h->stat, sizeof(RunStat), hipHostMallocDefault);
     if (e != hipSuccess) return bail(fail(PFDD_ERR_HIP, "hipHostMalloc: %s", hipGetErrorString(e)));
     *h->stat = RunStat{};
-    e = hipMemsetAsync(h->ticket, 0, sizeof(unsigned), h->stream);
-    if (e != hipSuccess) return bail(fail(PFDD_ERR_HIP, "hipMemset: %s", hipGetErrorString(e)));
-    if ((rc = alloc((void **)&h->done, sizeof(int))) || (rc = alloc((void **)&h->steps, sizeof(int))))
-        return bail(rc);
-    reset_run(h, h->stream);
-
     // obstacle mask + quirk Q3 predecessor table (restarting with every member)
     if (d->xo) {
         const long long n = (long long)h->SM * h->N, nmem = (long long)h->S * h->N;
