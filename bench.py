@@ -103,7 +103,7 @@ def roofline(s, prof_steps=50, warm_steps=50):
 
 def load_pmc_traffic(tag, kernel):
     """HBM bytes per launch of the kernel instance `kernel` (its template name,
-    e.g. "k_update<float, 128, 2, false>") from the committed rocprofv3 PMC
+    e.g. "k_update_r<float, 128, 1, true, 2, false>") from the committed rocprofv3 PMC
     summary (FETCH_SIZE + WRITE_SIZE, calibrated with a copy kernel), or None
     when that instance was not measured."""
     path = os.path.join(ROOT, "profiles", f"pmc_traffic_{tag}.json")
@@ -120,28 +120,43 @@ def load_pmc_traffic(tag, kernel):
 def kernel_instance(s, role, tiles):
     """Template name of the kernel that runs `role` for solver s with the
     tuning choice `tiles` (fwd z, fwd y, inv y, inv z + update, iteration),
-    as rocprofv3 reports it (sine-series core: the update's GEN flag is false)."""
+    as rocprofv3 reports it, inside a run (the update followed by the next
+    iteration's forward transform; a core of up to two sine terms, no mask and
+    no amplitude field: GEN and MA are false)."""
     T = "double" if s.precision == pfdd_gl.PFDD_FP64 else "float"
     nx, ny, nz = s.shape
     S = s.S
+    reg = (32, 64, 128, 256, 512)      # lengths with register transforms
+    two_plans = (16, 48, 80, 128, 256)  # lengths whose radix-16 plan differs
+
+    def plan(n, tq):
+        return int(tq >= 3 and n in two_plans)
     if role == "fwd_yz":
         return f"k_plane_fwd<{T}, {ny}, {nz}>"
     if role == "inv_yz_update":
-        return f"k_plane_upd<{T}, {ny}, {nz}, false>"
+        return f"k_plane_upd<{T}, {ny}, {nz}, false, true>"
     if role == "x_contract":
         if STORED_B:
             return f"k_mid<{T}, {T}, {nx}, {S}>"
+        if nx in reg and tiles[4] != 2:
+            return f"k_mid_r<{T}, {nx}, {S}>"
         return {0: "k_mid_otf", 1: "k_mid_otf_pipe", 2: "k_mid_otf_pl"}[tiles[4]] + f"<{T}, {nx}, {S}>"
     if role == "inv_z_update":
-        return f"k_update<{T}, {nz}, {tiles[3]}, false>"
+        if nz in reg:
+            return f"k_update_r<{T}, {nz}, {plan(nz, tiles[0])}, true, 2, false>"
+        return f"k_update<{T}, {nz}, {tiles[3]}, false, {1 + plan(nz, tiles[0])}>"
     n, inv, tq = {"fwd_z": (nz, "false", tiles[0]), "fwd_y": (ny, "false", tiles[1]),
                   "inv_y": (ny, "true", tiles[2])}[role]
-    return f"k_fft_pass<{T}, {n}, {inv}, {tq}>"
+    if n in reg:
+        ends = "true, false" if inv == "false" else "false, true"
+        return f"k_pass_r<{T}, {n}, {plan(n, tq)}, {inv}, {ends}>"
+    return f"k_fft_pass<{T}, {n}, {inv}, {tq % 3}, {plan(n, tq)}>"
 
 
 # kernel families of the GL iteration and the roles they play
-KERNEL_ROLES = {"k_mid_otf": "x_contract", "k_mid<": "x_contract", "k_update<": "inv_z_update",
-                "k_plane_fwd": "fwd_yz", "k_plane_upd": "inv_yz_update", "k_fft_pass": "line_pass"}
+KERNEL_ROLES = {"k_mid_otf": "x_contract", "k_mid<": "x_contract", "k_mid_r<": "x_contract",
+                "k_update<": "inv_z_update", "k_update_r<": "inv_z_update", "k_plane_fwd": "fwd_yz",
+                "k_plane_upd": "inv_yz_update", "k_fft_pass": "line_pass", "k_pass_r": "line_pass"}
 
 
 PROBE_STEPS = 3
@@ -214,8 +229,9 @@ def pmc_summarize(fetch_dir, write_dir, size, out_dir):
         kbytes, _ = s.traffic()
         s.close()
         # algorithmic bytes per launch: 2 S N e for a line pass or the x pass,
-        # 3 S N e for an update (the plane kernels: 2 and 3 S N e as well)
-        two, three = kbytes[0], kbytes[4]
+        # 4 S N e for an update with the next forward transform, 3 S N e for
+        # one without (the plane kernels: 2, 4 and 3 S N e as well)
+        two, four = kbytes[0], kbytes[4]
         res = {"copy_calibration": {"kernel": copy_name, "bytes_read": nbytes, "bytes_written": nbytes,
                                     "fetch_kib": copy_f, "write_kib": copy_w,
                                     "fetch_scale": sf, "write_scale": sw}, "kernels": {}}
@@ -230,7 +246,12 @@ def pmc_summarize(fetch_dir, write_dir, size, out_dir):
             (f, _), (w, _) = per_kernel(fetch, m, PROBE_STEPS), per_kernel(write, m, PROBE_STEPS)
             if f is None or w is None:
                 continue
-            algo = three if role in ("inv_z_update", "inv_yz_update") else two
+            algo = two
+            if role in ("inv_z_update", "inv_yz_update"):
+                arg = kn[kn.index("<") + 1:-1].split(", ")
+                fused = {"k_update_r": arg[3:4] == ["true"], "k_plane_upd": arg[4:5] == ["true"],
+                         "k_update": arg[4:5] != ["0"]}[kn[:kn.index("<")]]
+                algo = four if fused else 0.75 * four
             res["kernels"][kn] = {"role": role, "launches": PROBE_STEPS,
                                   "fetch_bytes": f * 1024.0 * sf, "write_bytes": w * 1024.0 * sw,
                                   "hbm_bytes_per_launch": f * 1024.0 * sf + w * 1024.0 * sw,
