@@ -79,3 +79,25 @@ def test_run_counters_over_runs_of_every_kind():
             h.close()
     finally:
         g.close()
+
+
+def test_gradients_do_not_depend_on_the_tuning():
+    """Reverse mode on a handle tuned to the plane iteration sums its blocks as
+    on any other.  Tolerance: the sums over 1e5 cells are taken in another
+    order, each term below the largest (error below 1e5 u = 2e-11 of it,
+    typically its square root)."""
+    case = P.make_case(shape=(32, 32, 32), systems="basal3", core="sine", noise=1e-2, sigma_mu=0.004)
+    rng = np.random.default_rng(5)
+    seed = rng.standard_normal((3, 32, 32, 32)) + 1j * rng.standard_normal((3, 32, 32, 32))
+    out = []
+    for choice in ([1, 1, 1, 1, 0], [1, 1, 1, 1, 2], [0, 1, 1, 2, 2]):
+        g = P.gpu_solver(case)
+        try:
+            g.set_tuning(choice)
+            g.tape_record(5, 3)
+            out.append(g.tape_backward(seed, 2))
+        finally:
+            g.close()
+    for got in out[1:]:
+        for a, b in zip(got, out[0]):
+            assert np.max(np.abs(np.asarray(a) - np.asarray(b))) <= 2e-11 * np.max(np.abs(np.asarray(b)))
