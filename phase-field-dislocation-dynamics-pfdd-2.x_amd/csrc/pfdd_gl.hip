@@ -549,7 +549,7 @@ struct pfdd_gl {
     UpdNone *none = nullptr;
     double *partial = nullptr;
     long long pstride = 0;
-    int nb3 = 0, nb5 = 0, nb5max = 0; // blocks of pass 3 / pass 5 (current tile, smallest tile)
+    int nb3 = 0, nb5max = 0; // blocks of pass 3 / of pass 5 with its smallest tile
     int tq[4] = {1, 1, 1, 1};          // tile shape of fwd z, fwd y, inv y, inv z + update
     int xpipe = 0;                     // x pass: 0 one tile per block, 1 persistent pipelined
     int plane = 0;                     // 1: three-kernel plane iteration (pfdd_plane.hip)
@@ -743,6 +743,7 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
     // E_core as the reference accumulates it (sum / nx); core_energy_extended
     // and core_energy_pyrII do not accumulate it (fft_fftw_slab.cpp:1320,1483)
     const bool no_eref = P.model == PFDD_CORE_EXTENDED || P.model == PFDD_CORE_PYRII;
+    int nb5 = 0; // partials of the update
     if (h->plane) {
         // plane iteration: 2-D forward pass xo -> T1, x pass on T1 in its
         // plane layout, 2-D inverse pass + update T1 + xo -> T2.  The slots
@@ -771,6 +772,7 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
         arm(4);
         HIPCHK(launch_plane_upd<R>(h->ny, h->nz, !last, h->T1, xo, T2, h->mask, h->prev, h->cof ? h->cof : h->amp,
                                    nplanes, h->nx, last ? h->nbC : h->nbCF, P, h->tw[1], h->tw[2], h->partial, h->pstride, h->done, st));
+        nb5 = (int)nplanes;
     } else {
     if (first) {
         arm(0);
@@ -795,11 +797,11 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
     // the field does not depend on how a run is cut into calls
     HIPCHK(launch_update<R>(h->nz, h->tq[3], h->tq[0] / 3, !last, h->T1, xo, T2, h->mask, h->prev,
                             h->cof ? h->cof : h->amp, m.p5i, m.p5o, m.n5, (long long)h->nx * h->ny, P, h->tw[2],
-                            h->none, ord.keep, h->partial, h->pstride, h->done, st));
+                            h->none, ord.keep, h->partial, h->pstride, h->done, st, &nb5));
     }
     arm(5);
     PFDD_LAUNCH(k_sums, dim3(NB2), dim3(NTHR), st,
-                Sums{h->partial, h->pstride, h->nb5, h->nb3, 1.0 / (double)h->N, no_eref ? 0.0 : 1.0 / (double)h->nx,
+                Sums{h->partial, h->pstride, nb5, h->nb3, 1.0 / (double)h->N, no_eref ? 0.0 : 1.0 / (double)h->nx,
                      tol, h->stage2, h->ticket, h->stat, h->done, h->steps, last});
     HIPCHK(hipGetLastError());
     return PFDD_OK;
@@ -828,14 +830,6 @@ void set_tiles(pfdd_gl *h, const int tq[5])
     // pass, 2 the three-kernel plane iteration where the grid allows it
     h->plane = (tq[4] == 2 && h->plane_ok) ? 1 : 0;
     h->xpipe = (h->stored_B || tq[4] != 1) ? 0 : 1;
-    if (h->plane) {
-        h->nb5 = (int)((long long)h->SM * h->nx); // one partial per y-z plane
-    } else {
-        const long long n5 = (long long)h->SM * h->nx * h->ny;
-        const int nl = h->prec == PFDD_FP64 ? update_lines<double>(h->nz, h->tq[3], m)
-                                            : update_lines<float>(h->nz, h->tq[3], m);
-        h->nb5 = (int)((n5 + nl - 1) / nl);
-    }
     ++h->version; // captured graphs hold the old launch shapes
 }
 
@@ -1754,14 +1748,7 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
 
     // per-block partials
     const long long n5 = (long long)h->SM * h->nx * h->ny;
-    const int nl5min = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, 0) : tile_lines_rt<float>(h->nz, 0);
-    h->nb5max = (int)((n5 + nl5min - 1) / nl5min);
-    {
-        // the register update's tiles are smaller on short lines
-        const int nlr = h->prec == PFDD_FP64 ? update_lines<double>(h->nz, 0, d->core_model)
-                                             : update_lines<float>(h->nz, 0, d->core_model);
-        h->nb5max = std::max(h->nb5max, (int)((n5 + nlr - 1) / nlr));
-    }
+    h->nb5max = h->prec == PFDD_FP64 ? update_blocks_max<double>(h->nz, n5) : update_blocks_max<float>(h->nz, n5);
     h->nb3 = h->M * (h->prec == PFDD_FP64 ? mid_blocks<double>(h->nx, h->S, (long long)h->ny * h->nz)
                                           : mid_blocks<float>(h->nx, h->S, (long long)h->ny * h->nz));
     {
@@ -1813,7 +1800,7 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
     }
     {
         const int dflt[5] = {1, 1, 1, 1, 0};
-        set_tiles(h, dflt); // nb5 of the model's update tile
+        set_tiles(h, dflt);
     }
     if ((rc = alloc((void **)&h->partial, sizeof(double) * NSLOT * h->pstride))) return bail(rc);
     e = hipHostMalloc((void **)&h->stat, sizeof(RunStat), hipHostMallocDefault);

@@ -447,19 +447,21 @@ hipError_t launch_pass(int n, const void *in, void *out, LineMap mi, LineMap mo,
 
 // Last inverse pass + GL update, and its reverse mode (pfdd_update.hip).
 // plan: radix plan of the z transforms; fw: also the next iteration's forward
-// z pass of the new field (T1 in place).  Blocks (partials) of a launch:
-// nlines / update_lines.
+// z pass of the new field (T1 in place).  *nblocks: blocks, that is partials
+// per slot, of the launch: the kernel and its tile follow from P.model, which
+// pfdd_gl_set_core_coef changes on a handle (and a recorded run keeps its own),
+// so only the launch knows.  update_blocks_max: the most of any model and tile.
 struct UpdNone {  // device constants read where a run has no mask or no amplitude
     double one64;
     float one32;
     uint8_t zero;
 };
-template <typename R> int update_lines(int n, int tq, int model);
+template <typename R> int update_blocks_max(int n, long long nlines);
 template <typename R>
 hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
                          const long long *prev, const void *amp, LineMap mi, LineMap mo, long long nlines,
                          long long lps, const StepParams &P, const void *tw, const UpdNone *none, bool keep,
-                         double *partial, long long pstride, const int *done, hipStream_t st);
+                         double *partial, long long pstride, const int *done, hipStream_t st, int *nblocks);
 template <typename R>
 hipError_t launch_adj_update(int n, int tq, const void *T1, const void *lam, const void *xs, void *lam_out,
                              const uint8_t *mask, const void *amp, LineMap mi, LineMap mo, long long nlines,

@@ -418,20 +418,24 @@ __global__ void __launch_bounds__(NTHR)
 }
 
 
-template <typename R> int update_lines(int n, int tq, int model)
+template <typename R> int update_blocks_max(int n, long long nlines)
 {
-    const bool gen = model == PFDD_CORE_EXTENDED || model == PFDD_CORE_PYRII || model == PFDD_CORE_FOURIER;
-#define PFDD_CASE(n_) if (n == n_ && reg_length<n_>() && !gen) return RegTile<R, n_>::NL;
+    // the smallest tiles: shape 0, and on short lines the register update's
+    int nl = tile_lines_rt<R>(n, 0);
+#define PFDD_CASE(n_)                                                                          \
+    if (n == n_) {                                                                             \
+        if constexpr (reg_length<n_>()) nl = RegTile<R, n_>::NL < nl ? RegTile<R, n_>::NL : nl; \
+    }
     PFDD_SIZES(PFDD_CASE)
 #undef PFDD_CASE
-    return tile_lines_rt<R>(n, tq);
+    return (int)((nlines + nl - 1) / nl);
 }
 
 template <typename R>
 hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void *xo, void *xn, const uint8_t *mask,
                          const long long *prev, const void *amp, LineMap mi, LineMap mo, long long nlines,
                          long long lps, const StepParams &P, const void *tw, const UpdNone *none, bool keep,
-                         double *partial, long long pstride, const int *done, hipStream_t st)
+                         double *partial, long long pstride, const int *done, hipStream_t st, int *nblocks)
 {
     typedef typename cvec<R>::type V;
     const uint8_t *no_mask = &none->zero;
@@ -445,7 +449,7 @@ hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void 
     // plan 1 falls back to plan 0 where the two coincide
 #define PFDD_UPR_(PL_, FW_, NM_, MA_)                                                                \
     PFDD_LAUNCH((k_update_r<R, N, (PL_ && radix16_plan_differs<N>()), FW_, NM_, MA_>),               \
-                dim3((unsigned)(nlines / RegTile<R, N>::NL)), dim3(RegTile<R, N>::W), st, (V *)T1,   \
+                dim3((unsigned)*nblocks), dim3(RegTile<R, N>::W), st, (V *)T1,                       \
                 (const V *)xo, (V *)xn, mask ? mask : no_mask, prev,                                 \
                 amp ? (const R *)amp : no_amp, mask ? 1u : 0u, amp ? 1u : 0u, (unsigned)mi.D,        \
                 (unsigned)lps, P, (const V *)tw, keep, partial, pstride, done)
@@ -462,20 +466,21 @@ hipError_t launch_update(int n, int tq, int plan, bool fw, void *T1, const void 
         }                                                                                            \
     } while (0)
 #define PFDD_UPD(TQ_, GEN_, FW_)                                                                     \
-    PFDD_LAUNCH((k_update<R, N, TQ_, GEN_, FW_>),                                                    \
-                dim3((unsigned)((nlines + tile_lines_u<R, N, TQ_>() - 1) / tile_lines_u<R, N, TQ_>())), \
-                dim3(NTHR), st, (V *)T1, (const V *)xo, (V *)xn, mask, prev, (const R *)amp, mi, mo, \
+    *nblocks = (int)((nlines + tile_lines_u<R, N, TQ_>() - 1) / tile_lines_u<R, N, TQ_>());          \
+    PFDD_LAUNCH((k_update<R, N, TQ_, GEN_, FW_>), dim3((unsigned)*nblocks), dim3(NTHR), st,         \
+                (V *)T1, (const V *)xo, (V *)xn, mask, prev, (const R *)amp, mi, mo, \
                 nlines, lps, P, (const V *)tw, keep, partial, pstride, done)
 #define PFDD_UPD_FW(TQ_, GEN_)                                                                       \
-    if (!fw) PFDD_UPD(TQ_, GEN_, 0);                                                                 \
-    else if (plan == 1 && radix16_plan_differs<N>()) PFDD_UPD(TQ_, GEN_, (radix16_plan_differs<N>() ? 2 : 1)); \
-    else PFDD_UPD(TQ_, GEN_, 1)
+    if (!fw) { PFDD_UPD(TQ_, GEN_, 0); }                                                             \
+    else if (plan == 1 && radix16_plan_differs<N>()) { PFDD_UPD(TQ_, GEN_, (radix16_plan_differs<N>() ? 2 : 1)); } \
+    else { PFDD_UPD(TQ_, GEN_, 1); }
 #define PFDD_CASE(n_)                                                                                \
     if (n == n_) {                                                                                   \
         constexpr int N = n_;                                                                        \
         if constexpr (reg_length<N>()) {                                                             \
             if (!gen) {                                                                              \
                 const bool p1 = plan == 1 && radix16_plan_differs<N>();                              \
+                *nblocks = (int)(nlines / RegTile<R, N>::NL);                                        \
                 if (p1 && fw) PFDD_UPR(1, true);                                                     \
                 else if (p1) PFDD_UPR(1, false);                                                     \
                 else if (fw) PFDD_UPR(0, true);                                                      \
@@ -525,11 +530,11 @@ hipError_t launch_adj_update(int n, int tq, const void *T1, const void *lam, con
 }
 
 #define PFDD_INST(R)                                                                                          \
-    template int update_lines<R>(int, int, int);                                                                      \
+    template int update_blocks_max<R>(int, long long);                                                                \
     template hipError_t launch_update<R>(int, int, int, bool, void *, const void *, void *, const uint8_t *,           \
                                          const long long *, const void *, LineMap, LineMap, long long, long long, \
                                          const StepParams &, const void *, const UpdNone *, bool, double *, long long, \
-                                         const int *, hipStream_t);                                               \
+                                         const int *, hipStream_t, int *);                                        \
     template hipError_t launch_adj_update<R>(int, int, const void *, const void *, const void *, void *,         \
                                              const uint8_t *, const void *, LineMap, LineMap, long long,          \
                                              long long, const StepParams &, const void *, double *, long long,    \
