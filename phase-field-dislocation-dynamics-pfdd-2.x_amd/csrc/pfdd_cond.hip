@@ -21,6 +21,24 @@ __device__ __forceinline__ void cond_point(double2 c, const double *f, double2 &
     b = make_double2(c.x * r * f[1], c.y * r * f[1]);
 }
 
+// Raises *done where a total of the update before (nu partials per slot, 0 at the
+// start of a run) is not finite; called by one block of a kernel that runs
+// between two updates.  From there on the updates and the line passes return at
+// once, so c stays as that iteration left it.  The kernels that call this do not
+// read the flag themselves: their blocks run while it is raised.
+template <int W>
+__device__ __forceinline__ void cond_check(const double *part, long long pstride, int nu, int *done, double *red,
+                                           int tid)
+{
+    double v[3] = {0.0, 0.0, 0.0};
+    const int slot[3] = {0, 2, 3};
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+        for (int b = tid; b < nu; b += W) v[q] += part[slot[q] * pstride + b];
+    block_sum<3, W>(v, red, tid);
+    if (tid == 0 && !(isfinite(v[0]) && isfinite(v[1]) && isfinite(v[2]))) *done = 1;
+}
+
 // divcurrent on the transformed field in the [k][j][i] layout, written as
 // [2][k][j][i].  The block also sums sig[(ny - j) mod ny] Re a over its
 // k-points: backwardcond called a second time on its own output (the trailing
@@ -28,11 +46,11 @@ __device__ __forceinline__ void cond_point(double2 c, const double *f, double2 &
 // unnormalised inverse transforms give N a(-r).
 __global__ void __launch_bounds__(NTHR)
     k_cond_div(const double2 *__restrict__ ch, double2 *__restrict__ ab, const double *__restrict__ sig, CondParams P,
-               long long N, double *__restrict__ part, const int *__restrict__ done)
+               long long N, double *__restrict__ part, long long pstride, int nu, int *done)
 {
-    if (*done) return;
-    __shared__ double red[NTHR / 64];
+    __shared__ double red[3 * (NTHR / 64)];
     const int tid = threadIdx.x;
+    if (blockIdx.x == 0) cond_check<NTHR>(part, pstride, nu, done, red, tid);
     const long long idx = (long long)blockIdx.x * NTHR + tid;
     double v[1] = {0.0};
     if (idx < N) {
@@ -49,7 +67,7 @@ __global__ void __launch_bounds__(NTHR)
         v[0] = sig[(P.ny - j) % P.ny] * a.x;
     }
     block_sum<1, NTHR>(v, red, tid);
-    if (tid == 0) part[blockIdx.x] = v[0];
+    if (tid == 0) part[4 * pstride + blockIdx.x] = v[0];
 }
 
 // The same between the forward x transform and the two inverse ones: a block
@@ -62,17 +80,18 @@ template <int N> struct CondX {
 template <int N>
 __global__ void __launch_bounds__((CondX<N>::W)) __attribute__((amdgpu_waves_per_eu(2, 8)))
     k_cond_x(const double2 *__restrict__ ch, double2 *__restrict__ ab, const double *__restrict__ sig, CondParams P,
-             long long ntot, const double2 *__restrict__ tw, double *__restrict__ part, const int *__restrict__ done)
+             long long ntot, const double2 *__restrict__ tw, double *__restrict__ part, long long pstride, int nu,
+             int *done)
 {
     typedef CondX<N> X;
     constexpr int VPT = X::VPT, D = X::D, W = X::W, NL = X::NL;
     typedef RegSwzX<N> L;
-    if (*done) return;
     __shared__ __align__(16) char mem[N * NL * RegLds<double2>::bytes];
     __shared__ double2 tws[N];
-    __shared__ double red[W / 64];
+    __shared__ double red[3 * (W / 64)];
     RegLds<double2> lds{(double *)mem};
     const int t = threadIdx.x, l = t / D, p0 = t % D;
+    if (blockIdx.x == 0) cond_check<W>(part, pstride, nu, done, red, t);
     const long long line = (long long)blockIdx.x * NL + l;
     const long long at = line * N + p0;
     double2 v[VPT], w[VPT];
@@ -96,7 +115,7 @@ __global__ void __launch_bounds__((CondX<N>::W)) __attribute__((amdgpu_waves_per
     }
     double sum[1] = {sig[j ? P.ny - j : 0] * s};
     block_sum<1, W>(sum, red, t);
-    if (t == 0) part[blockIdx.x] = sum[0];
+    if (t == 0) part[4 * pstride + blockIdx.x] = sum[0];
     int t2 = t;
     __asm__ volatile("" : "+v"(t2)); // addresses formed again, as in k_update_r
     reg_fft<N, 1, 1, NL, VPT, true, true, true, false, L>(w, lds, tws, t2);
@@ -134,18 +153,12 @@ struct CondCell {
     }
 };
 
-// A block's sums, and the stop flag where they are not finite.
-__device__ __forceinline__ void cond_put(const double *v, double *part, long long pstride, int *done)
-{
-    for (int q = 0; q < 4; ++q) part[q * pstride + blockIdx.x] = v[q];
-    if (!isfinite(v[0]) || !isfinite(v[2]) || !isfinite(v[3])) *done = 1;
-}
-
 __global__ void __launch_bounds__(NTHR)
     k_cond_update(const double2 *__restrict__ ab, double2 *__restrict__ c, const double *__restrict__ sig,
                   const double *__restrict__ dsig, CondParams P, long long N, double *__restrict__ part,
-                  long long pstride, int *done)
+                  long long pstride, const int *__restrict__ done)
 {
+    if (*done) return;
     __shared__ double red[4 * (NTHR / 64)];
     const int tid = threadIdx.x;
     const long long idx = (long long)blockIdx.x * NTHR + tid;
@@ -156,7 +169,8 @@ __global__ void __launch_bounds__(NTHR)
         c[idx] = cell.update(cell.from_a(ab[idx], P, v), ab[N + idx], c[idx], P, v);
     }
     block_sum<4, NTHR>(v, red, tid);
-    if (tid == 0) cond_put(v, part, pstride, done);
+    if (tid == 0)
+        for (int q = 0; q < 4; ++q) part[q * pstride + blockIdx.x] = v[q];
 }
 
 // The same after the two inverse z transforms (a, b in the [2][i][k][j] layout,
@@ -168,10 +182,12 @@ template <int N, bool FW>
 __global__ void __launch_bounds__((RegTile<double, N>::W)) __attribute__((amdgpu_waves_per_eu(2, 8)))
     k_cond_update_r(const double2 *__restrict__ ab, double2 *__restrict__ c, double2 *__restrict__ T,
                     const double *__restrict__ sig, const double *__restrict__ dsig, CondParams P, long long ntot,
-                    const double2 *__restrict__ tw, double *__restrict__ part, long long pstride, int *done)
+                    const double2 *__restrict__ tw, double *__restrict__ part, long long pstride,
+                    const int *__restrict__ done)
 {
     typedef RegTile<double, N> G;
     constexpr int NL = G::NL, VPT = G::VPT, D = G::D, W = G::W;
+    if (*done) return;
     __shared__ __align__(16) char mem[N * NL * RegLds<double2>::bytes];
     __shared__ double2 tws[N];
     __shared__ double red[4 * (W / 64)];
@@ -214,7 +230,8 @@ __global__ void __launch_bounds__((RegTile<double, N>::W)) __attribute__((amdgpu
         for (int m = 0; m < VPT; ++m) T[row0 + (size_t)(D * m) * ny + o1] = a[m];
     }
     block_sum_comp<4, W>(v, red, t);
-    if (t == 0) cond_put(v, part, pstride, done);
+    if (t == 0)
+        for (int q = 0; q < 4; ++q) part[q * pstride + blockIdx.x] = v[q];
 }
 
 // The sums of a run's last iteration: nu partials of the update (slots 0-3), nd
@@ -256,16 +273,17 @@ bool cond_reg_length(int n)
 }
 
 hipError_t launch_cond_div(const double2 *ch, double2 *ab, const double *sig, const CondParams &P, double *part,
-                           int *nparts, const int *done, hipStream_t st)
+                           long long pstride, int nu, int *nparts, int *done, hipStream_t st)
 {
     const long long N = (long long)P.nx * P.ny * P.nz;
     *nparts = (int)((N + NTHR - 1) / NTHR);
-    hipLaunchKernelGGL(k_cond_div, dim3((unsigned)*nparts), dim3(NTHR), 0, st, ch, ab, sig, P, N, part, done);
+    hipLaunchKernelGGL(k_cond_div, dim3((unsigned)*nparts), dim3(NTHR), 0, st, ch, ab, sig, P, N, part, pstride,
+                       nu, done);
     return hipGetLastError();
 }
 
 hipError_t launch_cond_x(const double2 *ch, double2 *ab, const double *sig, const CondParams &P, const void *tw,
-                         double *part, int *nparts, const int *done, hipStream_t st)
+                         double *part, long long pstride, int nu, int *nparts, int *done, hipStream_t st)
 {
     const long long lines = (long long)P.ny * P.nz;
 #define PFDD_CASE(n_)                                                                                           \
@@ -275,7 +293,7 @@ hipError_t launch_cond_x(const double2 *ch, double2 *ab, const double *sig, cons
             if (lines % X::NL) return hipErrorInvalidValue;                                                     \
             *nparts = (int)(lines / X::NL);                                                                     \
             hipLaunchKernelGGL((k_cond_x<n_>), dim3((unsigned)*nparts), dim3(X::W), 0, st, ch, ab, sig, P,      \
-                               lines * n_, (const double2 *)tw, part, done);                                    \
+                               lines * n_, (const double2 *)tw, part, pstride, nu, done);                       \
             return hipGetLastError();                                                                           \
         }                                                                                                       \
     }
@@ -285,7 +303,7 @@ hipError_t launch_cond_x(const double2 *ch, double2 *ab, const double *sig, cons
 }
 
 hipError_t launch_cond_update(const double2 *ab, double2 *c, const double *sig, const double *dsig,
-                              const CondParams &P, double *part, long long pstride, int *nparts, int *done,
+                              const CondParams &P, double *part, long long pstride, int *nparts, const int *done,
                               hipStream_t st)
 {
     const long long N = (long long)P.nx * P.ny * P.nz;
@@ -297,7 +315,7 @@ hipError_t launch_cond_update(const double2 *ab, double2 *c, const double *sig, 
 
 hipError_t launch_cond_update_r(bool fw, const double2 *ab, double2 *c, double2 *T, const double *sig,
                                 const double *dsig, const CondParams &P, const void *tw, double *part,
-                                long long pstride, int *nparts, int *done, hipStream_t st)
+                                long long pstride, int *nparts, const int *done, hipStream_t st)
 {
     const long long lines = (long long)P.nx * P.ny;
 #define PFDD_UPD(FW_)                                                                                           \

@@ -2478,6 +2478,7 @@ void cond_release(pfdd_gl_cond *h)
 Maps cond_maps(const pfdd_gl_cond *h, long long S) { return make_maps_dims(h->nx, h->ny, h->nz, S); }
 
 // One iteration of a run.  first: c enters the run here; last: nothing follows.
+// nu: partials of the update before (0: none), then of this one's; nd: of divcurrent.
 int cond_step(pfdd_gl_cond *h, bool first, bool last, int &nu, int &nd)
 {
     hipStream_t st = h->stream;
@@ -2495,12 +2496,12 @@ int cond_step(pfdd_gl_cond *h, bool first, bool last, int &nu, int &nd)
     HIPCHK((launch_pass<double, false>(h->ny, in, out, m1.p2i, m1.p2o, m1.n2, h->tw[1], h->done, st)));
     swap();
     if (xr) {
-        HIPCHK(launch_cond_x(in, out, h->sig, h->P, h->tw[0], h->part + 4 * h->nb, &nd, h->done, st));
+        HIPCHK(launch_cond_x(in, out, h->sig, h->P, h->tw[0], h->part, h->nb, nu, &nd, h->done, st));
         swap();
     } else {
         HIPCHK((launch_pass<double, false>(h->nx, in, out, xs, xs, ncol, h->tw[0], h->done, st)));
         swap();
-        HIPCHK(launch_cond_div(in, out, h->sig, h->P, h->part + 4 * h->nb, &nd, h->done, st));
+        HIPCHK(launch_cond_div(in, out, h->sig, h->P, h->part, h->nb, nu, &nd, h->done, st));
         swap();
         HIPCHK((launch_pass<double, true>(h->nx, in, out, xs, xs, 2 * ncol, h->tw[0], h->done, st)));
         swap();
@@ -2624,7 +2625,8 @@ int pfdd_gl_cond_step(pfdd_gl_cond *h, int nsteps, pfdd_gl_cond_reduce *out)
     HIPCHK(hipSetDevice(h->device));
     // the host waits once, at the end of the run (a wait, a copy of the
     // partials and a sum on the host after every iteration cost 70 us of 225
-    // at 128^3); an iteration with sums that are not finite stops the rest
+    // at 128^3); after an iteration with sums that are not finite the field does
+    // not move on
     int nu = 0, nd = 0;
     for (int s = 0; s < nsteps; ++s) {
         const int rc = cond_step(h, s == 0, s == nsteps - 1, nu, nd);

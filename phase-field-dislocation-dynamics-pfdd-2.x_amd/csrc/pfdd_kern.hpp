@@ -506,8 +506,10 @@ hipError_t launch_plane_upd(int ny, int nz, bool fw, void *T, const void *xo, vo
 // transforms around it; the updates read a, b as [2][i][j][k], and
 // launch_cond_update_r, which also makes the z transforms before it (and with
 // fw the next forward one, into T [i][k][j]), as [2][i][k][j].  nparts: blocks,
-// that is partial sums, of a launch.  *done is raised by an update whose sums
-// are not finite; everything but the updates then returns at once.
+// that is partial sums, of a launch, part[slot * pstride + block]: slots 0-3 of
+// the update, 4 of divcurrent.  divcurrent also looks at the totals of the
+// update before it (nu partials, 0 where a run starts) and raises *done where
+// they are not finite; line passes and updates then return at once.
 struct CondParams {
     double four[9];
     double El;       // material->El[1]
@@ -522,15 +524,15 @@ struct CondStat {
 };
 bool cond_reg_length(int n); // the length has the fused kernels
 hipError_t launch_cond_div(const double2 *ch, double2 *ab, const double *sig, const CondParams &P, double *part,
-                           int *nparts, const int *done, hipStream_t st);
+                           long long pstride, int nu, int *nparts, int *done, hipStream_t st);
 hipError_t launch_cond_x(const double2 *ch, double2 *ab, const double *sig, const CondParams &P, const void *tw,
-                         double *part, int *nparts, const int *done, hipStream_t st);
+                         double *part, long long pstride, int nu, int *nparts, int *done, hipStream_t st);
 hipError_t launch_cond_update(const double2 *ab, double2 *c, const double *sig, const double *dsig,
-                              const CondParams &P, double *part, long long pstride, int *nparts, int *done,
+                              const CondParams &P, double *part, long long pstride, int *nparts, const int *done,
                               hipStream_t st);
 hipError_t launch_cond_update_r(bool fw, const double2 *ab, double2 *c, double2 *T, const double *sig,
                                 const double *dsig, const CondParams &P, const void *tw, double *part,
-                                long long pstride, int *nparts, int *done, hipStream_t st);
+                                long long pstride, int *nparts, const int *done, hipStream_t st);
 hipError_t launch_cond_sums(const double *part, long long pstride, int nu, int nd, CondStat *stat, int *done,
                             hipStream_t st);
 
