@@ -228,12 +228,14 @@ struct Sums {
 // on convergence or a non-finite result.  Where a run ends, it writes them to
 // the host's memory itself: three copies of a few bytes and the launch that
 // cleared the counters cost 60 of the 150 us of a one-iteration run at 32^3.
-// stage2 goes through relaxed agent-scope atomics, which reach the point where
-// all XCDs agree: only the wait for the stores stands before the ticket, no
-// fence with its write-back of the L2.  Having the update's last blocks do all
-// this (no launch of its own, 7 us) was slower from 64^3 x 3 up (53.0 -> 54.9
-// us per iteration, 749 -> 758 at 128^3 x 12): the wait for its stores holds a
-// wave of every block.
+// The ticket is taken with release and acquire at agent scope, which orders every
+// block's stage2 before the last one's loads (the block's barrier carries the
+// acquire to its other threads); a relaxed ticket behind a wait for the stores
+// is no faster: 75.75 and 75.65 us a run of one at 32^3 x 3, 41.6 and 41.7 us an
+// iteration at 64^3 x 1.  Having the update's last blocks do all this (no launch
+// of its own, 7 us) was slower from 64^3 x 3 up (53.0 -> 54.9 us per iteration,
+// 749 -> 758 at 128^3 x 12): the wait for its stores holds a wave of every
+// block.
 constexpr int NB2 = 32;
 static_assert(NB2 <= NTHR, "the last block reads stage2 one value per thread");
 
@@ -263,8 +265,7 @@ __global__ void __launch_bounds__(NTHR) k_sums(Sums F)
         for (int q = 0; q < NSLOT; ++q)
             __hip_atomic_store((long long *)&F.stage2[q * NB2 + blockIdx.x], __double_as_longlong(w[q]),
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        last = __hip_atomic_fetch_add(F.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == NB2 - 1;
+        last = __hip_atomic_fetch_add(F.ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == NB2 - 1;
     }
     __syncthreads();
     if (!last) return;
