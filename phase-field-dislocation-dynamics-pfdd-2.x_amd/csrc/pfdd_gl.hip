@@ -574,6 +574,7 @@ struct pfdd_gl {
     int ncu = 0;                       // compute units of the device
     double *stage2 = nullptr; // NSLOT * NB2
     unsigned *ticket = nullptr;
+    PinnedUser pinned;
     RunStat *stat = nullptr;  // pinned host memory
     // the host knows that *done == 0 and *steps == steps0: set by
     // collect_steps, and a run that starts so needs no k_reset
@@ -593,7 +594,6 @@ struct pfdd_gl {
     void *dw[2] = {nullptr, nullptr}; // output-step field workspace, max(S,6)*N complex each
     double2 *deps = nullptr;          // strain field (complex), 6 components of N
     double *dsig = nullptr;           // stress field (real) without sigma_rot, 6 components of N
-    Stage stage;                      // fields to and from the caller's memory
     double *xs_part = nullptr;        // XS_NB * SM block sums of xi_sums, pinned host memory
     bool tau_stale = true;            // single-run handle: taud does not hold P.tau
     // reverse mode: checkpoints of a recorded run and the adjoint workspace
@@ -1147,9 +1147,8 @@ void destroy_all(pfdd_gl *h)
         if (p) hipFree(p);
     for (void *p : h->tape.seg)
         if (p) hipFree(p);
-    if (h->stat) (void)hipHostFree(h->stat);
+    Pinned::get().unblock(h->stat);
     if (h->xs_part) (void)hipHostFree(h->xs_part);
-    h->stage.release();
     if (h->own_stream && h->stream) hipStreamDestroy(h->stream);
     delete h;
 }
@@ -1283,15 +1282,15 @@ int build_B(pfdd_gl *h)
 }
 
 // bytes to pageable host memory as they are.
-int copy_out(Stage &stage, const void *dev, void *host, size_t bytes, hipStream_t st)
+int copy_out(const void *dev, void *host, size_t bytes, hipStream_t st)
 {
-    if (bytes < Stage::MIN_BYTES) {
+    if (bytes < STAGE_MIN_BYTES) {
         HIPCHK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
         return PFDD_OK;
     }
-    HIPCHK(stage.out((char *)dev, bytes, st,
-                      [&](char *slot, size_t o, size_t n) { std::memcpy((char *)host + o, slot, n); }));
+    HIPCHK(stage_out((char *)dev, bytes, st,
+                     [&](char *slot, size_t o, size_t n) { std::memcpy((char *)host + o, slot, n); }));
     return PFDD_OK;
 }
 
@@ -1324,8 +1323,8 @@ int upload_field_f64(pfdd_gl *h, const double *host, void *dst)
 int download_field_f64(pfdd_gl *h, const void *src, double *host)
 {
     const size_t n = (size_t)h->SM * h->N * 2;
-    if (h->prec == PFDD_FP64) return copy_out(h->stage, src, host, n * 8, h->stream);
-    HIPCHK(h->stage.out((char *)src, n * 4, h->stream, [&](char *slot, size_t o, size_t len) {
+    if (h->prec == PFDD_FP64) return copy_out(src, host, n * 8, h->stream);
+    HIPCHK(stage_out((char *)src, n * 4, h->stream, [&](char *slot, size_t o, size_t len) {
         const float *from = (const float *)slot;
         double *to = host + o / 4;
         for (size_t q = 0; q < len / 4; ++q) to[q] = (double)from[q];
@@ -1400,7 +1399,7 @@ int diag_fields(pfdd_gl *h, const double *sigma_rot, const double *avepst, const
         }
     };
     if (data_eps)
-        HIPCHK(h->stage.out((char *)h->deps, sizeof(double2) * 6 * N, st, [&](char *slot, size_t o, size_t len) {
+        HIPCHK(stage_out((char *)h->deps, sizeof(double2) * 6 * N, st, [&](char *slot, size_t o, size_t len) {
             spread(slot, o, len, sizeof(double2), [&](int c, size_t r0, size_t n, const char *from) {
                 std::memcpy(data_eps + 2 * ((ci[c] + 3 * cj[c]) * N + r0), from, n * sizeof(double2));
                 if (ci[c] != cj[c])
@@ -1408,7 +1407,7 @@ int diag_fields(pfdd_gl *h, const double *sigma_rot, const double *avepst, const
             });
         }));
     if (data_sigma)
-        HIPCHK(h->stage.out((char *)h->dsig, sizeof(double) * 6 * N, st, [&](char *slot, size_t o, size_t len) {
+        HIPCHK(stage_out((char *)h->dsig, sizeof(double) * 6 * N, st, [&](char *slot, size_t o, size_t len) {
             spread(slot, o, len, sizeof(double), [&](int c, size_t r0, size_t n, const char *from) {
                 const double *v = (const double *)from;
                 const int i = ci[c], j = cj[c];
@@ -1804,8 +1803,8 @@ int pfdd_gl_create_batch(const pfdd_gl_desc *d, int nbatch, pfdd_gl **out)
         set_tiles(h, dflt);
     }
     if ((rc = alloc((void **)&h->partial, sizeof(double) * NSLOT * h->pstride))) return bail(rc);
-    e = hipHostMalloc((void **)&h->stat, sizeof(RunStat), hipHostMallocDefault);
-    if (e != hipSuccess) return bail(fail(PFDD_ERR_HIP, "hipHostMalloc: %s", hipGetErrorString(e)));
+    static_assert(sizeof(RunStat) <= Pinned::BLOCK && sizeof(CondStat) <= Pinned::BLOCK, "one block each");
+    if (!(h->stat = (RunStat *)Pinned::get().block())) return bail(fail(PFDD_ERR_HIP, "no pinned host memory"));
     *h->stat = RunStat{};
     // obstacle mask + quirk Q3 predecessor table (restarting with every member)
     if (d->xo) {
@@ -2459,8 +2458,8 @@ struct pfdd_gl_cond {
     int *done = nullptr;
     std::vector<double> sig_h;
     long long nb = 0;         // most partials of a kernel
+    PinnedUser pinned;
     CondStat *stat = nullptr; // pinned host memory
-    Stage stage;
 };
 
 namespace {
@@ -2470,8 +2469,7 @@ void cond_release(pfdd_gl_cond *h)
     for (void *p : {(void *)h->c, (void *)h->w0, (void *)h->w1, (void *)h->sig, (void *)h->dsig, (void *)h->part,
                     (void *)h->done, h->tw[0], h->tw[1], h->tw[2]})
         if (p) hipFree(p);
-    if (h->stat) (void)hipHostFree(h->stat);
-    h->stage.release();
+    Pinned::get().unblock(h->stat);
     if (h->own_stream && h->stream) hipStreamDestroy(h->stream);
 }
 
@@ -2572,9 +2570,9 @@ int pfdd_gl_cond_create(const pfdd_gl_cond_desc *d, pfdd_gl_cond **out)
         (e = hipMalloc((void **)&h->sig, sizeof(double) * d->ny)) != hipSuccess ||
         (e = hipMalloc((void **)&h->dsig, sizeof(double) * d->ny)) != hipSuccess ||
         (e = hipMalloc((void **)&h->part, sizeof(double) * 5 * h->nb)) != hipSuccess ||
-        (e = hipMalloc((void **)&h->done, sizeof(int))) != hipSuccess ||
-        (e = hipHostMalloc((void **)&h->stat, sizeof(CondStat), hipHostMallocDefault)) != hipSuccess)
+        (e = hipMalloc((void **)&h->done, sizeof(int))) != hipSuccess)
         return bail(fail(PFDD_ERR_HIP, "hipMalloc: %s", hipGetErrorString(e)));
+    if (!(h->stat = (CondStat *)Pinned::get().block())) return bail(fail(PFDD_ERR_HIP, "no pinned host memory"));
     const int dims[3] = {h->nx, h->ny, h->nz};
     for (int q = 0; q < 3; ++q) {
         std::vector<double> tw;
@@ -2616,7 +2614,7 @@ int pfdd_gl_cond_get(pfdd_gl_cond *h, double *c_host)
 {
     if (!h || !c_host) return fail(PFDD_ERR_ARG, "null argument");
     HIPCHK(hipSetDevice(h->device));
-    return copy_out(h->stage, h->c, c_host, sizeof(double2) * h->N, h->stream);
+    return copy_out(h->c, c_host, sizeof(double2) * h->N, h->stream);
 }
 
 int pfdd_gl_cond_step(pfdd_gl_cond *h, int nsteps, pfdd_gl_cond_reduce *out)
