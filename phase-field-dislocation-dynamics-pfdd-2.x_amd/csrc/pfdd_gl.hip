@@ -891,8 +891,15 @@ std::map<TuneKey, std::array<int, 5>> g_tune_cache;
 template <typename R>
 int autotune(pfdd_gl *h, int nsteps, int choice[5])
 {
+    // what selects the kernels besides the grid: the contraction, and the
+    // update's instance (mask, amplitude or core flag 5's angle factor with its
+    // kernel, the family of the core model, the terms of a sine series)
+    const int m = h->P.model;
+    const bool gen = m == PFDD_CORE_EXTENDED || m == PFDD_CORE_PYRII || m == PFDD_CORE_FOURIER;
     const TuneKey key{h->nx, h->ny, h->nz, h->S, h->M, h->prec,
-                      (h->stored_B ? 1 : 0) | (h->mask ? 2 : 0) | (h->amp ? 4 : 0)};
+                      (h->stored_B ? 1 : 0) | (h->mask ? 2 : 0) | (h->amp ? 4 : 0) | (h->cof ? 8 : 0) |
+                          (m == PFDD_CORE_EXTENDED ? 16 : gen ? 32 : 0) |
+                          (gen || h->P.ncoef <= 2 ? 0 : h->P.ncoef <= 4 ? 64 : 128)};
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         auto it = g_tune_cache.find(key);
