@@ -252,6 +252,12 @@ int pfdd_gl_theta(pfdd_gl *h, double *theta);
  * -- plus, for the first three, the FFT radix plan: choice 3, 4, 5 are shapes
  * 0, 1, 2 with radix-16 stages wherever they save a stage (lengths 16, 48,
  * 80, 128, 256: 128 = 16 x 8 instead of 8 x 8 x 2); 0-2 use radix 8 first.
+ * The shapes act where a transform keeps its stages in LDS.  Lines of 32, 64,
+ * 128, 256 and 512 points are transformed in registers: there the line passes
+ * and the update of a sine-series core have one shape (any choice of one radix
+ * plan launches the same kernel, and the tuner reports 1), choice[3] sets the
+ * tile of the reverse mode only, and the x pass has one form (variants 0 and 1
+ * are the same).
  * choice[4] is the iteration variant:
  *   0  five kernels, x pass one tile per workgroup;
  *   1  five kernels, x pass on persistent workgroups that load the next tile
@@ -269,7 +275,7 @@ int pfdd_gl_theta(pfdd_gl *h, double *theta);
  * fastest of the three wins), and variant 2 replaces the winner if its whole
  * iteration is faster (choice[5], may be NULL).  The field and step counters
  * are restored; the choice is cached for the process per grid, system count,
- * batch, precision and options.  Tile shapes and iteration variants give the
+ * batch, precision, options and kind of core model (the update it launches).  Tile shapes and iteration variants give the
  * same xi bit for bit; the two radix plans round differently (relative
  * differences of a few ulp per transform).  The update of core models 2, 4
  * and 9 always uses tile shape 0. */

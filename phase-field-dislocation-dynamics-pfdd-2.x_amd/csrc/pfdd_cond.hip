@@ -264,14 +264,6 @@ __global__ void __launch_bounds__(NTHR)
 }
 
 // ---------------------------------------------------------------- launchers
-bool cond_reg_length(int n)
-{
-#define PFDD_CASE(n_) if (n == n_) return reg_length<n_>();
-    PFDD_SIZES(PFDD_CASE)
-#undef PFDD_CASE
-    return false;
-}
-
 hipError_t launch_cond_div(const double2 *ch, double2 *ab, const double *sig, const CondParams &P, double *part,
                            long long pstride, int nu, int *nparts, int *done, hipStream_t st)
 {

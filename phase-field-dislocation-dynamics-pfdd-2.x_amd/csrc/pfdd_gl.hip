@@ -935,7 +935,10 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
     // the same shapes with the radix-16 plan in the line passes (q + 3,
     // where the z or y length has that plan); then (on-the-fly contraction
     // only) the pipelined x pass, then (where the grid allows it) the
-    // three-kernel plane iteration.  The clock of an idle GPU ramps up over
+    // three-kernel plane iteration.  A pass whose kernel does not depend on the
+    // shape (register transforms; the update of the coupled and Fourier models)
+    // has one shape, `own`; a candidate that launches the same kernels as one
+    // before it is not timed.  The clock of an idle GPU ramps up over
     // the first few dozen dispatches, so all candidates are timed after a
     // common warm-up, in two interleaved rounds, keeping each kernel's best
     // time per candidate.  The five-kernel iteration takes the best shape and
@@ -944,9 +947,31 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
     // pass that starts a run is not part of the sums).
     const bool plan_z = radix16_plan_differs_rt(h->nz), plan_y = radix16_plan_differs_rt(h->ny);
     const int nshape = (plan_z || plan_y) ? 6 : 3;
-    const int c_pipe = h->stored_B ? -1 : nshape;
+    const bool reg_y = reg_length_rt(h->ny), reg_z = reg_length_rt(h->nz);
+    const int c_pipe = h->stored_B || reg_length_rt(h->nx) ? -1 : nshape;
     const int c_plane = (!h->stored_B && h->plane_ok) ? nshape + 1 : -1;
-    const int ncand = nshape + (c_pipe >= 0 ? 1 : 0) + (c_plane >= 0 ? 1 : 0);
+    // the reverse mode needs blocks of one system
+    auto upd_ok = [&](int q) {
+        const int nl = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, q) : tile_lines_rt<float>(h->nz, q);
+        return ((long long)h->nx * h->ny) % nl == 0;
+    };
+    // the choice of pass p (0 fwd z, 1 fwd y, 2 inv y, 3 update) that candidate
+    // q stands for
+    auto own = [&](int q, int p) {
+        const bool z = p == 0 || p == 3;
+        const int plan = (z ? plan_z : plan_y) ? q / 3 * 3 : 0;
+        if (p == 3 && gen) return plan;
+        if (z ? reg_z : reg_y) return plan + (p == 3 && !upd_ok(1) ? 0 : 1);
+        return plan + q % 3;
+    };
+    auto repeats = [&](int q) { // of an earlier candidate
+        for (int e = 0; e < q; ++e) {
+            bool same = true;
+            for (int p = 0; p < 4; ++p) same = same && own(e, p) == own(q, p);
+            if (same) return true;
+        }
+        return false;
+    };
     double tmin[8][5];
     for (int c = 0; c < 8; ++c)
         for (int p = 0; p < 5; ++p) tmin[c][p] = 1e300;
@@ -956,15 +981,19 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
         rc = time_passes<R>(h, 20, warm);
     }
     for (int round = 0; round < 2 && !rc; ++round)
-        for (int c = 0; c < ncand && !rc; ++c) {
-            const int ln = c < nshape ? c : 1, up = c < nshape ? c % 3 : 1;
+        for (int c = 0; c < nshape + 2 && !rc; ++c) {
+            if (c < nshape ? repeats(c) : c != c_pipe && c != c_plane) continue;
+            const int q = c < nshape ? c : 1;
             const int var = c < nshape ? 0 : c == c_pipe ? 1 : 2;
-            const int all[5] = {ln, ln, ln, up, var};
+            const int all[5] = {own(q, 0), own(q, 1), own(q, 2), own(q, 3) % 3, var};
             set_tiles(h, all);
             reset_run(h, h->stream);
             double warm[5], t[5];
             if ((rc = time_passes<R>(h, 1, warm)) || (rc = time_passes<R>(h, nsteps, t))) break;
-            for (int p = 0; p < 5; ++p) tmin[c][p] = t[p] < tmin[c][p] ? t[p] : tmin[c][p];
+            for (int p = 0; p < 5; ++p) {
+                double &best = tmin[p < 4 && c < nshape ? own(c, p) : c][p];
+                best = t[p] < best ? t[p] : best;
+            }
         }
     // the fastest shape of the forward z pass (run once per run) among those
     // of one radix plan
@@ -979,13 +1008,8 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
         // the radix plan of the z transforms are chosen together
         int zplan = 0;
         for (int q = 0; q < nshape; ++q) {
-            const int nl = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, q) : tile_lines_rt<float>(h->nz, q);
-            const bool upd_ok = ((long long)h->nx * h->ny) % nl == 0;
-            // a plan-1 candidate counts for a pass only where its length has a
-            // distinct radix-16 plan
-            const bool use[4] = {false, q < 3 || plan_y, q < 3 || plan_y, (q < 3 || plan_z) && upd_ok};
             for (int p = 1; p < 4; ++p)
-                if (use[p] && tmin[q][p] < best[p]) {
+                if ((p < 3 || upd_ok(q)) && tmin[q][p] < best[p]) {
                     best[p] = tmin[q][p];
                     arg[p] = q % 3 + (p < 3 ? q / 3 * 3 : 0);
                     if (p == 3) zplan = q / 3;
@@ -1011,17 +1035,15 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
             int u1 = -1, u2 = -1;
             double s1 = 1e300, s2 = 1e300;
             for (int q = 0; q < nshape; ++q) {
-                const double s = tmin[q][1] + tmin[q][2] + tmin[q][3] + tmin[q][4];
+                if (repeats(q)) continue;
+                const double s = tmin[own(q, 1)][1] + tmin[own(q, 2)][2] + tmin[own(q, 3)][3] + tmin[q][4];
                 if (s < s1) { s2 = s1; u2 = u1; s1 = s; u1 = q; }
                 else if (s < s2) { s2 = s; u2 = q; }
             }
             for (const int q : {u1, u2}) {
                 if (q < 0) continue;
-                const int nl = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, q % 3)
-                                                    : tile_lines_rt<float>(h->nz, q % 3);
-                const bool upd_ok = ((long long)h->nx * h->ny) % nl == 0;
-                const int u[5] = {best_z(plan_z ? q / 3 : 0), q < 3 || plan_y ? q : q % 3,
-                                  q < 3 || plan_y ? q : q % 3, upd_ok ? q % 3 : arg[3], arg[4]};
+                const int u[5] = {best_z(plan_z ? q / 3 : 0), own(q, 1), own(q, 2),
+                                  upd_ok(own(q, 3)) ? own(q, 3) % 3 : arg[3], arg[4]};
                 bool dup = false;
                 for (int c = 0; c < nc; ++c) dup = dup || std::equal(u, u + 5, cand[c]);
                 if (!dup) {
@@ -2491,7 +2513,7 @@ int cond_step(pfdd_gl_cond *h, bool first, bool last, int &nu, int &nd)
     const Maps m1 = cond_maps(h, 1), m2 = cond_maps(h, 2);
     const long long ncol = (long long)h->ny * h->nz;
     const LineMap xs = {h->nx, 0, 0, 1, 1, 1};
-    const bool xr = cond_reg_length(h->nx), zr = cond_reg_length(h->nz);
+    const bool xr = reg_length_rt(h->nx), zr = reg_length_rt(h->nz);
     // forwardcond: FFT of c; divcurrent; backwardcond's two inverse
     // transforms; every pass from one work buffer to the other
     double2 *in = h->w0, *out = h->w1;

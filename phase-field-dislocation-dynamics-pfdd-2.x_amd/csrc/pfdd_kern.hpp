@@ -382,6 +382,18 @@ inline bool radix16_plan_differs_rt(int n)
     return false;
 }
 
+// Line lengths with register transforms (pfdd_reg.hpp): powers of two with two
+// or three stages.  Other lengths (an odd factor, or a single stage) keep the
+// stages in LDS.
+template <int N> constexpr bool reg_length() { return N == 32 || N == 64 || N == 128 || N == 256 || N == 512; }
+inline bool reg_length_rt(int n)
+{
+#define PFDD_CASE(n_) if (n == n_) return reg_length<n_>();
+    PFDD_SIZES(PFDD_CASE)
+#undef PFDD_CASE
+    return false;
+}
+
 inline bool systems_supported(int s) { return s == 1 || s == 2 || s == 3 || s == 4 || s == 6 || s == 12; }
 
 // Lines per tile of the update kernels for tile shape tq.
@@ -522,7 +534,6 @@ struct CondStat {
     double s[5]; // Re j, Im j, |dc|^2, Re c, sig Re a (divcurrent)
     int done;
 };
-bool cond_reg_length(int n); // the length has the fused kernels
 hipError_t launch_cond_div(const double2 *ch, double2 *ab, const double *sig, const CondParams &P, double *part,
                            long long pstride, int nu, int *nparts, int *done, hipStream_t st);
 hipError_t launch_cond_x(const double2 *ch, double2 *ab, const double *sig, const CondParams &P, const void *tw,

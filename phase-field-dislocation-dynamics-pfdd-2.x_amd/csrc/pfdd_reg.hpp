@@ -215,11 +215,6 @@ __device__ __forceinline__ void reg_twiddles(V *tws, const V *__restrict__ tw, i
         if (N % W == 0 || t + m * W < N) tws[t + m * W] = tw[t + m * W];
 }
 
-// Line lengths with register transforms: powers of two with two or three
-// stages.  Other lengths (an odd factor, or a single stage) keep the stages in
-// LDS.
-template <int N> constexpr bool reg_length() { return N == 32 || N == 64 || N == 128 || N == 256 || N == 512; }
-
 // Values per thread and lines per tile of the line passes and the update: 256
 // bytes of neighbouring lines (16 FP64, 32 FP32 lines) where the exchange tile
 // stays within 32 KB, and the 128 bytes of 16 FP32 lines beyond.  Half of that

@@ -33,3 +33,20 @@ def test_a_choice_is_kept_for_its_own_core_model():
         kept = min(_seconds(case, 0, 300) for _ in range(3))
         print(f"core {case['core_flag']} with {case['nm']} terms: {tuned * 1e3:.1f} ms, kept {kept * 1e3:.1f} ms", flush=True)
         assert tuned > 3 * kept, (case["core_flag"], case["nm"])
+
+
+@pytest.mark.parametrize("core", ["sine", "extended"])
+def test_tile_shapes_are_not_chosen_where_they_change_nothing(core):
+    """At 32, 64, 128, 256 and 512 points one line pass (and one sine-series
+    update, one x pass) serves every tile shape, and the coupled model has one
+    update shape: there the choice is the default, not a matter of timing."""
+    case = P.make_case(shape=(32, 64, 128), core=core)
+    g = P.gpu_solver(case)
+    try:
+        c = g.autotune(4)
+    finally:
+        g.close()
+    print(f"{core}: {c}", flush=True)
+    assert [v % 3 for v in c[:3]] == [1, 1, 1]
+    assert c[3] == (0 if core == "extended" else 1)
+    assert c[4] == 0
