@@ -217,7 +217,7 @@ struct Sums {
     unsigned *ticket; // zero between launches
     RunStat *stat;
     int *done, *steps;
-    bool last;        // the run ends here
+    bool report;      // leave the scalars in stat
 };
 
 // Deterministic reduction of the block partials in two levels: every block
@@ -284,7 +284,7 @@ __global__ void __launch_bounds__(NTHR) k_sums(Sums F)
     const int steps = (int)((unsigned)*F.steps + 1u);
     *F.steps = steps;
     if (done) *F.done = done;
-    if (!F.last && !done) return;
+    if (!F.report && !done) return;
     F.stat->res[0] = xinorm;
     F.stat->res[1] = w[1];
     F.stat->res[2] = e_el;
@@ -717,10 +717,11 @@ int graph_tau(pfdd_gl *h, hipStream_t st)
 // iterations that each start from the previous one's result.  first: xo
 // enters the run here, so pass 1 (or the forward plane pass) runs; otherwise
 // the previous iteration left it in T1.  last: nothing follows, so the update
-// does not transform its result.  A run of one is first and last.
+// does not transform its result.  A run of one is first and last.  report: the
+// scalars go to the host (where a run ends, and where a profile does).
 template <typename R>
 int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, const StepParams &P, bool first,
-              bool last)
+              bool last, bool report)
 {
     const Maps m = make_maps(h, h->SM);
     hipStream_t st = h->stream;
@@ -803,15 +804,15 @@ int step_core(pfdd_gl *h, double tol, hipEvent_t *ev, const void *xo, void *T2, 
     arm(5);
     PFDD_LAUNCH(k_sums, dim3(NB2), dim3(NTHR), st,
                 Sums{h->partial, h->pstride, nb5, h->nb3, 1.0 / (double)h->N, no_eref ? 0.0 : 1.0 / (double)h->nx,
-                     tol, h->stage2, h->ticket, h->stat, h->done, h->steps, last});
+                     tol, h->stage2, h->ticket, h->stat, h->done, h->steps, report});
     HIPCHK(hipGetLastError());
     return PFDD_OK;
 }
 
 template <typename R>
-int step_once(pfdd_gl *h, double tol, hipEvent_t *ev, bool first, bool last)
+int step_once(pfdd_gl *h, double tol, hipEvent_t *ev, bool first, bool last, bool report)
 {
-    const int rc = step_core<R>(h, tol, ev, h->xi[h->cur], h->xi[1 - h->cur], h->P, first, last);
+    const int rc = step_core<R>(h, tol, ev, h->xi[h->cur], h->xi[1 - h->cur], h->P, first, last, report);
     if (rc) return rc;
     h->cur = 1 - h->cur;
     h->stepped = true;
@@ -837,8 +838,8 @@ void set_tiles(pfdd_gl *h, const int tq[5])
 // One iteration of h in its precision (see step_core).
 int step_any(pfdd_gl *h, double tol, bool first, bool last)
 {
-    return h->prec == PFDD_FP64 ? step_once<double>(h, tol, nullptr, first, last)
-                                : step_once<float>(h, tol, nullptr, first, last);
+    return h->prec == PFDD_FP64 ? step_once<double>(h, tol, nullptr, first, last, last)
+                                : step_once<float>(h, tol, nullptr, first, last, last);
 }
 
 // Device time (ms) of the five tunable kernels, summed over nsteps GL
@@ -853,7 +854,7 @@ int time_passes(pfdd_gl *h, int nsteps, double acc[5])
     const int pass_k[5] = {0, 1, 3, 4, 2}; // fwd z, fwd y, inv y, inv z + update, x pass
     int rc = PFDD_OK;
     for (int s = 0; s < nsteps && !rc; ++s) {
-        rc = step_once<R>(h, 0.0, ev, s == 0, false);
+        rc = step_once<R>(h, 0.0, ev, s == 0, false, false);
         if (rc) break;
         if (hipEventSynchronize(ev[11]) != hipSuccess) {
             rc = fail(PFDD_ERR_HIP, "autotune timing failed");
@@ -1528,8 +1529,8 @@ int tape_backward_any(pfdd_gl *h, const void *dxi_T, bool dev_in, void *dxi_0, b
         for (int j = 1; j < len; ++j) {
             const bool first = j == 1, last = j == len - 1;
             rc = h->prec == PFDD_FP64
-                     ? step_core<double>(h, 0.0, nullptr, xs[j - 1], T.seg[j - 1], T.P, first, last)
-                     : step_core<float>(h, 0.0, nullptr, xs[j - 1], T.seg[j - 1], T.P, first, last);
+                     ? step_core<double>(h, 0.0, nullptr, xs[j - 1], T.seg[j - 1], T.P, first, last, last)
+                     : step_core<float>(h, 0.0, nullptr, xs[j - 1], T.seg[j - 1], T.P, first, last, last);
             if (rc) return rc;
             xs[j] = T.seg[j - 1];
         }
@@ -2254,8 +2255,8 @@ int pfdd_gl_profile(pfdd_gl *h, int nsteps, double *ms, int *nkernels)
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     reset_run(h, h->stream);
     for (int s = 0; s < nsteps && !rc; ++s)
-        rc = h->prec == PFDD_FP64 ? step_once<double>(h, 0.0, &ev[12 * s], s == 0, false)
-                                  : step_once<float>(h, 0.0, &ev[12 * s], s == 0, false);
+        rc = h->prec == PFDD_FP64 ? step_once<double>(h, 0.0, &ev[12 * s], s == 0, false, s == nsteps - 1)
+                                  : step_once<float>(h, 0.0, &ev[12 * s], s == 0, false, s == nsteps - 1);
     if (!rc && hipEventSynchronize(ev.back()) != hipSuccess) rc = fail(PFDD_ERR_HIP, "profile wait failed");
     for (int s = 0; s < nsteps && !rc; ++s) {
         const hipEvent_t *e = &ev[12 * s];
