@@ -1405,16 +1405,23 @@ int diag_fields(pfdd_gl *h, const double *sigma_rot, const double *avepst, const
     const Maps ms = make_maps(h, S), m6 = make_maps(h, 6);
     const long long ncol = (long long)h->ny * h->nz;
     const LineMap xs = {h->nx, 0, 0, 1, 1, 1}; // x lines of the [.][k][j][i] layout
-    HIPCHK((launch_pass<R, false>(h->nz, pre, h->dw[0], ms.p1i, ms.p1o, ms.n1, h->tw[2], h->done, st)));
-    HIPCHK((launch_pass<R, false>(h->ny, h->dw[0], h->dw[1], ms.p2i, ms.p2o, ms.n2, h->tw[1], h->done, st)));
-    HIPCHK((launch_pass<R, false>(h->nx, h->dw[1], h->dw[0], xs, xs, S * ncol, h->tw[0], h->done, st)));
+    const Order ord = {order_of((size_t)(S > 6 ? S : 6) * N * h->esz, (int)h->esz).keep, false};
+    HIPCHK((launch_pass<R, false>(h->nz, pre, h->dw[0], ms.p1i, ms.p1o, ms.n1, h->tw[2], h->done, st,
+                                   nullptr, 1, ord)));
+    HIPCHK((launch_pass<R, false>(h->ny, h->dw[0], h->dw[1], ms.p2i, ms.p2o, ms.n2, h->tw[1], h->done, st,
+                                   nullptr, 1, ord)));
+    HIPCHK((launch_pass<R, false>(h->nx, h->dw[1], h->dw[0], xs, xs, S * ncol, h->tw[0], h->done, st,
+                                   nullptr, 1, ord)));
     const unsigned nb = (unsigned)((N + NTHR - 1) / NTHR);
     typedef typename cvec<R>::type V;
     hipLaunchKernelGGL((k_diag_comp<R>), dim3(nb), dim3(NTHR), 0, st, (const V *)h->dw[0], (V *)h->dw[1], P, N);
     HIPCHK(hipGetLastError());
-    HIPCHK((launch_pass<R, true>(h->nx, h->dw[1], h->dw[0], xs, xs, 6 * ncol, h->tw[0], h->done, st)));
-    HIPCHK((launch_pass<R, true>(h->ny, h->dw[0], h->dw[1], m6.p2o, m6.p2i, m6.n2, h->tw[1], h->done, st)));
-    HIPCHK((launch_pass<R, true>(h->nz, h->dw[1], h->dw[0], m6.p5i, m6.p5o, m6.n5, h->tw[2], h->done, st)));
+    HIPCHK((launch_pass<R, true>(h->nx, h->dw[1], h->dw[0], xs, xs, 6 * ncol, h->tw[0], h->done, st,
+                                   nullptr, 1, ord)));
+    HIPCHK((launch_pass<R, true>(h->ny, h->dw[0], h->dw[1], m6.p2o, m6.p2i, m6.n2, h->tw[1], h->done, st,
+                                   nullptr, 1, ord)));
+    HIPCHK((launch_pass<R, true>(h->nz, h->dw[1], h->dw[0], m6.p5i, m6.p5o, m6.n5, h->tw[2], h->done, st,
+                                   nullptr, 1, ord)));
     hipLaunchKernelGGL((k_diag_real<R>), dim3(nb), dim3(NTHR), 0, st, (const V *)h->dw[0],
                        (const V *)h->xi[h->cur], h->deps, h->dsig, P, N);
     HIPCHK(hipGetLastError());
@@ -2514,6 +2521,7 @@ int cond_step(pfdd_gl_cond *h, bool first, bool last, int &nu, int &nd)
     const Maps m1 = cond_maps(h, 1), m2 = cond_maps(h, 2);
     const long long ncol = (long long)h->ny * h->nz;
     const LineMap xs = {h->nx, 0, 0, 1, 1, 1};
+    const Order ord = {order_of(2 * sizeof(double2) * (size_t)h->N, sizeof(double2)).keep, false};
     const bool xr = reg_length_rt(h->nx), zr = reg_length_rt(h->nz);
     // forwardcond: FFT of c; divcurrent; backwardcond's two inverse
     // transforms; every pass from one work buffer to the other
@@ -2521,21 +2529,25 @@ int cond_step(pfdd_gl_cond *h, bool first, bool last, int &nu, int &nd)
     auto swap = [&] { std::swap(in, out); };
     if (first || !zr) // (with the radix plan of the update's own forward transform)
         HIPCHK((launch_pass<double, false>(h->nz, h->c, in, m1.p1i, m1.p1o, m1.n1, h->tw[2], h->done, st, nullptr,
-                                           zr ? 4 : 1)));
-    HIPCHK((launch_pass<double, false>(h->ny, in, out, m1.p2i, m1.p2o, m1.n2, h->tw[1], h->done, st)));
+                                           zr ? 4 : 1, ord)));
+    HIPCHK((launch_pass<double, false>(h->ny, in, out, m1.p2i, m1.p2o, m1.n2, h->tw[1], h->done, st, nullptr, 1,
+                                       ord)));
     swap();
     if (xr) {
         HIPCHK(launch_cond_x(in, out, h->sig, h->P, h->tw[0], h->part, h->nb, nu, &nd, h->done, st));
         swap();
     } else {
-        HIPCHK((launch_pass<double, false>(h->nx, in, out, xs, xs, ncol, h->tw[0], h->done, st)));
+        HIPCHK((launch_pass<double, false>(h->nx, in, out, xs, xs, ncol, h->tw[0], h->done, st, nullptr, 1,
+                                       ord)));
         swap();
         HIPCHK(launch_cond_div(in, out, h->sig, h->P, h->part, h->nb, nu, &nd, h->done, st));
         swap();
-        HIPCHK((launch_pass<double, true>(h->nx, in, out, xs, xs, 2 * ncol, h->tw[0], h->done, st)));
+        HIPCHK((launch_pass<double, true>(h->nx, in, out, xs, xs, 2 * ncol, h->tw[0], h->done, st, nullptr, 1,
+                                       ord)));
         swap();
     }
-    HIPCHK((launch_pass<double, true>(h->ny, in, out, m2.p2o, m2.p2i, m2.n2, h->tw[1], h->done, st)));
+    HIPCHK((launch_pass<double, true>(h->ny, in, out, m2.p2o, m2.p2i, m2.n2, h->tw[1], h->done, st, nullptr, 1,
+                                       ord)));
     swap();
     if (zr) {
         // in is w1 here: the transform of the new c goes to w0, where the next
@@ -2543,7 +2555,8 @@ int cond_step(pfdd_gl_cond *h, bool first, bool last, int &nu, int &nd)
         HIPCHK(launch_cond_update_r(!last, in, h->c, out, h->sig, h->dsig, h->P, h->tw[2], h->part, h->nb, &nu,
                                     h->done, st));
     } else {
-        HIPCHK((launch_pass<double, true>(h->nz, in, out, m2.p5i, m2.p5o, m2.n5, h->tw[2], h->done, st)));
+        HIPCHK((launch_pass<double, true>(h->nz, in, out, m2.p5i, m2.p5o, m2.n5, h->tw[2], h->done, st, nullptr, 1,
+                                       ord)));
         swap();
         HIPCHK(launch_cond_update(in, h->c, h->sig, h->dsig, h->P, h->part, h->nb, &nu, h->done, st));
     }
