@@ -52,15 +52,12 @@ template <typename R, int N, int S> constexpr int mid_pairs()
     return np;
 }
 
-// Tile addressing of the on-the-fly x pass: Swz8 for its 24-line FP64 tiles
-// (12 systems x 2 columns at 96 and 128 points); unpadded rows for FP64
-// lines of 512 points, whose padded tile (57.6 KB) leaves room for only two
-// blocks per CU; RowPad otherwise.
+// Tile addressing of the on-the-fly x pass where its stages are in LDS: Swz8 for
+// 24-line FP64 tiles (12 systems x 2 columns, at 96 points and, in the plane
+// layout, 128); RowPad otherwise.
 template <typename R, int N, int S> struct XLay {
     static constexpr int NL = S * mid_pairs<R, N, S>();
-    typedef typename std::conditional<
-        (sizeof(R) == 8 && NL == 24 && N % 16 == 0), Swz8<NL>,
-        typename std::conditional<(sizeof(R) == 8 && N >= 512), RowPad<NL, 0>, RowPad<NL>>::type>::type type;
+    typedef typename std::conditional<(sizeof(R) == 8 && NL == 24 && N % 16 == 0), Swz8<NL>, RowPad<NL>>::type type;
 };
 
 template <typename R, typename RB, int N, int S>

@@ -38,16 +38,11 @@ template <int PL> constexpr int plan_radix(int m) { return PL == 1 ? pick_radix_
 // padding.  The position comes as pv | ps with disjoint bits, ps known at
 // compile time: the ps part folds into constants.
 template <int NL> struct RegSwz {
-    static_assert(NL == 8 || NL % 16 == 0, "tiles of 8 lines or a multiple of 16");
-    __device__ __forceinline__ static constexpr int f(int p)
-    {
-        if constexpr (NL == 8) return (p & 6) | ((p >> 3) & 1) | (((p ^ (p >> 3) ^ (p >> 4)) & 1) << 3);
-        else return ((p & 7) << 1) | ((p >> 3) & 1);
-    }
+    static_assert(NL % 16 == 0, "tiles of a multiple of 16 lines");
+    __device__ __forceinline__ static constexpr int f(int p) { return ((p & 7) << 1) | ((p >> 3) & 1); }
     __device__ __forceinline__ static int at(int pv, int ps, int l)
     {
-        if constexpr (NL == 8) return (pv >> 1) * 16 + ((l ^ f(pv)) ^ f(ps)) + (ps >> 1) * 16;
-        else return pv * NL + ((l ^ f(pv)) ^ f(ps)) + ps * NL;
+        return pv * NL + ((l ^ f(pv)) ^ f(ps)) + ps * NL;
     }
 };
 

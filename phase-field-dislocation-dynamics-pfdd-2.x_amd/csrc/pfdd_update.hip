@@ -11,10 +11,9 @@ namespace pfdd {
 // does (it reads data_fftw = xi before the update).  Masked cells keep their
 // value; their xinorm term uses the previous unmasked cell's old value in
 // (a, i, j, k) order (prev[] precomputed on the host, -1 = the initial 0).
-// The FP64 sine-series update on its smallest tile at 32-128 points (8
-// lines at 128 points, 19-20 KB of LDS: 8 blocks per CU) asks for 8 waves per
-// SIMD: 64 instead of 68 VGPRs, 229 -> 224.5 us at 128^3 x 12.  The same
-// hint made the FP32 one 9 % slower.
+// The FP64 sine-series update on its smallest tile at 40-96 points (19-20 KB
+// of LDS: 8 blocks per CU) asks for 8 waves per SIMD (64 instead of 68 VGPRs;
+// the same hint made the FP32 one 9 % slower).
 //
 // FW: 0 the update alone (last iteration of a run); 1, 2 the update followed
 // by the forward z transform of the new field, written back over the block's
@@ -24,7 +23,7 @@ namespace pfdd {
 // kernels.
 template <typename R, int N, int TQ, bool GEN, int FW> constexpr int update_waves()
 {
-    return (sizeof(R) == 8 && TQ == 0 && !GEN && FW < 2 && N >= 32 && N <= 128) ? 8 : 1;
+    return (sizeof(R) == 8 && TQ == 0 && !GEN && FW < 2 && N >= 40 && N <= 96) ? 8 : 1;
 }
 
 template <typename R, int N, int TQ, bool GEN, int FW>
