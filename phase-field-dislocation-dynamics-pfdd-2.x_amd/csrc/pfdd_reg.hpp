@@ -31,12 +31,17 @@ template <int PL> constexpr int plan_radix(int m) { return PL == 1 ? pick_radix_
 
 // Exchange tile of NL lines: value (p, l) at an address whose low four bits
 // (the 8-byte slot within 128 bytes of LDS, which serves 16 lanes at a time)
-// are a linear function of the bits of p and l.  It has full rank on every
-// group of 16 lanes that the exchanges use: 16 lines of a row, 8 lines of two
-// rows that are 1, 8 or 16 apart, 16 consecutive positions of a line, 8
-// consecutive positions of two lines.  So there are no bank conflicts and no
-// padding.  The position comes as pv | ps with disjoint bits, ps known at
-// compile time: the ps part folds into constants.
+// are a linear function of the bits of p and l.  It has full rank on these
+// groups of 16 lanes: 16 lines of a row, 16 consecutive positions of a line, 8
+// consecutive positions of two lines; there are no conflicts there and no
+// padding.  It has not on the first exchange of a transform that starts
+// position-fastest, as the one after an update does: neighbouring lanes write
+// rows RAD apart, f knows two values on multiples of 8, and 8 lanes share a slot
+// (16 where RAD is 16 and a line has 16 threads, at 256 points).  Counted at 128^3
+// x 12: 2.25e7 (FP64) and 1.1e7 (FP32) conflict cycles a launch of the update
+// with that transform, 4.9e5 and 0 without; the forward line passes 0, the
+// inverse ones 1.6e6 and 7.9e5.  The position comes as pv | ps with disjoint
+// bits, ps known at compile time: the ps part folds into constants.
 template <int NL> struct RegSwz {
     static_assert(NL % 16 == 0, "tiles of a multiple of 16 lines");
     __device__ __forceinline__ static constexpr int f(int p) { return ((p & 7) << 1) | ((p >> 3) & 1); }
@@ -211,8 +216,9 @@ __device__ __forceinline__ void reg_twiddles(V *tws, const V *__restrict__ tw, i
 }
 
 // Values per thread and lines per tile of the line passes and the update: 256
-// bytes of neighbouring lines (16 FP64, 32 FP32 lines) where the exchange tile
-// stays within 32 KB, and the 128 bytes of 16 FP32 lines beyond.  Half of that
+// bytes of neighbouring lines (16 FP64, 32 FP32 lines), and the 128 bytes of 16
+// FP32 lines from 256 points up: exchange tiles of 4 to 32 KB, and of 64 KB at 512
+// points.  Half of that
 // cost the FP64 update at 512 x 512 x 256 x 3 2317 -> 2545 us; twice the LDS
 // cost the FP32 one 1245 -> 1459 us.
 template <typename R, int N> struct RegTile {

@@ -154,8 +154,8 @@ __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(updat
 // row of xi (position-fastest: runs of D cells), updates them in place and,
 // with FW, transforms them forward from the same registers and writes T1.  Two
 // LDS accesses per value and transform are left (six in k_update at 128
-// points) and no barrier at all where a tile is one wave (FP64 up to 128
-// points).  The twiddles sit in LDS: loads from memory would wait, in order,
+// points) and no barrier at all where a tile is one wave (FP64 at 32 points).
+// The twiddles sit in LDS: loads from memory would wait, in order,
 // for the streams in flight.
 //
 // NM: terms of the core's sine series, padded to 2, 4 or 8; MA: with an
