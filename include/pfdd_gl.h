@@ -271,14 +271,14 @@ int pfdd_gl_theta(pfdd_gl *h, double *theta);
  * interleaved rounds of `nsteps` GL iterations per candidate, keeping each
  * kernel's best time; the fastest shape and plan per line pass and the
  * faster x-pass variant form a mix, which is timed as a whole iteration
- * against the two uniform candidates with the smallest iteration sums (the
- * fastest of the three wins), and variant 2 replaces the winner if its whole
- * iteration is faster (choice[5], may be NULL).  The field and step counters
- * are restored; the choice is cached for the process per grid, system count,
- * batch, precision, options and kind of core model (the update it launches).  Tile shapes and iteration variants give the
- * same xi bit for bit; the two radix plans round differently (relative
- * differences of a few ulp per transform).  The update of core models 2, 4
- * and 9 always uses tile shape 0. */
+ * against the two uniform candidates with the smallest iteration sums and,
+ * where the grid allows it, variant 2 (three interleaved rounds of `nsteps`
+ * iterations; the fastest wins; choice[5], may be NULL).  The field and step
+ * counters are restored; the choice is cached for the process per grid, system
+ * count, batch, precision, options and kind of core model (the update it
+ * launches).  Tile shapes and iteration variants give the same xi bit for bit;
+ * the two radix plans round differently (relative differences of a few ulp per
+ * transform).  The update of core models 2, 4 and 9 always uses tile shape 0. */
 int pfdd_gl_autotune(pfdd_gl *h, int nsteps, int choice[5]);
 /* Sets the choices explicitly (same meaning as pfdd_gl_autotune's output). */
 int pfdd_gl_set_tuning(pfdd_gl *h, const int choice[5]);

@@ -870,6 +870,29 @@ int time_passes(pfdd_gl *h, int nsteps, double acc[5])
     return rc;
 }
 
+// Device time (ms) of nsteps iterations from inside a run with the handle's
+// current choices, as they follow each other: kernels, reduction and the gaps.
+template <typename R>
+int time_steps(pfdd_gl *h, int nsteps, double &ms)
+{
+    hipEvent_t ev[2] = {};
+    float t = 0;
+    int rc = PFDD_OK;
+    hipError_t e = hipSuccess;
+    for (int q = 0; q < 2 && e == hipSuccess; ++q) e = hipEventCreate(&ev[q]);
+    for (int s = 0; s <= nsteps && !rc && e == hipSuccess; ++s) { // the first one starts the run
+        rc = step_once<R>(h, 0.0, nullptr, s == 0, false, false);
+        if (!rc && (s == 0 || s == nsteps)) e = hipEventRecord(ev[s == 0 ? 0 : 1], h->stream);
+    }
+    if (!rc && e == hipSuccess) e = hipEventSynchronize(ev[1]);
+    if (!rc && e == hipSuccess) e = hipEventElapsedTime(&t, ev[0], ev[1]);
+    for (hipEvent_t v : ev)
+        if (v) (void)hipEventDestroy(v);
+    ms = t;
+    if (!rc && e != hipSuccess) rc = fail(PFDD_ERR_HIP, "autotune timing failed: %s", hipGetErrorString(e));
+    return rc;
+}
+
 int self_graph_ready(pfdd_gl *h, double tol);
 
 struct TuneKey {
@@ -884,9 +907,9 @@ std::map<TuneKey, std::array<int, 5>> g_tune_cache;
 
 // Times every tile shape (0, 1, 2) of each line pass, with both radix plans
 // where the pass length has two (tq 3-5: the shapes with the radix-16 plan),
-// and the x-pass / iteration variants, keeps the fastest per kernel and then
-// the fastest whole step of that mix and the two best uniform choices.  The
-// field, ping-pong parity and step counters are restored.  Choices that would
+// and the x-pass variants, keeps the fastest per kernel and then the fastest
+// whole step of that mix, the two best uniform choices and the plane
+// iteration.  The field, ping-pong parity and step counters are restored.  Choices that would
 // break the reverse mode's one-system-per-block rule for the update pass are
 // skipped.
 template <typename R>
@@ -935,22 +958,21 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
     // candidates: tile shape q = 0, 1, 2 with the one-tile-per-block x pass;
     // the same shapes with the radix-16 plan in the line passes (q + 3,
     // where the z or y length has that plan); then (on-the-fly contraction
-    // only) the pipelined x pass, then (where the grid allows it) the
-    // three-kernel plane iteration.  A pass whose kernel does not depend on the
+    // only) the pipelined x pass.  A pass whose kernel does not depend on the
     // shape (register transforms; the update of the coupled and Fourier models)
     // has one shape, `own`; a candidate that launches the same kernels as one
     // before it is not timed.  The clock of an idle GPU ramps up over
     // the first few dozen dispatches, so all candidates are timed after a
     // common warm-up, in two interleaved rounds, keeping each kernel's best
-    // time per candidate.  The five-kernel iteration takes the best shape and
-    // plan of each kernel; the plane iteration replaces it if its whole step
-    // is faster than that sum (both as inside a run: the forward z or plane
-    // pass that starts a run is not part of the sums).
+    // time per candidate (the forward z pass runs once per run and is no part
+    // of the sums).  The best shape and plan of each kernel then meet, as whole
+    // steps, the best uniform choices and, where the grid allows it, the plane
+    // iteration.
     const bool plan_z = radix16_plan_differs_rt(h->nz), plan_y = radix16_plan_differs_rt(h->ny);
     const int nshape = (plan_z || plan_y) ? 6 : 3;
     const bool reg_y = reg_length_rt(h->ny), reg_z = reg_length_rt(h->nz);
     const int c_pipe = h->stored_B || reg_length_rt(h->nx) ? -1 : nshape;
-    const int c_plane = (!h->stored_B && h->plane_ok) ? nshape + 1 : -1;
+    const bool has_plane = !h->stored_B && h->plane_ok;
     // the reverse mode needs blocks of one system
     auto upd_ok = [&](int q) {
         const int nl = h->prec == PFDD_FP64 ? tile_lines_rt<double>(h->nz, q) : tile_lines_rt<float>(h->nz, q);
@@ -982,10 +1004,10 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
         rc = time_passes<R>(h, 20, warm);
     }
     for (int round = 0; round < 2 && !rc; ++round)
-        for (int c = 0; c < nshape + 2 && !rc; ++c) {
-            if (c < nshape ? repeats(c) : c != c_pipe && c != c_plane) continue;
+        for (int c = 0; c < nshape + 1 && !rc; ++c) {
+            if (c < nshape ? repeats(c) : c != c_pipe) continue;
             const int q = c < nshape ? c : 1;
-            const int var = c < nshape ? 0 : c == c_pipe ? 1 : 2;
+            const int var = c < nshape ? 0 : 1;
             const int all[5] = {own(q, 0), own(q, 1), own(q, 2), own(q, 3) % 3, var};
             set_tiles(h, all);
             reset_run(h, h->stream);
@@ -1022,13 +1044,16 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
             best[4] = tmin[c_pipe][4];
             arg[4] = 1;
         }
-        double five = best[1] + best[2] + best[3] + best[4];
         // The kernels of a step share the last-level cache (a whole FP32
         // field of 128^3 x 12 fits in it), so a kernel's time depends on the
         // tiles of its neighbours, and the mix of per-kernel winners was
         // never timed as one step.  Contest: the mix against the two
-        // candidates whose uniform choices had the smallest step sums, as
-        // whole steps in two interleaved rounds; the smallest step wins.
+        // candidates whose uniform choices had the smallest step sums, and the
+        // plane iteration, as whole steps in three interleaved rounds; the
+        // smallest step wins.  (Sums of kernel times leave out the gaps between
+        // launches, of which the plane iteration has half as many: at 64^3 x 3
+        // they took the five kernels in one process of six, 105.9 us a state
+        // against 99.9.)
         if (!rc) {
             int cand[3][5], nc = 0;
             for (int p = 0; p < 5; ++p) cand[nc][p] = arg[p];
@@ -1052,28 +1077,24 @@ int autotune(pfdd_gl *h, int nsteps, int choice[5])
                     ++nc;
                 }
             }
-            if (nc > 1) {
-                double ts[3] = {1e300, 1e300, 1e300};
-                for (int round = 0; round < 2 && !rc; ++round)
-                    for (int c = 0; c < nc && !rc; ++c) {
-                        set_tiles(h, cand[c]);
+            if (nc > 1 || has_plane) {
+                double ts[4] = {1e300, 1e300, 1e300, 1e300}; // ts[nc]: the plane iteration
+                for (int round = 0; round < 3 && !rc; ++round)
+                    for (int c = 0; c < nc + (has_plane ? 1 : 0) && !rc; ++c) {
+                        int one[5];
+                        for (int p = 0; p < 5; ++p) one[p] = cand[c < nc ? c : 0][p];
+                        if (c == nc) one[4] = 2;
+                        set_tiles(h, one);
                         reset_run(h, h->stream);
-                        double warm[5], t[5];
-                        if ((rc = time_passes<R>(h, 1, warm)) || (rc = time_passes<R>(h, nsteps, t))) break;
-                        const double s = t[1] + t[2] + t[3] + t[4];
+                        double s = 0.0;
+                        if ((rc = time_steps<R>(h, nsteps, s))) break;
                         ts[c] = s < ts[c] ? s : ts[c];
                     }
                 int bc = 0;
                 for (int c = 1; c < nc; ++c) bc = ts[c] < ts[bc] ? c : bc;
-                if (!rc) {
-                    for (int p = 0; p < 5; ++p) arg[p] = cand[bc][p];
-                    five = ts[bc];
-                }
+                for (int p = 0; p < 5; ++p) arg[p] = cand[bc][p];
+                if (has_plane && ts[nc] < ts[bc]) arg[4] = 2;
             }
-        }
-        if (!rc && c_plane >= 0) {
-            const double two = tmin[c_plane][3] + tmin[c_plane][4];
-            if (two < five) arg[4] = 2;
         }
     }
     int rc2 = restore();
